@@ -7,6 +7,7 @@ instructions are disabled.
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -18,22 +19,31 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
          "-Wno-unused-function"]
 
 
+# (object, source, extra flags): the step loop is compiled once per precision
+# and transport mode
+UNITS = [(os.path.splitext(f)[0], f, []) for f in SOURCES] + [
+    ("gxt_loop_%s_%d" % (r, m), "gxt_loop.hip", ["-DGXT_LOOP_R=" + r, "-DGXT_LOOP_MODE=%d" % m])
+    for r in ("double", "float") for m in range(5)]
+
+
+def _compile(unit, build_dir, verbose):
+    name, src, defs = unit
+    obj = os.path.join(build_dir, name + ".o")
+    cmd = [HIPCC] + (["-x", "hip"] if src.endswith(".cpp") else []) + FLAGS + defs + \
+        ["-c", os.path.join(CSRC, src), "-o", obj]
+    if verbose:
+        print(" ".join(cmd))
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("hipcc failed on %s:\n%s" % (src, r.stdout + r.stderr))
+    return obj
+
+
 def build(verbose=False):
-    objs = []
     build_dir = os.path.join(HERE, "_build")
     os.makedirs(build_dir, exist_ok=True)
-    for src in SOURCES:
-        obj = os.path.join(build_dir, os.path.splitext(src)[0] + ".o")
-        cmd = [HIPCC] + FLAGS + ["-c", os.path.join(CSRC, src), "-o", obj]
-        if src.endswith(".cpp"):
-            cmd = [HIPCC, "-x", "hip"] + FLAGS + ["-c", os.path.join(CSRC, src), "-o", obj]
-        if verbose:
-            print(" ".join(cmd))
-        r = subprocess.run(cmd, capture_output=True, text=True)
-        if r.returncode != 0:
-            sys.stderr.write(r.stdout + r.stderr)
-            raise RuntimeError("hipcc failed on %s" % src)
-        objs.append(obj)
+    with ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as ex:
+        objs = list(ex.map(lambda u: _compile(u, build_dir, verbose), UNITS))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp] + objs + ["-lpthread"]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -283,8 +283,8 @@ __device__ __forceinline__ void jump_row(const uint32_t *T, int c, int k, int d,
 // Substream idx of the stream seeded with s: (A^(2^76))^idx s, as the
 // product over the 8 bytes d_k of idx of A^(d_k 2^(76+8k)) (powers of one
 // matrix commute).  T[((c * 8 + k) * 256 + d) * kJumpRow + i], i < 9, holds
-// A_c^(d 2^(76+8k)) mod m_c, the identity for d = 0.  The loop is unrolled
-// so the rows' loads, which depend only on idx, issue ahead of the products.
+// A_c^(d 2^(76+8k)) mod m_c, the identity for d = 0.  The rows' loads depend
+// only on idx: two bytes' rows are in flight at a time.
 __device__ __forceinline__ void jump_substream(const uint32_t *T, const uint32_t s[6], uint64_t idx,
                                                uint32_t v1[3], uint32_t v2[3]) {
   v1[0] = s[0];
@@ -293,7 +293,7 @@ __device__ __forceinline__ void jump_substream(const uint32_t *T, const uint32_t
   v2[0] = s[3];
   v2[1] = s[4];
   v2[2] = s[5];
-#pragma unroll
+#pragma unroll 2
   for (int k = 0; k < 8; ++k) {
     const int d = (int)((idx >> (8 * k)) & 255u);
     uint32_t M1[9], M2[9];

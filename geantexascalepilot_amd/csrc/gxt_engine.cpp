@@ -1,10 +1,10 @@
 // gxt_engine.cpp -- host driver of the step loop and the C ABI of libgxt.so.
 //
-// One gxt_ctx owns one HIP stream, the device copy of the physics data, a
-// double-buffered SoA track pool, the interaction queues and the tallies.
-// Jobs (groups of primaries) are admitted into the shared pool by estimated
-// footprint; the device step loop runs several iterations between host
-// synchronisations; a job completes when its live-track counter reaches 0.
+// One gxt_ctx owns one HIP stream, the device copy of the physics data, the
+// pages of the live tracks and the tallies.  Jobs (groups of primaries) are
+// admitted into the shared pages by estimated footprint; launches of the
+// persistent step loop run between host synchronisations; a job completes
+// when its live-track counters reach 0.
 // This replaces ProxyDeviceManager (proxy/src/ProxyDeviceManager.cpp:41-276)
 // and the host wave loop DoStep<> (proxy/test/test_BasicCpuTransport.cpp:517-550).
 #include <hip/hip_runtime.h>
@@ -46,10 +46,6 @@ int set_err(int code, const std::string &msg) {
 int gxt::set_error(int code, const std::string &msg) { return set_err(code, msg); }
 
 namespace {
-
-// Largest table copy the transports stage in LDS (beside 11 KB of wave
-// histograms per workgroup).
-constexpr int kLdsTablesMax = 40 * 1024;
 
 #define HIP_TRY(expr)                                                                        \
   do {                                                                                       \
@@ -194,43 +190,6 @@ int upload(HostData &hd, DeviceData &dd) {
   return GXT_OK;
 }
 
-template <class R>
-struct DevPool {
-  Pool<R> p{};
-  int alloc(int64_t cap, bool trace) {
-    p.cap = cap;
-    HIP_TRY(dalloc(&p.x, cap));
-    HIP_TRY(dalloc(&p.y, cap));
-    HIP_TRY(dalloc(&p.z, cap));
-    HIP_TRY(dalloc(&p.dx, cap));
-    HIP_TRY(dalloc(&p.dy, cap));
-    HIP_TRY(dalloc(&p.dz, cap));
-    HIP_TRY(dalloc(&p.e, cap));
-    HIP_TRY(dalloc(&p.nil0, cap));
-    HIP_TRY(dalloc(&p.nil1, cap));
-    HIP_TRY(dalloc(&p.nil2, cap));
-    HIP_TRY(dalloc(&p.rng, 6 * cap));
-    HIP_TRY(dalloc(&p.event, cap));
-    HIP_TRY(dalloc(&p.meta, cap));
-    HIP_TRY(dalloc(&p.nsteps, cap));
-    HIP_TRY(dalloc(&p.aed, cap));
-    HIP_TRY(dalloc(&p.avis, cap));
-    HIP_TRY(dalloc(&p.alen, cap));
-    if (trace) {
-      HIP_TRY(dalloc(&p.uid, cap));
-      HIP_TRY(dalloc(&p.tedep, cap));
-    }
-    return GXT_OK;
-  }
-  void release() {
-    void *ptrs[] = {p.x, p.y, p.z, p.dx, p.dy, p.dz, p.e, p.nil0, p.nil1, p.nil2, p.rng, p.event, p.meta,
-                    p.nsteps, p.aed, p.avis, p.alen, p.uid, p.tedep};
-    for (void *q : ptrs)
-      if (q) (void)hipFree(q);
-    p = Pool<R>{};
-  }
-};
-
 double now_ms(std::chrono::steady_clock::time_point t0) {
   return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
@@ -264,24 +223,23 @@ struct gxt_ctx {
   std::string err;
   int device = 0;
   hipStream_t stream = nullptr;
-  StepStreams ss{};  // main = stream, side stream; fork, join and entry events
   HostData hd;
   DeviceData dd;
   int precision = GXT_FP64;
   int64_t cap = 0;
   bool trace = false;
-  DevPool<double> pd[2];
-  DevPool<float> pf[2];
-  int parity = 0;
-  int grid = 1024;
-  int32_t *queues = nullptr;
-  int32_t *newlist = nullptr;
+  int groups = 256;          // workgroups of a step-loop launch
+  char *pages = nullptr;     // npages pages (gxt_types.h)
+  int npages = 0;
+  uint32_t *list = nullptr;  // rings of the pages with tracks and of the free ones
+  uint32_t *freel = nullptr;
+  uint32_t ring_mask = 0;
   Counters *cnt = nullptr;
-  Counters *hcnt = nullptr;  // pinned
+  Snapshot *hsnap = nullptr;  // pinned
   DevEvent *ev = nullptr;
   int *ev_live = nullptr;    // live tracks of event slot e at ev_live[e * kLiveStride]
   int *hev_live = nullptr;   // pinned: ev_live[e * kLiveStride] at [e], the host's snapshot
-  Counters *dhcnt = nullptr;  // device addresses of hcnt and hev_live
+  Snapshot *dhsnap = nullptr;  // device addresses of hsnap and hev_live
   int *dhev_live = nullptr;
   double *rows = nullptr;
   unsigned long long *spec = nullptr;
@@ -290,10 +248,7 @@ struct gxt_ctx {
   int64_t trace_cap = 0;
   hipEvent_t snap = nullptr;      // recorded after a round's counter snapshot
   size_t ev_snap = 0;             // profiling entries recorded before that snapshot
-  int64_t snap_iter = 0;          // step-loop iterations launched before that snapshot
-  int gen = 0;                    // counter generation of the next iteration's current pool
-  int snap_gen = 0;               // the same when the snapshot was queued
-  bool side_behind = true;        // main holds work the e-/e+ chain must follow (launch_side_sync)
+  int64_t snap_iter = 0;          // step-loop launches queued before that snapshot
   // non-uniform field
   gxt_field_map fmap;
   std::string fmap_path;
@@ -303,8 +258,9 @@ struct gxt_ctx {
   std::vector<gxt_placement> tree_pl;
   gxt_navigator *nav = nullptr;
   int32_t *cell = nullptr;
-  int transport_mode = 0;  // e-/e+ transport kernel (StepArgs::transport_mode)
-  int inner_steps = 4;     // StepArgs::inner_steps
+  int transport_mode = 0;  // LoopArgs::mode
+  int inner_steps = 4;     // LoopArgs::inner_steps
+  int lds_tables = 0, lds_bytes = 0;  // LoopArgs
   // jobs
   std::mutex mu;
   std::deque<std::unique_ptr<Job>> jobs;   // submitted, not finished (FIFO)
@@ -319,7 +275,8 @@ struct gxt_ctx {
   // kernel timing (profile_kernels)
   bool prof = false;
   int prof_level = 1;
-  std::vector<std::array<hipEvent_t, kStepEvents>> ev_free, ev_pending;
+  std::vector<std::array<hipEvent_t, 2>> ev_free, ev_pending;  // start and end of a launch
+  double loop_ms = 0;               // summed durations of the launches timed
   gxt_kernel_stats kst{};
   // stats
   int64_t iterations = 0;
@@ -333,32 +290,30 @@ struct gxt_ctx {
   std::atomic<int> serve_rc{GXT_OK};  // first error of the serving thread
   std::mutex err_mu;                  // guards err (the serving thread writes it)
 
-  StepArgs args() {
-    StepArgs a;
+  LoopArgs args() {
+    LoopArgs a;
     a.P = dd.P;
     a.cnt = cnt;
     a.ev = ev;
     a.ev_live = ev_live;
-    a.queues = queues;
-    a.newlist = newlist;
+    a.pages = pages;
+    a.list = list;
+    a.freel = freel;
+    a.mask = ring_mask;
+    a.npages = npages;
     a.rows.bins = rows;
     a.rows.spec = spec;
     a.rows.stride = row_stride;
-    a.rows.nrows = grid;
+    a.rows.nrows = groups;
     a.trace = trace_buf;
     a.trace_cap = trace_cap;
-    a.transport_mode = transport_mode;
+    a.mode = transport_mode;
     a.inner_steps = inner_steps;
-    a.gen = gen;
-    // the transports stage their tables in LDS when they take at most
-    // kLdsTablesMax bytes
-    const int nb = precision == GXT_FP32 ? (int)sizeof(Node32) : (int)sizeof(Node64);
-    for (int l = 0; l < 2; ++l) {
-      const int bytes = hd.params.lds_nodes[l] * nb;
-      // (the e-/e+ tables in LDS do not include the multiple-scattering ones)
-      const bool lds_ok = l == 0 || transport_mode == 0 || (transport_mode == 4 && !hd.params.msc);
-      a.lds_bytes[l] = (bytes > 0 && bytes <= kLdsTablesMax && lds_ok) ? bytes : 0;
-    }
+    a.lds_tables = lds_tables;
+    a.lds_bytes = lds_bytes;
+    a.groups = groups;
+    a.ticks = 100000;
+    a.prof = prof ? 1 : 0;
     return a;
   }
 
@@ -377,13 +332,6 @@ struct gxt_ctx {
 };
 
 namespace {
-
-// Live tracks of the pool of counter generation g.
-int64_t live_tracks(const Counters &h, int g) {
-  int64_t n = 0;
-  for (int s = 0; s < kStripes; ++s) n += (int64_t)h.ctr(g, kPool0, s) + h.ctr(g, kPool1, s);
-  return n;
-}
 
 // Estimated peak live tracks of an event, from its primaries' energy.
 // Peak live tracks expected of event e: 16 per primary plus the learned
@@ -474,70 +422,47 @@ int admit(gxt_ctx *c) {
   // jobs' primaries were copied to the device at submission, earlier on the
   // same stream); the slots of a new job belong to events without tracks, so
   // the look-ahead iterations still running do not touch them
-  if (!zero_ranges.empty() || !ranges.empty()) c->side_behind = true;
   for (auto &r : zero_ranges) {
     HIP_TRY(hipMemsetAsync(c->ev + r.first, 0, r.second * sizeof(DevEvent), c->stream));
     HIP_TRY(hipMemsetAsync(c->ev_live + (size_t)r.first * kLiveStride, 0, (size_t)r.second * kLiveStride * sizeof(int),
                            c->stream));
   }
-  const StepArgs a = c->args();
+  const LoopArgs a = c->args();
   for (const Range &r : ranges) {
     hipError_t e;
-    if (c->precision == GXT_FP32) {
-      PoolArgs<float> pa{c->pf[c->parity].p, c->pf[1 - c->parity].p};
-      e = r.prim ? launch_inject<float>(a, pa, r.prim, r.n, r.event_base, c->stream)
-                 : launch_inject<float>(a, pa, r.trk, r.n, r.event_base, c->stream);
-    } else {
-      PoolArgs<double> pa{c->pd[c->parity].p, c->pd[1 - c->parity].p};
-      e = r.prim ? launch_inject<double>(a, pa, r.prim, r.n, r.event_base, c->stream)
-                 : launch_inject<double>(a, pa, r.trk, r.n, r.event_base, c->stream);
-    }
+    // spread over the workgroups: pages of 64 once there are that many for each
+    const int fill = std::min(kPageTracks, (r.n + c->groups - 1) / c->groups);
+    if (c->precision == GXT_FP32)
+      e = r.prim ? launch_inject<float>(a, r.prim, r.n, fill, r.event_base, c->stream)
+                 : launch_inject<float>(a, r.trk, r.n, fill, r.event_base, c->stream);
+    else
+      e = r.prim ? launch_inject<double>(a, r.prim, r.n, fill, r.event_base, c->stream)
+                 : launch_inject<double>(a, r.trk, r.n, fill, r.event_base, c->stream);
     if (e != hipSuccess) return c->fail(GXT_EHIP, std::string("inject: ") + hipGetErrorString(e));
   }
   return GXT_OK;
 }
 
-int iterate(gxt_ctx *c, int k) {
-  StepArgs a = c->args();
-  // the e-/e+ chain follows what main holds that it must see (injections,
-  // cleared event slots; a snapshot, which must see no iteration in
-  // progress); otherwise it follows only the photon chains
-  if (c->side_behind) {
-    const hipError_t se = launch_side_sync(c->ss);
-    if (se != hipSuccess) return c->fail(GXT_EHIP, std::string("step: ") + hipGetErrorString(se));
-    c->side_behind = false;
-  }
-  for (int i = 0; i < k; ++i) {
-    a.gen = c->gen;
-    hipError_t e;
-    hipEvent_t *evs = nullptr;
-    if (c->prof) {
-      if (c->ev_free.empty()) {
-        // level 2 times only the photon interactions and the e-/e+ transport
-        // (kernels 1 and 3: events 2, 3, 6, 7); the events only time kernels,
-        // so they need no system-scope fence
-        std::array<hipEvent_t, kStepEvents> q{};
-        for (int k = 0; k < kStepEvents; ++k)
-          if (c->prof_level == 1 || k / 2 == 1 || k / 2 == 3)
-            HIP_TRY(hipEventCreateWithFlags(&q[k], hipEventDisableSystemFence));
-        c->ev_free.push_back(q);
-      }
-      c->ev_pending.push_back(c->ev_free.back());
-      c->ev_free.pop_back();
-      evs = c->ev_pending.back().data();
+// One launch of the step loop.
+int iterate(gxt_ctx *c) {
+  const LoopArgs a = c->args();
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (c->prof) {
+    if (c->ev_free.empty()) {
+      // the events only time kernels, so they need no system-scope fence
+      std::array<hipEvent_t, 2> q{};
+      for (int k = 0; k < 2; ++k) HIP_TRY(hipEventCreateWithFlags(&q[k], hipEventDisableSystemFence));
+      c->ev_free.push_back(q);
     }
-    if (c->precision == GXT_FP32) {
-      PoolArgs<float> pa{c->pf[c->parity].p, c->pf[1 - c->parity].p};
-      e = launch_step<float>(a, pa, c->grid, c->ss, evs);
-    } else {
-      PoolArgs<double> pa{c->pd[c->parity].p, c->pd[1 - c->parity].p};
-      e = launch_step<double>(a, pa, c->grid, c->ss, evs);
-    }
-    if (e != hipSuccess) return c->fail(GXT_EHIP, std::string("step: ") + hipGetErrorString(e));
-    c->parity = 1 - c->parity;
-    c->gen = gen_next(c->gen);
-    ++c->iterations;
+    c->ev_pending.push_back(c->ev_free.back());
+    c->ev_free.pop_back();
+    e0 = c->ev_pending.back()[0];
+    e1 = c->ev_pending.back()[1];
   }
+  const hipError_t e = c->precision == GXT_FP32 ? launch_loop<float>(a, c->stream, e0, e1)
+                                                : launch_loop<double>(a, c->stream, e0, e1);
+  if (e != hipSuccess) return c->fail(GXT_EHIP, std::string("step: ") + hipGetErrorString(e));
+  ++c->iterations;
   return GXT_OK;
 }
 
@@ -546,23 +471,19 @@ int iterate(gxt_ctx *c, int k) {
 int collect(gxt_ctx *c, bool &idle) {
   for (size_t qi = 0; qi < c->ev_snap; ++qi) {
     auto &q = c->ev_pending[qi];
-    // kernel j ran between events 2j and 2j + 1
-    float t[kStepKernels] = {};
-    for (int j = 0; j < kStepKernels; ++j)
-      if (q[2 * j] && q[2 * j + 1]) HIP_TRY(hipEventElapsedTime(&t[j], q[2 * j], q[2 * j + 1]));
-    c->kst.transport_neutral_ms += t[0];
-    c->kst.interact_neutral_ms += t[1];
-    c->kst.transport_charged_ms += t[3];
-    c->kst.interact_charged_ms += t[4];
-    c->kst.derive_ms += t[2] + t[5];
+    float t = 0;
+    HIP_TRY(hipEventElapsedTime(&t, q[0], q[1]));
+    c->loop_ms += t;
     c->kst.launches++;
     c->ev_free.push_back(q);
   }
   c->ev_pending.erase(c->ev_pending.begin(), c->ev_pending.begin() + c->ev_snap);
   c->ev_snap = 0;
-  const Counters &h = *c->hcnt;
-  if (h.overflow) return c->fail(GXT_ECAPACITY, "track pool or queue overflow (increase pool_capacity)");
-  const int64_t live = live_tracks(h, c->snap_gen);
+  const Snapshot &h = *c->hsnap;
+  const int64_t live = h.live;
+  // a launch that found tracks but no page to run a task with will not get further
+  if (h.overflow || (live > 0 && c->snap_iter > 0 && h.ran == 0))
+    return c->fail(GXT_ECAPACITY, "track pool overflow (increase pool_capacity)");
   c->max_live = std::max<int64_t>(c->max_live, live);
   std::vector<Job *> fin;
   {
@@ -658,15 +579,12 @@ int collect(gxt_ctx *c, bool &idle) {
   return GXT_OK;
 }
 
-// Iterations queued behind a round's counter snapshot: the device runs them
-// while the host reads the snapshot and plans the next admission.
-constexpr int kLookahead = 1;
-
-// One scheduling round of k iterations: admit, run k - kLookahead iterations,
-// snapshot the counters, queue the look-ahead iterations, then collect from
-// the snapshot.  Admission thus sees counts kLookahead iterations old; each
-// event in flight reserves its expected peak, which covers the growth.
-int round_trip(gxt_ctx *c, int k, bool &idle) {
+// One scheduling round: admit, launch the step loop, snapshot the counters,
+// queue a look-ahead launch, which the device runs while the host reads the
+// snapshot and plans the next admission, then collect from the snapshot.
+// Admission thus sees counts one launch old; each event in flight reserves
+// its expected peak, which covers the growth.
+int round_trip(gxt_ctx *c, bool &idle) {
   int rc = admit(c);
   if (rc) return rc;
   bool any = false;
@@ -676,34 +594,28 @@ int round_trip(gxt_ctx *c, int k, bool &idle) {
       if (jp->started) any = true;
   }
   if (any) {
-    rc = iterate(c, std::max(k - kLookahead, 1));
+    rc = iterate(c);
     if (rc) return rc;
   }
   // one kernel writes the snapshot into pinned memory; the event's
   // system-scope release makes it visible to the host
-  HIP_TRY(launch_snapshot(c->cnt, c->gen, c->ev_live, c->cfg.max_events, c->dhcnt, c->dhev_live, c->stream));
+  HIP_TRY(launch_snapshot(c->cnt, c->ev_live, c->cfg.max_events, c->dhsnap, c->dhev_live, c->stream));
   HIP_TRY(hipEventRecord(c->snap, c->stream));
-  c->side_behind = true;
   c->ev_snap = c->ev_pending.size();
   c->snap_iter = c->iterations;
-  c->snap_gen = c->gen;
   if (any) {
-    rc = iterate(c, kLookahead);
+    rc = iterate(c);
     if (rc) return rc;
   }
   HIP_TRY(hipEventSynchronize(c->snap));
   return collect(c, idle);
 }
 
-int iters_per_sync(gxt_ctx *c) {
-  return live_tracks(*c->hcnt, c->snap_gen) > 100000 ? 8 : 4;
-}
-
 void serve_loop(gxt_ctx *c) {
   (void)hipSetDevice(c->device);
   while (!c->stop.load()) {
     bool idle = true;
-    const int rc = round_trip(c, iters_per_sync(c), idle);
+    const int rc = round_trip(c, idle);
     if (rc) {
       c->serve_rc = rc;
       break;
@@ -719,10 +631,6 @@ void destroy_ctx(gxt_ctx *c) {
   }
   // look-ahead iterations may still be in flight
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  for (int i = 0; i < 2; ++i) {
-    c->pd[i].release();
-    c->pf[i].release();
-  }
   for (auto &q : c->ev_free)
     for (auto &x : q)
       if (x) (void)hipEventDestroy(x);
@@ -738,20 +646,17 @@ void destroy_ctx(gxt_ctx *c) {
     if (jp->dprims) (void)hipFree(jp->dprims);
     if (jp->dtracks) (void)hipFree(jp->dtracks);
   }
-  (void)hipFree(c->queues);
-  (void)hipFree(c->newlist);
+  (void)hipFree(c->pages);
+  (void)hipFree(c->list);
+  (void)hipFree(c->freel);
   (void)hipFree(c->cnt);
-  (void)hipHostFree(c->hcnt);
+  (void)hipHostFree(c->hsnap);
   (void)hipFree(c->ev);
   (void)hipFree(c->ev_live);
   (void)hipHostFree(c->hev_live);
   (void)hipFree(c->rows);
   (void)hipFree(c->spec);
   (void)hipFree(c->trace_buf);
-  if (c->ss.fork) (void)hipEventDestroy(c->ss.fork);
-  if (c->ss.join) (void)hipEventDestroy(c->ss.join);
-  if (c->ss.entry) (void)hipEventDestroy(c->ss.entry);
-  if (c->ss.side) (void)hipStreamDestroy(c->ss.side);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -1004,8 +909,7 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
   c->data_dir = cfg->data_dir;
   c->cfg.data_dir = c->data_dir.c_str();
   c->precision = cfg->precision;
-  // whole stripes
-  c->cap = (cfg->pool_capacity + kStripes - 1) / kStripes * kStripes;
+  c->cap = cfg->pool_capacity;
   c->trace = cfg->trace_tracks > 0;
   c->prof = cfg->profile_kernels > 0;
   c->prof_level = cfg->profile_kernels > 1 ? 2 : 1;
@@ -1014,19 +918,11 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
   rc = scratch_setup(c->device);
   if (rc) return rc;
   HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-  HIP_TRY(hipStreamCreateWithFlags(&c->ss.side, hipStreamNonBlocking));
-  // the chains' events order kernels of this device only: the end of a
-  // kernel already makes its writes visible to the device's later kernels,
-  // so they skip the system-scope fence (a cache write-back each)
-  const unsigned sync_flags = hipEventDisableTiming | hipEventDisableSystemFence;
-  HIP_TRY(hipEventCreateWithFlags(&c->ss.fork, sync_flags));
-  HIP_TRY(hipEventCreateWithFlags(&c->ss.join, sync_flags));
-  HIP_TRY(hipEventCreateWithFlags(&c->ss.entry, sync_flags));
   HIP_TRY(hipEventCreateWithFlags(&c->snap, hipEventDisableTiming));
-  c->ss.main = c->stream;
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
-  c->grid = std::max(cus, 1) * 4;
+  // a workgroup per CU, fewer for small pools (at least 4096 tracks each)
+  c->groups = (int)std::min<int64_t>(std::max(cus, 1), std::max<int64_t>(c->cap / 4096, 1));
   // physics data
   DevParams &P = c->hd.params;
   std::memset(&P, 0, sizeof(P));
@@ -1101,34 +997,49 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
   }
   rc = upload(c->hd, c->dd);
   if (rc) return rc;
-  // pools, queues, counters, tallies
-  for (int i = 0; i < 2; ++i) {
-    rc = c->precision == GXT_FP32 ? c->pf[i].alloc(c->cap, c->trace) : c->pd[i].alloc(c->cap, c->trace);
-    if (rc) return rc;
+  {
+    const int nb = c->precision == GXT_FP32 ? (int)sizeof(Node32) : (int)sizeof(Node64);
+    const int room = kLoopLds - kLoopLdsFixed;
+    const int b0 = P.lds_nodes[0] * nb, b1 = P.lds_nodes[1] * nb;
+    c->lds_tables = b0 + b1 <= room ? 2 : (b0 <= room ? 1 : 0);
+    c->lds_bytes = c->lds_tables == 2 ? b0 + b1 : (c->lds_tables == 1 ? b0 : 0);
   }
-  HIP_TRY(dalloc(&c->queues, (size_t)kNumQueues * c->cap));
-  HIP_TRY(dalloc(&c->newlist, (size_t)2 * c->cap));
+  // pages, counters, tallies: pages for the capacity, and for each workgroup
+  // but one what it holds open or partly filled
+  const int64_t np = (c->cap + kPageTracks - 1) / kPageTracks + (int64_t)(c->groups - 1) * 96;
+  c->npages = (int)np;
+  // (a launch reads a ring's entries while workgroups that have ended write
+  // behind them: twice the pages)
+  int64_t ring = 1;
+  while (ring < 2 * np) ring *= 2;
+  c->ring_mask = (uint32_t)(ring - 1);
+  HIP_TRY(dalloc(&c->pages, (size_t)np * (c->precision == GXT_FP32 ? page_bytes<float>() : page_bytes<double>())));
+  HIP_TRY(dalloc(&c->list, (size_t)ring));
+  HIP_TRY(dalloc(&c->freel, (size_t)ring));
   HIP_TRY(dalloc(&c->cnt, 1));
   HIP_TRY(hipMemset(c->cnt, 0, sizeof(Counters)));
-  HIP_TRY(hipHostMalloc((void **)&c->hcnt, sizeof(Counters), hipHostMallocDefault));
-  std::memset(c->hcnt, 0, sizeof(Counters));
+  HIP_TRY(hipHostMalloc((void **)&c->hsnap, sizeof(Snapshot), hipHostMallocDefault));
+  std::memset(c->hsnap, 0, sizeof(Snapshot));
   HIP_TRY(dalloc(&c->ev, cfg->max_events));
   HIP_TRY(hipMemset(c->ev, 0, sizeof(DevEvent) * cfg->max_events));
   HIP_TRY(dalloc(&c->ev_live, (size_t)cfg->max_events * kLiveStride));
   HIP_TRY(hipMemset(c->ev_live, 0, sizeof(int) * (size_t)cfg->max_events * kLiveStride));
   HIP_TRY(hipHostMalloc((void **)&c->hev_live, sizeof(int) * cfg->max_events, hipHostMallocDefault));
   std::memset(c->hev_live, 0, sizeof(int) * cfg->max_events);
-  HIP_TRY(hipHostGetDevicePointer((void **)&c->dhcnt, c->hcnt, 0));
+  HIP_TRY(hipHostGetDevicePointer((void **)&c->dhsnap, c->hsnap, 0));
   HIP_TRY(hipHostGetDevicePointer((void **)&c->dhev_live, c->hev_live, 0));
   c->row_stride = cfg->n_zbins + cfg->n_rbins + P.geo.nvol;
-  HIP_TRY(dalloc(&c->rows, (size_t)c->grid * c->row_stride));
-  HIP_TRY(hipMemset(c->rows, 0, sizeof(double) * c->grid * c->row_stride));
-  HIP_TRY(dalloc(&c->spec, (size_t)c->grid * 3 * kSpecBins));
-  HIP_TRY(hipMemset(c->spec, 0, sizeof(unsigned long long) * c->grid * 3 * kSpecBins));
+  HIP_TRY(dalloc(&c->rows, (size_t)c->groups * c->row_stride));
+  HIP_TRY(hipMemset(c->rows, 0, sizeof(double) * c->groups * c->row_stride));
+  HIP_TRY(dalloc(&c->spec, (size_t)c->groups * 3 * kSpecBins));
+  HIP_TRY(hipMemset(c->spec, 0, sizeof(unsigned long long) * c->groups * 3 * kSpecBins));
   if (c->trace) {
     c->trace_cap = 4000000;
     HIP_TRY(dalloc(&c->trace_buf, (size_t)12 * c->trace_cap));
   }
+  // (the clears above ran on the null stream, which the context's does not wait for)
+  HIP_TRY(hipDeviceSynchronize());
+  HIP_TRY(launch_pages_init(c->args(), c->stream));
   c->ev_used.assign(cfg->max_events, 0);
   c->ev_counted.assign(cfg->max_events, 0);
   HIP_TRY(hipDeviceSynchronize());
@@ -1227,7 +1138,7 @@ int gxt_run(gxt_ctx *c, int64_t max_iterations) {
   int rc = GXT_OK;
   for (;;) {
     bool idle = false;
-    rc = round_trip(c, iters_per_sync(c), idle);
+    rc = round_trip(c, idle);
     if (rc || idle) break;
     if (max_iterations > 0 && c->iterations - start >= max_iterations) break;
   }
@@ -1282,13 +1193,13 @@ int gxt_get_event_tallies(gxt_ctx *c, uint64_t job_id, gxt_event_tally *out, int
 int gxt_get_profiles(gxt_ctx *c, double *ez, double *er, double *ev) {
   if (!c) return set_err(GXT_EINVAL, "null context");
   HIP_TRY(hipStreamSynchronize(c->stream));
-  std::vector<double> rows((size_t)c->grid * c->row_stride);
+  std::vector<double> rows((size_t)c->groups * c->row_stride);
   HIP_TRY(hipMemcpy(rows.data(), c->rows, rows.size() * sizeof(double), hipMemcpyDeviceToHost));
   const int nz = c->cfg.n_zbins, nr = c->cfg.n_rbins, nv = c->hd.params.geo.nvol;
   if (ez) std::fill(ez, ez + nz, 0.0);
   if (er) std::fill(er, er + nr, 0.0);
   if (ev) std::fill(ev, ev + nv, 0.0);
-  for (int g = 0; g < c->grid; ++g) {
+  for (int g = 0; g < c->groups; ++g) {
     const double *r = rows.data() + (size_t)g * c->row_stride;
     for (int i = 0; i < nz; ++i)
       if (ez) ez[i] += r[i];
@@ -1314,10 +1225,10 @@ int gxt_volume_bins(gxt_ctx *c, int *n_bins, int32_t *cell) {
 int gxt_get_spectra(gxt_ctx *c, int64_t *counts) {
   if (!c || !counts) return set_err(GXT_EINVAL, "bad arguments");
   HIP_TRY(hipStreamSynchronize(c->stream));
-  std::vector<unsigned long long> s((size_t)c->grid * 3 * kSpecBins);
+  std::vector<unsigned long long> s((size_t)c->groups * 3 * kSpecBins);
   HIP_TRY(hipMemcpy(s.data(), c->spec, s.size() * sizeof(s[0]), hipMemcpyDeviceToHost));
   std::fill(counts, counts + 3 * kSpecBins, 0);
-  for (int g = 0; g < c->grid; ++g)
+  for (int g = 0; g < c->groups; ++g)
     for (int i = 0; i < 3 * kSpecBins; ++i) counts[i] += (int64_t)s[(size_t)g * 3 * kSpecBins + i];
   return GXT_OK;
 }
@@ -1325,9 +1236,7 @@ int gxt_get_spectra(gxt_ctx *c, int64_t *counts) {
 int gxt_get_stats(gxt_ctx *c, gxt_stats *o) {
   if (!c || !o) return set_err(GXT_EINVAL, "bad arguments");
   HIP_TRY(hipStreamSynchronize(c->stream));
-  // ~100 KB (three generations of striped counters): on the heap, not the caller's stack
-  auto hp = std::make_unique<Counters>();
-  Counters &h = *hp;
+  Counters h;
   HIP_TRY(hipMemcpy(&h, c->cnt, sizeof(h), hipMemcpyDeviceToHost));
   o->track_steps = (int64_t)h.total(kStatSteps);
   o->iterations = c->iterations;
@@ -1340,11 +1249,20 @@ int gxt_get_stats(gxt_ctx *c, gxt_stats *o) {
 int gxt_get_kernel_stats(gxt_ctx *c, gxt_kernel_stats *o) {
   if (!c || !o) return set_err(GXT_EINVAL, "bad arguments");
   HIP_TRY(hipStreamSynchronize(c->stream));
-  // ~100 KB (three generations of striped counters): on the heap, not the caller's stack
-  auto hp = std::make_unique<Counters>();
-  Counters &h = *hp;
+  Counters h;
   HIP_TRY(hipMemcpy(&h, c->cnt, sizeof(h), hipMemcpyDeviceToHost));
   *o = c->kst;
+  // the launches' time by part, as the waves spent it
+  const double all = (double)(h.total(kStatTimeN) + h.total(kStatTimeC) + h.total(kStatTimeIN) +
+                              h.total(kStatTimeIC) + h.total(kStatTimeD));
+  auto part = [&](int k) { return all > 0 ? c->loop_ms * (double)h.total(k) / all : 0.0; };
+  o->transport_charged_ms = part(kStatTimeC);
+  o->interact_neutral_ms = part(kStatTimeIN);
+  if (c->prof_level == 1) {
+    o->transport_neutral_ms = part(kStatTimeN);
+    o->interact_charged_ms = part(kStatTimeIC);
+    o->derive_ms = part(kStatTimeD);
+  }
   o->track_steps = (int64_t)h.total(kStatSteps);
   o->charged_steps = (int64_t)h.total(kStatStepsCharged);
   o->neutral_steps = (int64_t)(h.total(kStatSteps) - h.total(kStatStepsCharged));
@@ -1365,15 +1283,14 @@ int gxt_reset_tallies(gxt_ctx *c) {
   if (!c) return set_err(GXT_EINVAL, "null context");
   if (c->serving.load()) return c->fail(GXT_ESTATE, "reset while serving");
   HIP_TRY(hipStreamSynchronize(c->stream));
-  HIP_TRY(hipMemset(c->rows, 0, sizeof(double) * c->grid * c->row_stride));
-  HIP_TRY(hipMemset(c->spec, 0, sizeof(unsigned long long) * c->grid * 3 * kSpecBins));
-  // ~100 KB (three generations of striped counters): on the heap, not the caller's stack
-  auto hp = std::make_unique<Counters>();
-  Counters &h = *hp;
+  HIP_TRY(hipMemset(c->rows, 0, sizeof(double) * c->groups * c->row_stride));
+  HIP_TRY(hipMemset(c->spec, 0, sizeof(unsigned long long) * c->groups * 3 * kSpecBins));
+  Counters h;
   HIP_TRY(hipMemcpy(&h, c->cnt, sizeof(h), hipMemcpyDeviceToHost));
   std::memset(h.stat, 0, sizeof(h.stat));
   h.trace_n = 0;
   c->kst = gxt_kernel_stats{};
+  c->loop_ms = 0;
   HIP_TRY(hipMemcpy(c->cnt, &h, sizeof(h), hipMemcpyHostToDevice));
   c->iterations = 0;
   c->max_live = 0;
@@ -1386,9 +1303,7 @@ int gxt_reset_tallies(gxt_ctx *c) {
 int gxt_get_trace(gxt_ctx *c, double *out, int64_t max_records, int64_t *n_out) {
   if (!c || !n_out) return set_err(GXT_EINVAL, "bad arguments");
   HIP_TRY(hipStreamSynchronize(c->stream));
-  // ~100 KB (three generations of striped counters): on the heap, not the caller's stack
-  auto hp = std::make_unique<Counters>();
-  Counters &h = *hp;
+  Counters h;
   HIP_TRY(hipMemcpy(&h, c->cnt, sizeof(h), hipMemcpyDeviceToHost));
   const int64_t n = std::min<int64_t>((int64_t)h.trace_n, c->trace_cap);
   *n_out = n;

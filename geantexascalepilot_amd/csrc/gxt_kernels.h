@@ -19,30 +19,28 @@ struct TallyRows {
   int pad;
 };
 
-struct StepArgs {
+// Arguments of a step-loop launch (k_loop) and of the injection.
+struct LoopArgs {
   const DevParams *P;
   Counters *cnt;
   DevEvent *ev;
   int *ev_live;      // live tracks of event slot e at ev_live[e * kLiveStride]
-  int32_t *queues;  // kNumQueues x cap
-  int32_t *newlist; // next-pool slots of the tracks created this iteration: 2 lists of cap
-                    // (photon interactions, e-/e+ interactions)
+  char *pages;       // npages pages of page_bytes<R>()
+  uint32_t *list;    // ring of the pages with tracks, mask + 1 entries (Rings)
+  uint32_t *freel;   // ring of the free pages, mask + 1 entries
+  uint32_t mask;
+  int npages;
   TallyRows rows;
   double *trace;
   int64_t trace_cap;
-  int transport_mode;  // e-/e+ transport: 0 plain, 1 with multiple scattering, 2 field map with the
-                       // local helix, 3 RK45 stepper
-  int inner_steps;     // steps a track may take in one transport launch while it neither
-                       // interacts nor ends (>= 1)
-  int lds_bytes[2];    // > 0: the photon (0) and e-/e+ (1) transports stage their tables
-                       // (DevParams::lds_*) in that much dynamic LDS; 0: they read them in place
-  int gen;             // counter generation of the current pool (Counters)
-};
-
-template <class R>
-struct PoolArgs {
-  Pool<R> cur;
-  Pool<R> nxt;
+  int mode;          // transport: 0 plain, 1 with e-/e+ multiple scattering, 2 e-/e+ in a field map with
+                     // the local helix, 3 with the RK45 stepper, 4 the volume tree
+  int inner_steps;   // steps a track may take in one task while it neither interacts nor ends (>= 1)
+  int lds_tables;    // tables staged in LDS: 0 none, 1 the photon ones, 2 all
+  int lds_bytes;     // dynamic LDS they take
+  int groups;        // workgroups launched (at most)
+  int ticks;         // 100 MHz ticks after which a workgroup starts no further task
+  int prof;          // accumulate the time of the loop's parts (kStatTime*)
 };
 
 struct SampleArgs {
@@ -59,37 +57,34 @@ struct SampleArgs {
   double *sec_dir;
 };
 
-// Streams of the step loop: main carries the photon chain, side the e-/e+
-// chain.  After its chain of an iteration each stream records its event
-// (main: fork, side: join) and waits for the other's, so an iteration's
-// chains both follow the previous iteration's, and the two waits run side
-// by side.  launch_side_sync makes side follow all work queued on main so
-// far (injections, snapshots) through the event entry.
-struct StepStreams {
-  hipStream_t main, side;
-  hipEvent_t fork, join, entry;
-};
-
-// One step-loop iteration of kStepKernels kernels: photon transport,
-// interactions and RNG derivation of their new tracks (main), then the same
-// for e-/e+ (side).  With ev (kStepEvents events, null entries not
-// recorded) kernel j takes its start and end times into ev[2j], ev[2j + 1].
-constexpr int kStepKernels = 6;
-constexpr int kStepEvents = 2 * kStepKernels;
+// One launch of the step loop (gxt_loop.h): a.groups workgroups of
+// kLoopBlock threads.  e0, e1 (may be null) take the kernel's start and end.
+constexpr int kLoopBlock = 512;
+// LDS of a launch beside its dynamic tables, and all of a workgroup's.
+constexpr int kLoopLdsFixed = 30 * 1024;
+constexpr int kLoopLds = 160 * 1024;
 template <class R>
-hipError_t launch_step(const StepArgs &a, const PoolArgs<R> &pa, int grid, const StepStreams &s,
-                       hipEvent_t *ev = nullptr);
-hipError_t launch_side_sync(const StepStreams &s);
+hipError_t launch_loop(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
+// The launch of one transport mode (each mode is compiled in a unit of its own).
+template <class R, int kMode>
+hipError_t launch_loop_mode(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
 // Injects n primaries or tracks in flight (In = gxt_primary, gxt_track) from
-// device memory; event slots are prim[i].event + event_base.
+// device memory as pages of up to `fill` tracks; event slots are
+// prim[i].event + event_base.
 template <class R, class In>
-hipError_t launch_inject(const StepArgs &a, const PoolArgs<R> &pa, const In *prim, int n, int event_base,
-                         hipStream_t st);
+hipError_t launch_inject(const LoopArgs &a, const In *prim, int n, int fill, int event_base, hipStream_t st);
+// Clears the rings and makes all pages free.
+hipError_t launch_pages_init(const LoopArgs &a, hipStream_t st);
 
-// The host's snapshot, into pinned host memory (device addresses out_cnt,
-// out_live): out_live[e] = ev_live[e * kLiveStride] for e < n, the pool
-// counts of counter generation g and the overflow flag into out_cnt.
-hipError_t launch_snapshot(const Counters *cnt, int g, const int *ev_live, int n, Counters *out_cnt, int *out_live,
+// What the host reads of the device's state after a launch.
+struct Snapshot {
+  long long live;    // tracks in pages
+  unsigned int ran;  // workgroups that ran a task in the last launch
+  int overflow;
+};
+// The host's snapshot, into pinned host memory (device addresses out,
+// out_live): out_live[e] = ev_live[e * kLiveStride] for e < n.
+hipError_t launch_snapshot(const Counters *cnt, const int *ev_live, int n, Snapshot *out, int *out_live,
                            hipStream_t st);
 hipError_t launch_rng_init(const DevParams *P, const uint32_t *seed, const uint64_t *idx, int n, uint32_t *out,
                            hipStream_t st);

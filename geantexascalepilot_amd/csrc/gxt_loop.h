@@ -1,0 +1,803 @@
+// gxt_loop.h -- the step loop as one persistent kernel.
+//
+// A launch runs on one workgroup of 8 waves per CU.  Each workgroup takes a
+// share of the pages with tracks (64 tracks that wait for the same task:
+// photon transport, e-/e+ transport, or one of the interactions) and of the
+// free pages, and its waves work on their own: a wave takes a page, runs its
+// task on the 64 tracks, and writes the tracks that come out, by value, into
+// the workgroup's open page of their next task; a page that is full joins the
+// ready pages of its task.  What the waves share (ready, open and free pages)
+// is in LDS under one lock, so a step costs no launch, no wait for the slowest
+// wave of a grid, no returning atomic in device memory and no gather: pages
+// are read and filled with contiguous accesses.  After its time a workgroup
+// hands its pages back; the next launch shares them out again.
+//
+// Every event's result is independent of the order of the tasks: a track's
+// randomness is its own substream, and tallies are sums.
+#pragma once
+
+#include <hip/hip_ext.h>
+#include <hip/hip_runtime.h>
+
+#include "gxt_step.h"
+
+namespace gxt {
+
+constexpr int kLoopWaves = kLoopBlock / 64;
+constexpr int kLP = 512;    // pages a workgroup holds at once, at most
+constexpr int kTake = 256;  // of which with tracks at its start, at most
+constexpr int kMinFree = 72;  // free pages per workgroup at its start, at least (one workgroup: what there is):
+                              // an open page for each type and what 8 running tasks may need
+
+// Shared state of a workgroup.  A page is known by its local number lp < kLP.
+struct Sched {
+  int lock;
+  int nfree;   // local pages on freestk
+  int need;    // pages that running tasks may still take from it
+  int active;  // running tasks
+  int stop;    // no further tasks
+  int ran;     // a task has run
+  int commits; // tasks that have ended: what a waiting wave watches
+  int head[kTypes], tail[kTypes];  // ready pages of a type: rq[type][head .. tail), positions mod kLP
+  int open[kTypes], fill[kTypes];  // the type's open page (-1: none) and its entries given out
+  uint16_t rq[kTypes][kLP];
+  uint16_t freestk[kLP];
+  uint16_t cnt[kLP];    // tracks written into a page
+  uint32_t gpage[kLP];  // local page -> page
+  int16_t dest[kLoopWaves][kTypes][4];  // pages of a wave's outputs by type, in order of entry / 64; -1: none
+  unsigned int base[4];
+  unsigned long long stat[16];
+};
+
+// The lock is taken by lane 0 for its wave.  Its holder never waits for
+// another wave, so every wait for it ends.
+__device__ __forceinline__ void sched_lock(Sched &S) {
+  if (lane() == 0)
+    while (__hip_atomic_exchange(&S.lock, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+      __builtin_amdgcn_s_sleep(1);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+__device__ __forceinline__ void sched_unlock(Sched &S) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  if (lane() == 0) __hip_atomic_store(&S.lock, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Pages a task of n tracks may take beside its own, which it frees first:
+// photons go on to 4 types, e-/e+ to 7 (at most one new page each); an
+// interaction gives up to 3 photons and 3 e-/e+ per track.
+__device__ __forceinline__ int task_need(int type, int n) {
+  return type == 0 ? 3 : (type == 1 ? 6 : 2 * ((63 + 3 * n) >> 6) - 1);
+}
+
+struct Task {
+  int type, lp, n;  // type < 0: the wave ends
+};
+
+// The next task of a wave: a ready page of the type that has most of them;
+// with none ready, the fullest open page that no wave is writing to; with
+// neither and no task running, or after the launch's time, none.  While other
+// waves run tasks the wave waits for what they produce.
+__device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
+  const int l = lane();
+  for (;;) {
+    const bool late = wall_clock64() - t_end >= 0;
+    sched_lock(S);
+    int key = -1;
+    if (l < kTypes) {
+      const int r = S.tail[l] - S.head[l];
+      const int o = S.open[l], f = S.fill[l];
+      if (r > 0)
+        key = (1 << 16) | (r << 4) | l;
+      else if (o >= 0 && f > 0 && (int)S.cnt[o] == f)
+        key = (f << 4) | l;
+    }
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1) key = max(key, __shfl_xor(key, d, 64));
+    key = __builtin_amdgcn_readfirstlane(key);
+    const int active = __builtin_amdgcn_readfirstlane(S.active);
+    const int seen = __builtin_amdgcn_readfirstlane(S.commits);
+    const bool stop = late || __builtin_amdgcn_readfirstlane(S.stop) != 0;
+    Task t;
+    t.type = -1;
+    t.lp = t.n = 0;
+    bool wait = false;
+    if (stop || key < 0) {
+      wait = !stop && active > 0;
+      if (late && l == 0) S.stop = 1;
+    } else {
+      const int type = key & 15;
+      int lp = 0, n = 0;
+      const bool ready = (key >> 16) != 0;
+      if (l == type) {
+        lp = ready ? S.rq[type][S.head[type] & (kLP - 1)] : S.open[type];
+        n = S.cnt[lp];
+      }
+      lp = __builtin_amdgcn_readlane(lp, type);
+      n = __builtin_amdgcn_readlane(n, type);
+      const int need = task_need(type, n);
+      if (__builtin_amdgcn_readfirstlane(S.nfree) - __builtin_amdgcn_readfirstlane(S.need) < need) {
+        // short of pages: a running task may free some, otherwise the
+        // workgroup hands its pages back
+        wait = active > 0;
+        if (!wait && l == 0) S.stop = 1;
+      } else {
+        t.type = type;
+        t.lp = lp;
+        t.n = n;
+        if (l == type) {
+          if (ready) {
+            S.head[type] = S.head[type] + 1;
+          } else {
+            S.open[type] = -1;
+            S.fill[type] = 0;
+          }
+        }
+        if (l == 0) {
+          S.active = active + 1;
+          S.need = S.need + need;
+          S.ran = 1;
+        }
+      }
+    }
+    sched_unlock(S);
+    if (!wait) return t;
+    // until a task ends (one is running), without the lock
+    while (__hip_atomic_load(&S.commits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == seen)
+      __builtin_amdgcn_s_sleep(2);
+  }
+}
+
+// Frees the task's page and gives out entries: lane t < kTypes asks for n
+// entries of type t and gets its first entry f; entry e of the type is slot
+// e % 64 of page S.dest[wave][t][e / 64].  With too few free pages (which
+// task_need excludes) the entries have no page (-1) and the overflow is
+// reported.
+__device__ __forceinline__ int reserve(Sched &S, Counters *cnt, const Task &task, int n) {
+  const int l = lane();
+  const int w = (int)(threadIdx.x >> 6);
+  sched_lock(S);
+  int nfree = S.nfree;
+  if (l == 0) S.freestk[nfree] = (uint16_t)task.lp;
+  ++nfree;
+  int f = 0, o = -1, np = 0;
+  if (l < kTypes && n > 0) {
+    o = S.open[l];
+    f = S.fill[l];
+    np = ((f + n + 63) >> 6) - (o >= 0 ? 1 : 0);
+  }
+  int incl = np;
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) {
+    const int t = __shfl_up(incl, d, 64);
+    if (l >= d) incl += t;
+  }
+  const int total = __builtin_amdgcn_readlane(incl, kTypes - 1);
+  const bool ok = total <= nfree;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // the freed page's number before it is read below
+  if (l < kTypes && n > 0) {
+    int top = nfree - 1 - (incl - np);
+    int last = o;
+    const int have = o >= 0 ? 1 : 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      int pg = ok && j == 0 && have ? o : -1;
+      if (ok && j >= have && j - have < np) {
+        pg = S.freestk[top--];
+        S.cnt[pg] = 0;
+        last = pg;
+      }
+      S.dest[w][l][j] = (int16_t)pg;
+    }
+    if (ok) {
+      const int rem = (f + n) & 63;
+      S.open[l] = rem ? last : -1;
+      S.fill[l] = rem;
+    }
+  }
+  if (l == 0) {
+    S.nfree = ok ? nfree - total : nfree;
+    S.need = S.need - task_need(task.type, task.n);
+    if (!ok) atomicOr(&cnt->overflow, 1);
+  }
+  sched_unlock(S);
+  return f;
+}
+
+// The wave's outputs are written: lane t's n entries of type t from entry f
+// on.  Pages that are now whole become ready; the task has ended.
+__device__ __forceinline__ void commit(Sched &S, int f, int n) {
+  const int l = lane();
+  const int w = (int)(threadIdx.x >> 6);
+  // the tracks' stores before the other waves can see the pages
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  sched_lock(S);
+  if (l < kTypes && n > 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = min(f + n, 64 * (j + 1)) - max(f, 64 * j);
+      const int pg = S.dest[w][l][j];
+      if (c > 0 && pg >= 0) {
+        const int have = S.cnt[pg] + c;
+        S.cnt[pg] = (uint16_t)have;
+        if (have == kPageTracks) {
+          const int t = S.tail[l];
+          S.rq[l][t & (kLP - 1)] = (uint16_t)pg;
+          S.tail[l] = t + 1;
+        }
+      }
+    }
+  }
+  if (l == 0) {
+    S.active = S.active - 1;
+    S.commits = S.commits + 1;
+  }
+  sched_unlock(S);
+}
+
+template <class R>
+__device__ __forceinline__ char *page_at(const LoopArgs &a, const Sched &S, int lp) {
+  return a.pages + (int64_t)S.gpage[lp] * page_bytes<R>();
+}
+
+// ------------------------------------------------------------------ staging
+extern __shared__ uint4 tab_lds[];
+
+// DevParams into LDS in 8-byte words: every thread issues its loads before its
+// stores, so the copy costs one memory latency.
+constexpr int kParamWords = (int)(sizeof(DevParams) / 8);
+constexpr int kParamPer = (kParamWords + kLoopBlock - 1) / kLoopBlock;
+
+__device__ __forceinline__ void stage_params(const DevParams *P, DevParams &sP) {
+  static_assert(sizeof(DevParams) % 8 == 0, "DevParams is copied in 8-byte words");
+  const unsigned long long *src = reinterpret_cast<const unsigned long long *>(P);
+  unsigned long long *dst = reinterpret_cast<unsigned long long *>(&sP);
+  unsigned long long v[kParamPer];
+#pragma unroll
+  for (int j = 0; j < kParamPer; ++j) {
+    const int k = j * kLoopBlock + (int)threadIdx.x;
+    if (k < kParamWords) v[j] = src[k];
+  }
+#pragma unroll
+  for (int j = 0; j < kParamPer; ++j) {
+    const int k = j * kLoopBlock + (int)threadIdx.x;
+    if (k < kParamWords) dst[k] = v[j];
+  }
+}
+
+// n 16-byte words from src to LDS dst by the workgroup's threads, four loads
+// in flight per thread before their stores.
+__device__ __forceinline__ void copy_words16(uint4 *dst, const uint4 *src, int n) {
+  for (int k = (int)threadIdx.x; k < n; k += 4 * kLoopBlock) {
+    const int k1 = k + kLoopBlock, k2 = k + 2 * kLoopBlock, k3 = k + 3 * kLoopBlock;
+    const uint4 v0 = src[k];
+    const uint4 v1 = k1 < n ? src[k1] : v0;
+    const uint4 v2 = k2 < n ? src[k2] : v0;
+    const uint4 v3 = k3 < n ? src[k3] : v0;
+    dst[k] = v0;
+    if (k1 < n) dst[k1] = v1;
+    if (k2 < n) dst[k2] = v2;
+    if (k3 < n) dst[k3] = v3;
+  }
+}
+
+// The physics vectors of layout `layout` (one node span per material slot)
+// into dynamic LDS from 16-byte word dst on; returns the word after them.
+template <class R>
+__device__ __forceinline__ int stage_tables(const DevParams *P, int layout, int dst) {
+  using T = typename NodeType<R>::T;
+  constexpr int w = sizeof(T) / sizeof(uint4);
+  const uint4 *src = reinterpret_cast<const uint4 *>(NodeType<R>::global(P));
+  for (int s = 0; s < kMaxSlots; ++s) {
+    const int n16 = P->lds_cnt[layout][s] * w;
+    copy_words16(tab_lds + dst, src + (int64_t)P->lds_src[layout][s] * w, n16);
+    dst += n16;
+  }
+  return dst;
+}
+
+// ------------------------------------------------------------------ transport task
+// The steps of one page of photons (kCharged false) or e-/e+; the species
+// class is a compile-time constant so each variant carries only its own code.
+// kMode as LoopArgs::mode.
+template <class R, bool kCharged, int kMode, class NS>
+__device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParams *P, const NS &N, Sched &S,
+                                               Hist &wh, const Task &task) {
+  const bool trace = P->trace_events > 0;
+  const R mine = (R)P->tracking_cut;
+  constexpr int kG = kMode == 4 ? 1 : 0;  // geo_cell form
+  const bool active = lane() < task.n;
+  TrackRegs<R> t;
+  int q = -1;
+  bool survive = false, annihilate = false, dies = false, killed = false, escaped = false;
+  int nsub = 0;  // steps taken in this task
+  double edep = 0.0;
+  if (active) {
+    load_track(PageSlot<R>(page_at<R>(a, S, task.lp), lane()), t, trace);
+    if (!kCharged) t.species = 0;
+    // species as a value the compiler can bound: 0 here, or 1 / 2 there
+    const int sp = kCharged ? (t.species == 2 ? 2 : 1) : 0;
+    const bool charged = kCharged;
+    // a track keeps stepping while it neither interacts nor ends, up to
+    // a.inner_steps steps
+    for (;;) {
+      survive = false;
+      edep = 0.0;
+      Dep dA, dB;  // along-step loss (mid-step, pre-step volume); local deposit at the end point
+      // material slot of the track's volume; -1 (tree form only): vacuum, no
+      // physics, the track flies to the next boundary
+      const int mslot = P->geo.slot[geo_cell<kG>(P->geo, t.vol)];
+      const bool vac = kMode == 4 && mslot < 0;
+      const DevMaterial &m = P->mat[vac ? 0 : mslot];
+      R xs0 = R(0), xs1 = R(0), xs2 = R(0);
+      double bestd = kHuge;
+      int sel = -1;
+      double lam1 = kMscNone;
+      // the step's table lookups share log(E) and the e-/e+ range at E
+      const R le = m_log(t.e);
+      R range = R(0);
+      if (!vac) {
+        gpil<0>(P, N, m, sp, t.e, le, t.nil0, xs0, t.rng, bestd, sel);
+        gpil<1>(P, N, m, sp, t.e, le, t.nil1, xs1, t.rng, bestd, sel);
+        if (sp != 1) gpil<2>(P, N, m, sp, t.e, le, t.nil2, xs2, t.rng, bestd, sel);
+        if (charged) {
+          const double al = (double)along_limit(N, m, sp == 2, t.e, le, mine, range);
+          if (al < bestd) {
+            bestd = al;
+            sel = -1;
+          }
+        }
+        // multiple scattering: its step limit; then the geometric length of the
+        // true path is propagated (the step is the true path for interaction
+        // lengths and loss); its tables are not among those in LDS
+        if constexpr (kMode != 0) {
+          if (charged && P->msc) {
+            lam1 = msc_lambda1<R>(Nodes<R>(P), m, sp == 2, t.e, le);
+            if (lam1 < kMscNone) {
+              const double saf = kMode == 4 ? nav_safety(P->geo.nav, t.vol, t.pos) : safety(P->geo, t.vol, t.pos);
+              const double tlim = fmax(fmax(kMscFacRange * fmax((double)range, lam1), kMscFacSafety * saf), kMscTmin);
+              if (tlim < bestd) {
+                bestd = tlim;
+                sel = -1;
+              }
+            }
+          }
+        }
+      }
+      const double pre[3] = {t.pos[0], t.pos[1], t.pos[2]};
+      const int prevol = t.vol;
+      double step = 0.0;
+      int status;
+      if constexpr (kMode != 0) {
+        const bool msc_on = lam1 < kMscNone;
+        const double request = msc_on ? msc_geom(bestd, lam1) : bestd;
+        double gstep = 0.0;
+        if constexpr (kMode == 4)
+          status = propagate_tree<R>(P, sp, t.e, t.pos, t.dir, t.vol, request, gstep);
+        else if constexpr (kMode == 2)
+          status = propagate_general<R, GXT_STEPPER_HELIX>(P, sp, t.e, t.pos, t.dir, t.vol, request, gstep);
+        else if constexpr (kMode == 3)
+          status = propagate_general<R, GXT_STEPPER_RK45>(P, sp, t.e, t.pos, t.dir, t.vol, request, gstep);
+        else
+          status = propagate<R>(P, sp, t.e, t.pos, t.dir, t.vol, request, gstep);
+        step = msc_on ? (status == kPhysics ? bestd : msc_true(gstep, lam1, bestd)) : gstep;
+      } else {
+        status = propagate<R>(P, sp, t.e, t.pos, t.dir, t.vol, bestd, step);
+      }
+      if (xs0 > R(0)) t.nil0 -= (R)step * xs0;
+      if (xs1 > R(0)) t.nil1 -= (R)step * xs1;
+      if (xs2 > R(0)) t.nil2 -= (R)step * xs2;
+      t.nsteps++;
+      if (charged && !vac) {
+        t.alen += step;
+        R loss = R(0);
+        t.e = along_doit(N, m, t.species == 2, t.e, le, range, (R)step, mine, loss);
+        const double mid[3] = {0.5 * (pre[0] + t.pos[0]), 0.5 * (pre[1] + t.pos[1]), 0.5 * (pre[2] + t.pos[2])};
+        dA.add<kG>(P, t, (double)loss, mid, prevol);
+        edep += (double)loss;
+        if constexpr (kMode != 0) {
+          if (lam1 < kMscNone && status != kEscaped && t.e > R(0) && step > 0.0)
+            msc_deflect<R>(step / lam1, t.dir, t.rng);
+        }
+      }
+      int tproc = status == kPhysics ? sel : (status == kBoundary ? -2 : (status == kEscaped ? -3 : -1));
+      if (status == kPhysics && sel < 0) tproc = -1;
+      if (status == kEscaped) {
+        if (trace) trace_rec(a, t, tproc, edep);
+        escaped = true;
+        dies = true;
+      } else if (t.e <= R(0)) {
+        if (trace) trace_rec(a, t, tproc, edep);
+        annihilate = t.species == 2;
+        dies = !annihilate;
+      } else if (status == kPhysics && sel >= 0) {
+        t.set_nil(sel, R(-1));
+        q = queue_of(t.species, sel);
+      } else {
+        if (trace) trace_rec(a, t, tproc, edep);
+        if (t.e < mine) {
+          dB.add<kG>(P, t, (double)t.e, t.pos, t.vol);
+          annihilate = t.species == 2;
+          dies = !annihilate;
+        } else if (t.nsteps >= P->max_steps) {
+          dB.add<kG>(P, t, (double)t.e, t.pos, t.vol);
+          killed = true;
+          dies = true;
+        } else {
+          survive = true;
+        }
+      }
+      // positron at rest: its two photons are made by the interaction task
+      if (annihilate) q = kQueueAtRest;
+      dA.flush(wh);
+      dB.flush(wh);
+      ++nsub;
+      if (!survive || nsub >= a.inner_steps) break;
+    }
+  }
+  // the track's next task, and its entry among the wave's tracks of that type
+  const int type = q >= 0 ? 2 + q : (survive ? (kCharged ? 1 : 0) : -1);
+  const unsigned long long lt = (1ULL << lane()) - 1;
+  int rank = 0, n = 0;
+  constexpr int kOut = kCharged ? kNumQueues - 3 + 1 : 3 + 1;
+#pragma unroll
+  for (int k = 0; k < kOut; ++k) {
+    const int ty = k == 0 ? (kCharged ? 1 : 0) : (kCharged ? 4 + k : 1 + k);
+    const unsigned long long m = __ballot(type == ty);
+    if (type == ty) rank = (int)__popcll(m & lt);
+    if (lane() == ty) n = (int)__popcll(m);
+  }
+  const int f = reserve(S, a.cnt, task, n);
+  const int e = __shfl(f, type >= 0 ? type : 0, 64) + rank;
+  if (type >= 0) {
+    const int pg = S.dest[threadIdx.x >> 6][type][e >> 6];
+    if (pg >= 0) {
+      const PageSlot<R> p(page_at<R>(a, S, pg), e & 63);
+      store_track(p, t, trace);
+      if (trace && q >= 0 && q != kQueueAtRest) p.f64(kPtedep) = edep;
+    }
+  }
+  commit(S, f, n);
+  // what needs no answer
+  if (active) {
+    if (escaped) unsafeAtomicAdd(&a.ev[t.event].leak, (double)t.e);
+    if (killed) atomicAdd(&S.stat[kStatKilled], 1ULL);
+    if (dies) {
+      retire(a, t);
+      atomicAdd(&a.ev_live[(int64_t)t.event * kLiveStride], -1);
+    }
+  }
+  const int steps = __builtin_amdgcn_readlane(wave_incl_scan(nsub), 63);
+  if (lane() == 0) {
+    atomicAdd(&S.stat[kStatSteps], (unsigned long long)steps);
+    if (kCharged) atomicAdd(&S.stat[kStatStepsCharged], (unsigned long long)steps);
+    atomicAdd(&S.stat[kCharged ? kStatLoaded1 : kStatLoaded0], (unsigned long long)task.n);
+  }
+}
+
+// ------------------------------------------------------------------ interaction task
+// Fate of a secondary: 1 pushed (>= tracking cut), 0 deposited, 2 deposited
+// and, a positron, annihilated at rest.
+template <class R>
+__device__ __forceinline__ int sec_fate(const DevParams *P, TrackRegs<R> &t, Dep &dp, const Sec<R> &s, R mine,
+                                        int &outN, int &outC, int &nannih) {
+  if (s.e < mine) {
+    dp.add(P, t, (double)s.e, t.pos, t.vol);
+    if (s.species == 2) {
+      ++nannih;
+      outN += 2;
+      return 2;
+    }
+    return 0;
+  }
+  if (s.species == 0)
+    outN++;
+  else
+    outC++;
+  return 1;
+}
+
+// One page of queue q: sample the final states, write the survivors and the
+// tracks created, each with its RNG state.
+template <class R>
+__device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams *P, Sched &S, Hist &wh,
+                                              const Task &task, long long &t_derive) {
+  const bool trace = P->trace_events > 0;
+  const R mine = (R)P->tracking_cut;
+  const int q = task.type - 2;
+  const bool active = lane() < task.n;
+  TrackRegs<R> t;
+  Interaction<R> o;
+  o.nsec = 0;
+  int fate0 = 0, fate1 = 0;
+  bool survive = false, prim_rest = false, killed = false, pair = false;
+  int outN = 0, outC = 0, nannih = 0;
+  Dep dp;  // every deposit of an interaction is at the track's position
+  if (active) {
+    const PageSlot<R> p(page_at<R>(a, S, task.lp), lane());
+    load_track(p, t, trace);
+    if (q == kQueueAtRest) {
+      // positron stopped by the continuous loss or the tracking cut
+      ++nannih;
+      prim_rest = true;
+      outN = 2;
+      t.e = R(0);
+    } else {
+      // an interacting track is in a material (the tree form's vacuum has no physics)
+      const DevMaterial &m = P->mat[max(P->geo.slot[geo_cell<2>(P->geo, t.vol)], 0)];
+      if (q < 3)
+        sample_neutral<R>(P, m, q, t.e, t.dir, t.rng, o);
+      else
+        sample_charged<R>(P, m, q, t.e, t.dir, t.rng, o);
+      pair = q == 1 && o.nsec == 2;
+      if (q == 7) ++nannih;
+      dp.add(P, t, (double)o.edep, t.pos, t.vol);
+      t.e = o.ekin;
+      t.dir[0] = o.d[0];
+      t.dir[1] = o.d[1];
+      t.dir[2] = o.d[2];
+      if (trace) trace_rec(a, t, queue_proc(q), p.f64(kPtedep) + (double)o.edep);
+      if (o.nsec > 0) fate0 = sec_fate(P, t, dp, o.sec[0], mine, outN, outC, nannih);
+      if (o.nsec > 1) fate1 = sec_fate(P, t, dp, o.sec[1], mine, outN, outC, nannih);
+    }
+    if (t.e > R(0)) {
+      if (t.e < mine) {
+        dp.add(P, t, (double)t.e, t.pos, t.vol);
+        if (t.species == 2) {
+          ++nannih;
+          prim_rest = true;
+          outN += 2;
+        }
+      } else if (t.nsteps >= P->max_steps) {
+        dp.add(P, t, (double)t.e, t.pos, t.vol);
+        killed = true;
+      } else {
+        survive = true;
+        if (t.species == 0)
+          outN++;
+        else
+          outC++;
+      }
+    }
+  }
+  const int inclN = wave_incl_scan(outN), inclC = wave_incl_scan(outC);
+  const int totN = __builtin_amdgcn_readlane(inclN, 63), totC = __builtin_amdgcn_readlane(inclC, 63);
+  const int n = lane() == 0 ? totN : (lane() == 1 ? totC : 0);
+  const int f = reserve(S, a.cnt, task, n);
+  int kN = __builtin_amdgcn_readlane(f, 0) + inclN - outN;
+  int kC = __builtin_amdgcn_readlane(f, 1) + inclC - outC;
+  const int w = (int)(threadIdx.x >> 6);
+  const long long t0 = a.prof ? wall_clock64() : 0;
+  // new tracks in the oracle's draw order: secondary 0, secondary 1, then the
+  // primary's annihilation at rest (two back-to-back 511 keV photons,
+  // isotropic); the survivor last
+#pragma unroll 1
+  for (int k = 0; k < 3; ++k) {
+    const int fate = k == 0 ? fate0 : (k == 1 ? fate1 : (prim_rest ? 2 : 0));
+    if (!__any(fate != 0)) continue;
+    const Sec<R> &s1 = o.sec[1];
+    int species = k == 1 ? s1.species : o.sec[0].species;
+    R e = k == 1 ? s1.e : o.sec[0].e;
+    R d0 = k == 1 ? s1.d[0] : o.sec[0].d[0], d1 = k == 1 ? s1.d[1] : o.sec[0].d[1],
+      d2 = k == 1 ? s1.d[2] : o.sec[0].d[2];
+    if (fate == 2) {
+      const double cost = 2.0 * t.rng.uniform() - 1.0;
+      const double sint = sqrt((1.0 - cost) * (1.0 + cost));
+      const double phi = kTwoPi * t.rng.uniform();
+      d0 = (R)(sint * m_cos(phi));
+      d1 = (R)(sint * m_sin(phi));
+      d2 = (R)cost;
+      e = (R)kMe;
+      species = 0;
+    }
+#pragma unroll 1
+    for (int j = 0; j < 2; ++j) {
+      const bool go = fate == 2 || (fate == 1 && j == 0);
+      if (!__any(go)) break;
+      if (go) {
+        const uint64_t uid = child_substream(t.rng);
+        uint32_t rng[6];
+        substream_state(P, uid, rng);
+        const int idx = species == 0 ? kN++ : kC++;
+        const int pg = S.dest[w][species == 0 ? 0 : 1][idx >> 6];
+        if (pg >= 0)
+          store_new(PageSlot<R>(page_at<R>(a, S, pg), idx & 63), t, species, e, d0, d1, d2, uid, rng, trace);
+        atomicAdd(&a.ev[t.event].nsec[species], 1ULL);
+        spectrum(wh, species, (double)e);
+        d0 = -d0;
+        d1 = -d1;
+        d2 = -d2;
+      }
+    }
+  }
+  if (survive) {
+    const int idx = t.species == 0 ? kN : kC;
+    const int pg = S.dest[w][t.species == 0 ? 0 : 1][idx >> 6];
+    if (pg >= 0) store_track(PageSlot<R>(page_at<R>(a, S, pg), idx & 63), t, trace);
+  }
+  commit(S, f, n);
+  if (a.prof) t_derive += wall_clock64() - t0;
+  if (active) {
+    dp.flush(wh);
+    if (pair) atomicAdd(&a.ev[t.event].npairs, 1ULL);
+    if (nannih) atomicAdd(&a.ev[t.event].nannihil, (unsigned long long)nannih);
+    if (killed) atomicAdd(&S.stat[kStatKilled], 1ULL);
+    if (!survive) retire(a, t);
+    if (outN + outC != 1) atomicAdd(&a.ev_live[(int64_t)t.event * kLiveStride], outN + outC - 1);
+  }
+  const int made = totN + totC - (int)__popcll(__ballot(survive));
+  if (lane() == 0) {
+    atomicAdd(&S.stat[kStatInteractions], (unsigned long long)task.n);
+    if (q < 3) atomicAdd(&S.stat[kStatInteractions0], (unsigned long long)task.n);
+    atomicAdd(&S.stat[kStatCreated], (unsigned long long)made);
+    if (q < 3) atomicAdd(&S.stat[kStatCreated0], (unsigned long long)made);
+  }
+}
+
+// ------------------------------------------------------------------ the loop
+// kLds: the tables in LDS (LoopArgs::lds_tables).
+template <class R, int kMode, int kLds>
+__global__ __launch_bounds__(kLoopBlock, 2) void k_loop(LoopArgs a) {
+  __shared__ Sched S;
+  __shared__ DevParams sP;
+  __shared__ Hist wh;
+  static_assert(sizeof(Sched) + sizeof(DevParams) + sizeof(Hist) <= kLoopLdsFixed, "LDS beside the tables");
+  const int tid = (int)threadIdx.x;
+  Rings &rg = a.cnt->rings;
+  // what the launch shares out (the heads and tails move when its last
+  // workgroup ends): workgroup b of `groups` takes pages with tracks lhead +
+  // b + groups j, j < kTake, and `nf` free pages from fhead + b nf on
+  const unsigned long long lhead = rg.lhead, ltail = rg.ltail, fhead = rg.fhead, ftail = rg.ftail;
+  const long long have = (long long)(ltail - lhead);
+  const int b = (int)blockIdx.x;
+  const long long spare = (long long)(ftail - fhead);
+  const int groups = (int)max(min(min((long long)gridDim.x, have), spare / kMinFree), 1LL);
+  const long long taken = min(have, (long long)groups * kTake);
+  const int nt = b < groups ? (int)((taken - b + groups - 1) / groups) : 0;
+  const int nf = (int)min(spare / groups, (long long)(kLP - kTake));
+  if (nt > 0) {
+    const long long t_end = wall_clock64() + a.ticks;
+    hist_clear(wh);
+    stage_params(a.P, sP);
+    int dyn = 0;
+    if (kLds >= 1) dyn = stage_tables<R>(a.P, 0, dyn);
+    if (kLds >= 2) (void)stage_tables<R>(a.P, 1, dyn);
+    if (tid < kTypes) {
+      S.head[tid] = S.tail[tid] = 0;
+      S.open[tid] = -1;
+      S.fill[tid] = 0;
+    }
+    if (tid < 16) S.stat[tid] = 0;
+    if (tid == 0) {
+      S.lock = S.need = S.active = S.stop = S.ran = S.commits = 0;
+      S.nfree = nf;
+    }
+    __syncthreads();
+    // local pages: [0, nt) with tracks, [nt, nt + nf) free
+    int start_live = 0;
+    for (int j = tid; j < nt + nf; j += kLoopBlock) {
+      if (j < nt) {
+        const uint32_t en = a.list[(uint32_t)(lhead + (unsigned)b + (unsigned long long)groups * j) & a.mask];
+        const int type = (int)(en >> 6 & 15u), n = (int)(en & 63u) + 1;
+        S.gpage[j] = en >> 10;
+        S.cnt[j] = (uint16_t)n;
+        start_live += n;
+        // the first partial page of a type is filled further, the others are
+        // tasks as they are
+        if (n < kPageTracks && atomicCAS(&S.open[type], -1, j) == -1)
+          S.fill[type] = n;
+        else
+          S.rq[type][atomicAdd(&S.tail[type], 1)] = (uint16_t)j;
+      } else {
+        S.gpage[j] = a.freel[(uint32_t)(fhead + (unsigned long long)b * nf + (j - nt)) & a.mask];
+        S.cnt[j] = 0;
+        S.freestk[j - nt] = (uint16_t)j;
+      }
+    }
+    __syncthreads();
+    {
+      const DevParams *P = &sP;
+      using T = typename NodeType<R>::T;
+      const NodesT<R, (kLds >= 1)> N0 = [&] {
+        if constexpr (kLds >= 1)
+          return NodesT<R, true>(reinterpret_cast<const T *>(tab_lds), P->hints);
+        else
+          return NodesT<R, false>(P);
+      }();
+      const NodesT<R, (kLds >= 2)> N1 = [&] {
+        if constexpr (kLds >= 2)
+          return NodesT<R, true>(reinterpret_cast<const T *>(tab_lds) + P->lds_nodes[0], P->hints);
+        else
+          return NodesT<R, false>(P);
+      }();
+      for (;;) {
+        const Task task = next_task(S, t_end);
+        if (task.type < 0) break;
+        const long long t0 = a.prof ? wall_clock64() : 0;
+        long long td = 0;
+        if (task.type == 0)
+          transport_task<R, false, (kMode == 4 ? 4 : 0)>(a, P, N0, S, wh, task);
+        else if (task.type == 1)
+          transport_task<R, true, kMode>(a, P, N1, S, wh, task);
+        else
+          interact_task<R>(a, P, S, wh, task, td);
+        if (a.prof && lane() == 0) {
+          const int part = task.type < 2 ? kStatTimeN + task.type : (task.type < 5 ? kStatTimeIN : kStatTimeIC);
+          atomicAdd(&S.stat[part], (unsigned long long)(wall_clock64() - t0 - td));
+          if (td) atomicAdd(&S.stat[kStatTimeD], (unsigned long long)td);
+        }
+      }
+    }
+    __syncthreads();
+    // hand back: pages with tracks (ready, then open ones) and free pages
+    if (tid == 0) {
+      int np = 0;
+      for (int t = 0; t < kTypes; ++t) np += S.tail[t] - S.head[t] + (S.open[t] >= 0 && S.fill[t] > 0 ? 1 : 0);
+      const unsigned long long lp = atomicAdd(&rg.lpush, (unsigned long long)np);
+      const unsigned long long fp = atomicAdd(&rg.fpush, (unsigned long long)S.nfree);
+      S.base[0] = (uint32_t)(ltail + lp);
+      S.base[1] = (uint32_t)(ftail + fp);
+      if (S.ran) atomicAdd(&rg.ran, 1u);
+    }
+    __syncthreads();
+    uint32_t at = S.base[0];
+    int live = -start_live;
+    for (int t = 0; t < kTypes; ++t) {
+      const int h = S.head[t], n = S.tail[t] - h;
+      for (int j = tid; j < n; j += kLoopBlock) {
+        const int lp = S.rq[t][(h + j) & (kLP - 1)];
+        const int c = S.cnt[lp];
+        a.list[(at + (uint32_t)j) & a.mask] = page_entry(S.gpage[lp], t, c);
+        live += c;
+      }
+      at += (uint32_t)n;
+      if (S.open[t] >= 0 && S.fill[t] > 0) {
+        if (tid == 0) {
+          a.list[at & a.mask] = page_entry(S.gpage[S.open[t]], t, S.fill[t]);
+          live += S.fill[t];
+        }
+        ++at;
+      }
+    }
+    for (int j = tid; j < S.nfree; j += kLoopBlock) a.freel[(S.base[1] + (uint32_t)j) & a.mask] = S.gpage[S.freestk[j]];
+    live = __builtin_amdgcn_readlane(wave_incl_scan(live), 63);
+    if (lane() == 0 && live != 0) atomicAdd((unsigned long long *)&rg.live, (unsigned long long)(long long)live);
+    hist_flush(a.rows, a.P, wh);
+    if (tid < kNumStats && S.stat[tid]) atomicAdd(&a.cnt->stat[b % kStripes][tid], S.stat[tid]);
+  }
+  // the last workgroup to end moves the rings on
+  __threadfence();
+  __syncthreads();
+  if (tid == 0 && atomicAdd(&rg.done, 1u) == gridDim.x - 1) {
+    const unsigned long long lp = atomicExch(&rg.lpush, 0ULL), fp = atomicExch(&rg.fpush, 0ULL);
+    rg.lhead = lhead + (unsigned long long)taken;
+    rg.ltail = ltail + lp;
+    rg.fhead = fhead + (unsigned long long)groups * nf;
+    rg.ftail = ftail + fp;
+    rg.ran_last = atomicExch(&rg.ran, 0u);
+    rg.done = 0;
+  }
+}
+
+template <class R, int kMode, int kLds>
+static hipError_t launch_one(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  auto kernel = k_loop<R, kMode, kLds>;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     kLoopLds - kLoopLdsFixed);
+  if (attr != hipSuccess) return attr;
+  if (e0 || e1)
+    hipExtLaunchKernelGGL(kernel, dim3(a.groups), dim3(kLoopBlock), (uint32_t)a.lds_bytes, st, e0, e1, 0, a);
+  else
+    hipLaunchKernelGGL(kernel, dim3(a.groups), dim3(kLoopBlock), (size_t)a.lds_bytes, st, a);
+  return hipGetLastError();
+}
+
+template <class R, int kMode>
+hipError_t launch_loop_mode(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  if (a.lds_tables == 2) return launch_one<R, kMode, 2>(a, st, e0, e1);
+  if (a.lds_tables == 1) return launch_one<R, kMode, 1>(a, st, e0, e1);
+  return launch_one<R, kMode, 0>(a, st, e0, e1);
+}
+
+}  // namespace gxt

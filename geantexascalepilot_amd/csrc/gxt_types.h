@@ -18,14 +18,8 @@ constexpr int kQueueAtRest = 8;
 constexpr int kSpecBins = 64;     // secondary spectrum bins per species
 constexpr int kInvRangeHints = 256;  // search-hint bins per inverse-range vector
 constexpr int kMaxShells = 128;   // shell binding energies over the elements of the slots
-// The pool, the interaction queues and the new-track list are split into
-// kStripes stripes of cap / kStripes slots, each with its own counters;
-// workgroup b appends to stripe b % kStripes, so each counter takes 1/kStripes
-// of the atomics (the workgroups of one stripe share an XCD under the
-// round-robin dispatch of workgroups to XCDs).  Measured on the 10 GeV e- /
-// PbWO4 batch: 16 stripes 2 % faster than 12 and 3 % faster than 32 (whose
-// per-stripe prefixes cost more than the atomics they spread), 5 % faster
-// than 8 in FP64 and 10 % in FP32.
+// Statistics counters are spread over kStripes rows (workgroup b adds to row
+// b % kStripes).
 constexpr int kStripes = 16;
 // Words per row of the substream jump tables: a 3x3 matrix padded to 48 bytes.
 constexpr int kJumpRow = 12;
@@ -211,57 +205,57 @@ struct DevParams {
   int lds_nodes[2];
 };
 
-// Structure-of-arrays track pool.  R is the precision of the physics state
-// (double, or float in the precision form); positions stay FP64.
+// ------------------------------------------------------------------ track pages
+// Live tracks sit in pages of 64, one structure-of-arrays block per page, so a
+// wave loads or fills a page with contiguous accesses.  Every page holds
+// tracks that wait for the same task: type 0 photon transport, 1 e-/e+
+// transport, 2 + q the interaction queue q.  R is the precision of the
+// physics state (double, or float in the precision form); positions and
+// tallies stay FP64.
+constexpr int kPageTracks = 64;
+constexpr int kTypes = 2 + kNumQueues;
+enum PageF64 { kPx = 0, kPy, kPz, kPaed, kPavis, kPalen,  // deposit, visible deposit, charged length of the track
+               kPtedep, kPuid,                            // tracing only: step deposit, substream index
+               kPageF64 };
+enum PageR { kPdx = 0, kPdy, kPdz, kPe, kPnil0, kPnil1, kPnil2, kPageR };
+enum PageU32 { kPrng = 0, kPevent = 6, kPmeta, kPnsteps, kPageU32 };  // meta: volume | species << 16
 template <class R>
-struct Pool {
-  int64_t cap;
-  double *x, *y, *z;
-  R *dx, *dy, *dz;
-  R *e;
-  R *nil0, *nil1, *nil2;
-  uint32_t *rng;      // 6 planes of cap words
-  int32_t *event;     // event slot
-  int32_t *meta;      // volume | species << 16
-  int32_t *nsteps;
-  double *aed, *avis, *alen;  // per-track tallies (deposit, visible deposit, charged length),
-                              // added to the event once, when the track dies
-  uint64_t *uid;      // substream index (written only while tracing)
-  double *tedep;      // step deposit carried to the interaction kernel (tracing only)
+__host__ __device__ constexpr int page_bytes() {
+  return kPageTracks * (kPageF64 * 8 + kPageR * (int)sizeof(R) + kPageU32 * 4);
+}
+
+// A page with tracks, as the step loop's list holds it between launches.
+__host__ __device__ constexpr uint32_t page_entry(uint32_t page, int type, int count) {
+  return page << 10 | (uint32_t)type << 6 | (uint32_t)(count - 1);
+}
+constexpr uint32_t kMaxPages = 1u << 22;
+
+// The step loop's page lists in device memory, two rings of `mask + 1` entries
+// (at least twice the pages, so that what a launch writes never reaches what it
+// has still to read):
+// list (page_entry of the pages with tracks, [lhead, ltail)) and free pages
+// ([fhead, ftail)).  A launch of the loop takes entries from the heads and
+// writes behind the tails (counted by lpush, fpush); its last workgroup to end
+// moves the heads and tails, so that a launch reads only what was written
+// before it began.
+struct alignas(128) Rings {
+  unsigned long long lhead, ltail, fhead, ftail;
+  unsigned long long lpush, fpush;
+  unsigned int done;        // workgroups of the launch that have ended
+  unsigned int ran, ran_last;  // workgroups that ran a task in this launch, in the last one
+  long long live;           // tracks in pages
 };
 
-// Device counters of the step loop, in three generations.  Generation g
-// holds, per stripe, the photon and e-/e+ track counts of a pool (kPool0,
-// kPool1) and the queue and new-track-list counts of the iteration that
-// fills that pool.  Iteration i reads the pool of generation g = i mod 3,
-// fills generation g + 1 (mod 3) and clears generation g + 2, which the
-// next iteration fills: no kernel between iterations moves counts from one
-// set to another, so each chain of the loop waits only for the other
-// chain's last kernel.  The counters of kind k of stripe s in generation g
-// are addressed ctr(g, k, s); each stripe's counters sit on cache lines no
-// other stripe uses, so the returning atomics of one stripe's workgroups
-// never wait behind another stripe's.  Statistics are per stripe as well
-// (summed by the host).
-enum CounterKind { kPool0 = 0, kPool1 = 1, kQ0 = 2, kNew0 = 2 + kNumQueues, kNew1 = 3 + kNumQueues,
-                   kNumKinds = 4 + kNumQueues };
-constexpr int kGens = 3;
-constexpr int kKindStride = 32;      // ints between the counters of one stripe
-constexpr int kStripeStride = 512;  // ints between stripes
-__host__ __device__ constexpr int gen_next(int g) { return g == kGens - 1 ? 0 : g + 1; }
 enum StatKind { kStatSteps = 0, kStatStepsCharged, kStatKilled, kStatInteractions, kStatCreated, kStatLoaded0,
-                kStatLoaded1, kStatInteractions0, kStatCreated0, kNumStats };
+                kStatLoaded1, kStatInteractions0, kStatCreated0,
+                // wave time (100 MHz ticks) in the loop's parts, with profiling on
+                kStatTimeN, kStatTimeC, kStatTimeIN, kStatTimeIC, kStatTimeD, kNumStats };
 struct alignas(256) Counters {
-  int32_t c[kGens * kStripes * kStripeStride];
+  Rings rings;
   unsigned long long stat[kStripes][16];  // 128 B per stripe
-  int32_t overflow;        // a pool or queue write would have gone out of range
+  int32_t overflow;        // the pages ran out: the tracks that found none are lost
   int32_t pad[31];
   unsigned long long trace_n; // trace records written
-  __host__ __device__ int32_t &ctr(int g, int kind, int s) {
-    return c[(g * kStripes + s) * kStripeStride + kind * kKindStride];
-  }
-  __host__ __device__ int32_t ctr(int g, int kind, int s) const {
-    return c[(g * kStripes + s) * kStripeStride + kind * kKindStride];
-  }
   __host__ __device__ unsigned long long total(int k) const {
     unsigned long long t = 0;
     for (int s = 0; s < kStripes; ++s) t += stat[s][k];

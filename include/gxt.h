@@ -97,10 +97,10 @@ typedef struct gxt_config {
   int32_t max_jobs;         /* concurrent job slots                                 */
   int32_t trace_tracks;     /* >0: record the first trace_steps steps of tracks     */
   int32_t trace_steps;
-  int32_t profile_kernels;  /* 1: time every step-loop launch with HIP events; 2: only the
-                               photon interaction and e-/e+ transport launches (the two
-                               largest kernels).  The events take each kernel's start and
-                               end from its own dispatch (no packets between kernels). */
+  int32_t profile_kernels;  /* 1: time the parts of the step loop; 2: report only the photon
+                               interactions and the e-/e+ transport.  Events take each launch's
+                               start and end from its own dispatch, the waves' clocks share
+                               that time out to the parts. */
   const char *data_dir;     /* directory holding the physics data files             */
   const char *field_map;    /* NULL: the uniform field above; else a cylindrical (r, z)
                                field-map file (see gxt_field_map_load), which replaces it */
@@ -152,7 +152,7 @@ typedef struct gxt_event_tally {
 /* Run statistics. */
 typedef struct gxt_stats {
   int64_t track_steps;      /* total track-steps                       */
-  int64_t iterations;       /* step-loop iterations                    */
+  int64_t iterations;       /* launches of the step loop               */
   int64_t max_live;         /* peak live tracks                        */
   int64_t killed_by_limit;  /* tracks killed by max_steps              */
   double wall_ms;           /* device time of the last gxt_run          */
@@ -160,24 +160,24 @@ typedef struct gxt_stats {
 
 /* Kernel timings of the step loop, accumulated while profile_kernels is set. */
 typedef struct gxt_kernel_stats {
-  double transport_neutral_ms; /* summed durations of the photon transport launches    */
-  double transport_charged_ms; /* summed durations of the e-/e+ transport launches     */
-  double interact_neutral_ms;  /* summed durations of the photon interaction launches  */
-  double interact_charged_ms;  /* summed durations of the e-/e+ interaction launches   */
-  double derive_ms;       /* summed durations of the new-track RNG derivation       */
-  double advance_ms;      /* 0: the step loop has no counter-advance launch (its
-                             counters rotate over generations); kept for layout */
-  int64_t launches;       /* step-loop iterations timed (one launch of each kernel) */
-  int64_t track_steps;    /* tracks stepped (one per live track per iteration)     */
+  /* the launches' durations, shared out by the time the waves spent in each part */
+  double transport_neutral_ms; /* photon transport                                     */
+  double transport_charged_ms; /* e-/e+ transport                                      */
+  double interact_neutral_ms;  /* photon interactions                                  */
+  double interact_charged_ms;  /* e-/e+ interactions                                   */
+  double derive_ms;       /* tracks created and survivors: RNG states and stores    */
+  double advance_ms;      /* 0 (the step loop has no such part); kept for layout    */
+  int64_t launches;       /* step-loop launches timed                               */
+  int64_t track_steps;    /* steps of tracks                                        */
   int64_t neutral_steps;  /* of which photon steps                                 */
   int64_t charged_steps;  /* of which e-/e+ steps                                  */
-  int64_t interactions;   /* tracks sampled by the interaction kernel              */
-  int64_t created;        /* tracks created by the interaction kernel              */
+  int64_t interactions;   /* tracks sampled by the interactions                    */
+  int64_t created;        /* tracks created by the interactions                    */
   int32_t record_bytes;   /* bytes of one track record in the pool                 */
   int32_t pad;
-  int64_t neutral_loaded; /* track records read by the photon transport launches (a
-                             track takes up to several steps per launch)          */
-  int64_t charged_loaded; /* track records read by the e-/e+ transport launches   */
+  int64_t neutral_loaded; /* track records read by the photon transport (a track
+                             takes up to several steps per task)                  */
+  int64_t charged_loaded; /* track records read by the e-/e+ transport            */
   int64_t neutral_interactions; /* of interactions, photons sampled               */
   int64_t neutral_created;      /* of created, tracks the photon interactions made */
 } gxt_kernel_stats;
@@ -193,7 +193,7 @@ typedef struct gxt_job_result {
   double admit_ms;
   double done_ms;
   int64_t track_steps;
-  int64_t iterations;     /* step-loop iterations from the job's admission to the
+  int64_t iterations;     /* step-loop launches from the job's admission to the
                              counter snapshot that found its last event finished */
 } gxt_job_result;
 
@@ -293,7 +293,8 @@ typedef struct gxt_track {
  * that holds the position) before anything is queued.  No reference
  * counterpart beyond the hand-off point cited above. */
 int gxt_submit_tracks(gxt_ctx *ctx, const gxt_track *tracks, int n, int n_events, uint64_t job_id);
-/* Run the step loop until every submitted job has finished (replaces
+/* Run the step loop until every submitted job has finished, in launches of
+ * about a millisecond, at most max_iterations of them and one more (replaces
  * ProxyDeviceManager::DoStep/DoGPIL, ProxyDeviceManager.cpp:206-276, and the
  * host wave loop DoStep<>, proxy/test/test_BasicCpuTransport.cpp:517-550).
  * max_iterations <= 0 means no limit. */
