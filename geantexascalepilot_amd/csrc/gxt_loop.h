@@ -81,7 +81,7 @@ struct Task {
 __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
   const int l = lane();
   for (;;) {
-    const bool late = wall_clock64() - t_end >= 0;
+    const bool over = wall_clock64() - t_end >= 0;
     sched_lock(S);
     int key = -1;
     if (l < kTypes) {
@@ -97,6 +97,8 @@ __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
     key = __builtin_amdgcn_readfirstlane(key);
     const int active = __builtin_amdgcn_readfirstlane(S.active);
     const int seen = __builtin_amdgcn_readfirstlane(S.commits);
+    // (a launch runs a task wherever it can, so that one that ran none is short of pages)
+    const bool late = over && __builtin_amdgcn_readfirstlane(S.ran) != 0;
     const bool stop = late || __builtin_amdgcn_readfirstlane(S.stop) != 0;
     Task t;
     t.type = -1;
@@ -654,7 +656,7 @@ __global__ __launch_bounds__(kLoopBlock, 2) void k_loop(LoopArgs a) {
   const int groups = (int)max(min(min((long long)gridDim.x, have), spare / kMinFree), 1LL);
   const long long taken = min(have, (long long)groups * kTake);
   const int nt = b < groups ? (int)((taken - b + groups - 1) / groups) : 0;
-  const int nf = (int)min(spare / groups, (long long)(kLP - kTake));
+  const int nf = have > 0 ? (int)min(spare / groups, (long long)(kLP - kTake)) : 0;
   if (nt > 0) {
     const long long t_end = wall_clock64() + a.ticks;
     hist_clear(wh);

@@ -96,3 +96,17 @@ def test_interrupted_run_continues(gpu_lib):
         assert np.array_equal(whole[k], parts[k]), k
     for k in ENERGIES:
         np.testing.assert_allclose(parts[k], whole[k], rtol=1e-9, atol=1e-9, err_msg=k)
+
+
+def test_every_page_comes_back(gpu_lib):
+    """A pool of one workgroup has 64 pages: 300 short jobs, one after the
+    other, each with launches that find no track left, need every page back."""
+    cfg = abi.config_lead_block(max_events=1, pool_capacity=4096)
+    p = gpu_lib.make_primaries(cfg.seed, abi.GAMMA, 5.0, 5.0, 0.0, 1)
+    with gpu_lib.Transport(cfg) as t:
+        steps = set()
+        for job in range(300):
+            t.submit(p, job)
+            t.run()
+            steps.add(int(t.event_tallies(job, 1)["n_steps"][0]))
+    assert len(steps) == 1
