@@ -236,34 +236,46 @@ struct Rng {
   template <class R> __device__ __forceinline__ R u() { return (R)uniform(); }
 };
 
-// a * b mod m for a, b < m < 2^32, exactly: the 64-bit product wraps
-// correctly, the FP64 quotient estimate (below 2^32) is within one of the
-// true quotient, and one correction each way restores the residue (no 64-bit
-// division; the operands stay 32-bit, so each conversion is one instruction).
-__device__ __forceinline__ uint32_t mulmod32(uint32_t a, uint32_t b, uint32_t m, double invm) {
-  const uint64_t p = (uint64_t)a * b;
-  const uint32_t q = (uint32_t)floor((double)a * (double)b * invm);
-  int64_t r = (int64_t)(p - (uint64_t)q * m);
-  if (r < 0) r += (int64_t)m;
-  if (r >= (int64_t)m) r -= (int64_t)m;
-  return (uint32_t)r;
+// Products modulo m = 2^32 - c (c = 209 and 22853 for the two components) need
+// no division: 2^32 = c (mod m), so a 64-bit value x folds to (x >> 32) c +
+// (x & (2^32 - 1)) <= (c + 1)(2^32 - 1).  A row of a matrix times a vector is
+// a chain of multiply-adds with a fold after each: with entries M <= m - 1 and
+// v <= 2^32 - 1, M v plus a folded value is at most 2^64 - 2^32, so no sum
+// overflows.  A last fold leaves less than 2^32 + c^2, brought below 2^32
+// by one conditional + c; the result is congruent but not reduced, as the
+// vector of the next product may be (v <= 2^32 - 1).  Seven multiply-adds per
+// row in place of three full modular products with FP64 quotients (about 22
+// instructions each).
+template <uint32_t c>
+__device__ __forceinline__ uint64_t fold(uint64_t x) {
+  return (uint64_t)(uint32_t)(x >> 32) * c + (uint32_t)x;
 }
-
-// (M v) mod m for 32-bit residues (M row-major 3x3).
-__device__ __forceinline__ void matvec_mod(const uint32_t M[9], uint32_t v[3], uint32_t m, double invm) {
-  uint32_t r[3];
+template <uint32_t c>
+__device__ __forceinline__ uint32_t dot3_fold(uint32_t M0, uint32_t M1, uint32_t M2, const uint32_t v[3]) {
+  uint64_t x = fold<c>((uint64_t)M0 * v[0]);
+  x = fold<c>((uint64_t)M1 * v[1] + x);
+  x = fold<c>((uint64_t)M2 * v[2] + x);
+  x = fold<c>(x);
+  return (uint32_t)x + ((x >> 32) ? c : 0u);
+}
+// v = M v, congruent mod m (M row-major 3x3 of residues).
+template <uint32_t c>
+__device__ __forceinline__ void matvec_fold(const uint32_t M[9], uint32_t v[3]) {
+  const uint32_t r0 = dot3_fold<c>(M[0], M[1], M[2], v);
+  const uint32_t r1 = dot3_fold<c>(M[3], M[4], M[5], v);
+  const uint32_t r2 = dot3_fold<c>(M[6], M[7], M[8], v);
+  v[0] = r0;
+  v[1] = r1;
+  v[2] = r2;
+}
+// The residue of v <= 2^32 - 1 (m > 2^31: one subtraction).
+template <uint32_t c>
+__device__ __forceinline__ void reduce3(uint32_t v[3]) {
+  constexpr uint32_t m = 0u - c;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    uint64_t acc = (uint64_t)mulmod32(M[i * 3], v[0], m, invm) + mulmod32(M[i * 3 + 1], v[1], m, invm) +
-                   mulmod32(M[i * 3 + 2], v[2], m, invm);
-    if (acc >= m) acc -= m;
-    if (acc >= m) acc -= m;
-    r[i] = (uint32_t)acc;
-  }
-  v[0] = r[0];
-  v[1] = r[1];
-  v[2] = r[2];
+  for (int k = 0; k < 3; ++k) v[k] = v[k] >= m ? v[k] - m : v[k];
 }
+constexpr uint32_t kC1 = 209u, kC2 = 22853u;  // 2^32 - m1, 2^32 - m2
 
 // One jump-table row: three 16-byte loads of a 48-byte aligned row.
 __device__ __forceinline__ void jump_row(const uint32_t *T, int c, int k, int d, uint32_t M[9]) {
@@ -299,9 +311,11 @@ __device__ __forceinline__ void jump_substream(const uint32_t *T, const uint32_t
     uint32_t M1[9], M2[9];
     jump_row(T, 0, k, d, M1);
     jump_row(T, 1, k, d, M2);
-    matvec_mod(M1, v1, 4294967087u, 1.0 / 4294967087.0);
-    matvec_mod(M2, v2, 4294944443u, 1.0 / 4294944443.0);
+    matvec_fold<kC1>(M1, v1);
+    matvec_fold<kC2>(M2, v2);
   }
+  reduce3<kC1>(v1);
+  reduce3<kC2>(v2);
 }
 
 __device__ __forceinline__ void substream_state(const DevParams *P, uint64_t idx, uint32_t out[6]) {
