@@ -57,11 +57,10 @@ struct SampleArgs {
   double *sec_dir;
 };
 
-// One launch of the step loop (gxt_loop.h): a.groups workgroups of
-// kLoopBlock threads.  e0, e1 (may be null) take the kernel's start and end.
-constexpr int kLoopBlock = 512;
+// One launch of the step loop (gxt_loop.h) on a.groups workgroups.  e0, e1 (may
+// be null) take the kernel's start and end.
 // LDS of a launch beside its dynamic tables, and all of a workgroup's.
-constexpr int kLoopLdsFixed = 30 * 1024;
+constexpr int kLoopLdsFixed = 31 * 1024;
 constexpr int kLoopLds = 160 * 1024;
 template <class R>
 hipError_t launch_loop(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);

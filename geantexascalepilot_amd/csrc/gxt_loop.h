@@ -7,7 +7,7 @@
 // task on the 64 tracks, and writes the tracks that come out, by value, into
 // the workgroup's open page of their next task; a page that is full joins the
 // ready pages of its task.  What the waves share (ready, open and free pages)
-// is in LDS under one lock, so a step costs no launch, no wait for the slowest
+// is in LDS, so a step costs no launch, no wait for the slowest
 // wave of a grid, no returning atomic in device memory and no gather: pages
 // are read and filled with contiguous accesses.  After its time a workgroup
 // hands its pages back; the next launch shares them out again.
@@ -23,186 +23,244 @@
 
 namespace gxt {
 
-constexpr int kLoopWaves = kLoopBlock / 64;
+constexpr int kLoopWaves = 8;  // per workgroup: kLoopWaves / 4 per SIMD
+constexpr int kLoopBlock = 64 * kLoopWaves;
 constexpr int kLP = 512;    // pages a workgroup holds at once, at most
 constexpr int kTake = 256;  // of which with tracks at its start, at most
-constexpr int kMinFree = 72;  // free pages per workgroup at its start, at least (one workgroup: what there is):
+constexpr int kMinFree = 96;  // free pages per workgroup at its start, at least (one workgroup: what there is):
                               // an open page for each type and what 8 running tasks may need
 
 // Shared state of a workgroup.  A page is known by its local number lp < kLP.
+// The waves work on it with LDS atomics and no lock: a lock around each of
+// the three accesses of a task cost 12,000 cycles per task, 28 % of the waves'
+// time (10 GeV e- in PbWO4, FP64).
+//  - Ready pages of a type are a ring: a writer draws a ticket from tail and
+//    fills its entry, a reader draws one from head (by compare-and-swap, below
+//    tail) and waits for the entry to be filled, which its writer does at once.
+//  - Free pages are such a ring too; `avail` counts those that no running task
+//    may still need, and a task starts only when its needs are covered, so a
+//    ticket always has, or is about to have, its entry.
+//  - A type's open page and its entries given out are one word, changed by
+//    compare-and-swap; cnt counts the tracks written into a page.
+constexpr uint16_t kNone16 = 0xffffu;
 struct Sched {
-  int lock;
-  int nfree;   // local pages on freestk
-  int need;    // pages that running tasks may still take from it
-  int active;  // running tasks
-  int stop;    // no further tasks
-  int ran;     // a task has run
-  int commits; // tasks that have ended: what a waiting wave watches
-  int head[kTypes], tail[kTypes];  // ready pages of a type: rq[type][head .. tail), positions mod kLP
-  int open[kTypes], fill[kTypes];  // the type's open page (-1: none) and its entries given out
-  uint16_t rq[kTypes][kLP];
-  uint16_t freestk[kLP];
-  uint16_t cnt[kLP];    // tracks written into a page
-  uint32_t gpage[kLP];  // local page -> page
-  int16_t dest[kLoopWaves][kTypes][4];  // pages of a wave's outputs by type, in order of entry / 64; -1: none
-  unsigned int base[4];
+  int head[16], tail[16];  // tickets of the ready rings, by type
+  int open[16];            // lp << 7 | entries given out (1 .. 63); -1: none
+  int busy;                // running tasks, + 256 x tasks ended
+  int avail;
+  int fhead, ftail;        // tickets of the free ring
+  int stop;                // no further tasks
+  int ran;                 // a task has run
+  unsigned int base[2];
+  int cnt[kLP];
+  uint32_t gpage[kLP];     // local page -> page
+  uint16_t rq[kTypes][kLP];  // lp | (tracks - 1) << 9; kNone16: not filled
+  uint16_t fr[kLP];          // lp; kNone16: not filled
+  int16_t dest[kLoopWaves][kTypes][4];  // pages of a wave's outputs by type, in order of entry / 64
   unsigned long long stat[16];
 };
+static_assert(kLP == 512, "ready entries hold 9 bits of page");
 
-// The lock is taken by lane 0 for its wave.  Its holder never waits for
-// another wave, so every wait for it ends.
-__device__ __forceinline__ void sched_lock(Sched &S) {
-  if (lane() == 0)
-    while (__hip_atomic_exchange(&S.lock, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
-      __builtin_amdgcn_s_sleep(1);
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+template <class T>
+__device__ __forceinline__ T lds_ld(const T &x) {
+  return __hip_atomic_load(&x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+template <class T>
+__device__ __forceinline__ void lds_st(T &x, T v) {
+  __hip_atomic_store(&x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ int lds_add(int &x, int v) {
+  return __hip_atomic_fetch_add(&x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ bool lds_cas(int &x, int from, int to) {
+  return __hip_atomic_compare_exchange_strong(&x, &from, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// The entry of a drawn ticket, once filled; emptied for the ring's next round.
+__device__ __forceinline__ int ring_take(uint16_t &e) {
+  uint16_t v;
+  while ((v = lds_ld(e)) == kNone16) __builtin_amdgcn_s_sleep(1);
+  lds_st(e, kNone16);
+  return v;
 }
 
-__device__ __forceinline__ void sched_unlock(Sched &S) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  if (lane() == 0) __hip_atomic_store(&S.lock, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+// Fills the entry of a drawn ticket, once the reader of the ring's last round
+// has emptied it.
+__device__ __forceinline__ void ring_put(uint16_t &e, int v) {
+  while (lds_ld(e) != kNone16) __builtin_amdgcn_s_sleep(1);
+  lds_st(e, (uint16_t)v);
 }
 
 // Pages a task of n tracks may take beside its own, which it frees first:
 // photons go on to 4 types, e-/e+ to 7 (at most one new page each); an
 // interaction gives up to 3 photons and 3 e-/e+ per track.
 __device__ __forceinline__ int task_need(int type, int n) {
-  return type == 0 ? 3 : (type == 1 ? 6 : 2 * ((63 + 3 * n) >> 6) - 1);
+  return type == 0 ? 3 : (type == 1 ? 6 : 2 * ((62 + 3 * n) >> 6) - 1);
 }
 
 struct Task {
   int type, lp, n;  // type < 0: the wave ends
+  int need;
 };
 
 // The next task of a wave: a ready page of the type that has most of them;
 // with none ready, the fullest open page that no wave is writing to; with
 // neither and no task running, or after the launch's time, none.  While other
-// waves run tasks the wave waits for what they produce.
+// waves run tasks the wave waits for one to end or begin.
 __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
   const int l = lane();
+  Task t;
+  t.type = -1;
+  t.lp = t.n = t.need = 0;
   for (;;) {
     const bool over = wall_clock64() - t_end >= 0;
-    sched_lock(S);
-    int key = -1;
+    const int busy = __builtin_amdgcn_readfirstlane(lds_ld(S.busy));
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    int key = -1, h = 0, o = -1;
     if (l < kTypes) {
-      const int r = S.tail[l] - S.head[l];
-      const int o = S.open[l], f = S.fill[l];
+      h = lds_ld(S.head[l]);
+      const int r = lds_ld(S.tail[l]) - h;
+      o = lds_ld(S.open[l]);
       if (r > 0)
         key = (1 << 16) | (r << 4) | l;
-      else if (o >= 0 && f > 0 && (int)S.cnt[o] == f)
-        key = (f << 4) | l;
+      else if (o >= 0 && lds_ld(S.cnt[o >> 7]) == (o & 127))
+        key = ((o & 127) << 4) | l;
     }
 #pragma unroll
     for (int d = 1; d < 16; d <<= 1) key = max(key, __shfl_xor(key, d, 64));
     key = __builtin_amdgcn_readfirstlane(key);
-    const int active = __builtin_amdgcn_readfirstlane(S.active);
-    const int seen = __builtin_amdgcn_readfirstlane(S.commits);
     // (a launch runs a task wherever it can, so that one that ran none is short of pages)
-    const bool late = over && __builtin_amdgcn_readfirstlane(S.ran) != 0;
-    const bool stop = late || __builtin_amdgcn_readfirstlane(S.stop) != 0;
-    Task t;
-    t.type = -1;
-    t.lp = t.n = 0;
+    if (__builtin_amdgcn_readfirstlane(lds_ld(S.stop)) != 0 ||
+        (over && __builtin_amdgcn_readfirstlane(lds_ld(S.ran)) != 0))
+      return t;
     bool wait = false;
-    if (stop || key < 0) {
-      wait = !stop && active > 0;
-      if (late && l == 0) S.stop = 1;
+    if (key < 0) {
+      if ((busy & 255) == 0 && __builtin_amdgcn_readfirstlane(lds_ld(S.busy)) == busy) return t;
+      wait = true;
     } else {
       const int type = key & 15;
-      int lp = 0, n = 0;
       const bool ready = (key >> 16) != 0;
-      if (l == type) {
-        lp = ready ? S.rq[type][S.head[type] & (kLP - 1)] : S.open[type];
-        n = S.cnt[lp];
+      const int need = task_need(type, ready ? kPageTracks : key >> 4);
+      // counted as running before it holds pages, so that a wave that finds none
+      // left sees who may give some back
+      int had = 0;
+      if (l == 0) {
+        lds_add(S.busy, 1);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        int v = lds_ld(S.avail);
+        while (v >= need && !lds_cas(S.avail, v, v - need)) v = lds_ld(S.avail);
+        had = v >= need;
       }
-      lp = __builtin_amdgcn_readlane(lp, type);
-      n = __builtin_amdgcn_readlane(n, type);
-      const int need = task_need(type, n);
-      if (__builtin_amdgcn_readfirstlane(S.nfree) - __builtin_amdgcn_readfirstlane(S.need) < need) {
-        // short of pages: a running task may free some, otherwise the
-        // workgroup hands its pages back
-        wait = active > 0;
-        if (!wait && l == 0) S.stop = 1;
-      } else {
-        t.type = type;
-        t.lp = lp;
-        t.n = n;
+      had = __builtin_amdgcn_readfirstlane(had);
+      int ok = 0;
+      if (had && l == type) ok = ready ? lds_cas(S.head[type], h, h + 1) : lds_cas(S.open[type], o, -1);
+      ok = __builtin_amdgcn_readlane(ok, type);
+      if (ok) {
+        int v = 0;
         if (l == type) {
           if (ready) {
-            S.head[type] = S.head[type] + 1;
+            v = ring_take(S.rq[type][h & (kLP - 1)]);
           } else {
-            S.open[type] = -1;
-            S.fill[type] = 0;
+            // closed: only the tracks given out before are still to come
+            while (lds_ld(S.cnt[o >> 7]) != (o & 127)) __builtin_amdgcn_s_sleep(1);
+            v = (o >> 7) | ((o & 127) - 1) << 9;
           }
+          lds_st(S.ran, 1);
         }
-        if (l == 0) {
-          S.active = active + 1;
-          S.need = S.need + need;
-          S.ran = 1;
+        v = __builtin_amdgcn_readlane(v, type);
+        t.type = type;
+        t.lp = v & (kLP - 1);
+        t.n = (v >> 9) + 1;
+        t.need = need;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        return t;
+      }
+      if (l == 0) {
+        if (had) lds_add(S.avail, need);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        lds_add(S.busy, -1);
+      }
+      if (!had) {
+        // short of pages: a running task may free some, otherwise the
+        // workgroup hands its pages back
+        wait = (busy & 255) != 0;
+        if (!wait && __builtin_amdgcn_readfirstlane(lds_ld(S.busy)) == busy) {
+          if (l == 0) lds_st(S.stop, 1);
+          return t;
         }
       }
     }
-    sched_unlock(S);
-    if (!wait) return t;
-    // until a task ends (one is running), without the lock
-    while (__hip_atomic_load(&S.commits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == seen)
-      __builtin_amdgcn_s_sleep(2);
+    if (wait)
+      while (__builtin_amdgcn_readfirstlane(lds_ld(S.busy)) == busy) __builtin_amdgcn_s_sleep(2);
   }
 }
 
 // Frees the task's page and gives out entries: lane t < kTypes asks for n
 // entries of type t and gets its first entry f; entry e of the type is slot
-// e % 64 of page S.dest[wave][t][e / 64].  With too few free pages (which
-// task_need excludes) the entries have no page (-1) and the overflow is
-// reported.
-__device__ __forceinline__ int reserve(Sched &S, Counters *cnt, const Task &task, int n) {
+// e % 64 of page S.dest[wave][t][e / 64].
+__device__ __forceinline__ int reserve(Sched &S, const Task &task, int n) {
   const int l = lane();
   const int w = (int)(threadIdx.x >> 6);
-  sched_lock(S);
-  int nfree = S.nfree;
-  if (l == 0) S.freestk[nfree] = (uint16_t)task.lp;
-  ++nfree;
-  int f = 0, o = -1, np = 0;
-  if (l < kTypes && n > 0) {
-    o = S.open[l];
-    f = S.fill[l];
-    np = ((f + n + 63) >> 6) - (o >= 0 ? 1 : 0);
-  }
-  int incl = np;
+  // the task's tracks have been read before the page may be written again
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  if (l == 0) ring_put(S.fr[lds_add(S.ftail, 1) & (kLP - 1)], task.lp);
+  int f = 0, o = -1, np = 0, hv = 0;
+  int p0 = 0, p1 = 0, p2 = 0;  // new pages in hand (at most 3: n <= 192)
+  bool todo = l < kTypes && n > 0;
+  do {
+    int ex = 0;
+    if (todo) {
+      o = lds_ld(S.open[l]);
+      f = o >= 0 ? o & 127 : 0;
+      np = ((f + n + 63) >> 6) - (o >= 0 ? 1 : 0);
+      ex = max(np - hv, 0);
+    }
+    int incl = ex;
 #pragma unroll
-  for (int d = 1; d < 16; d <<= 1) {
-    const int t = __shfl_up(incl, d, 64);
-    if (l >= d) incl += t;
-  }
-  const int total = __builtin_amdgcn_readlane(incl, kTypes - 1);
-  const bool ok = total <= nfree;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // the freed page's number before it is read below
-  if (l < kTypes && n > 0) {
-    int top = nfree - 1 - (incl - np);
-    int last = o;
-    const int have = o >= 0 ? 1 : 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      int pg = ok && j == 0 && have ? o : -1;
-      if (ok && j >= have && j - have < np) {
-        pg = S.freestk[top--];
-        S.cnt[pg] = 0;
-        last = pg;
+    for (int d = 1; d < 16; d <<= 1) {
+      const int t = __shfl_up(incl, d, 64);
+      if (l >= d) incl += t;
+    }
+    const int total = __builtin_amdgcn_readlane(incl, kTypes - 1);
+    if (total > 0) {
+      int tk = 0;
+      if (l == 0) tk = lds_add(S.fhead, total);
+      tk = __builtin_amdgcn_readfirstlane(tk) + incl - ex;
+      for (int j = 0; j < ex; ++j) {
+        const int pg = ring_take(S.fr[(tk + j) & (kLP - 1)]);
+        lds_st(S.cnt[pg], 0);
+        p0 = hv == 0 ? pg : p0;
+        p1 = hv == 1 ? pg : p1;
+        p2 = hv == 2 ? pg : p2;
+        ++hv;
       }
-      S.dest[w][l][j] = (int16_t)pg;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     }
-    if (ok) {
+    if (todo) {
       const int rem = (f + n) & 63;
-      S.open[l] = rem ? last : -1;
-      S.fill[l] = rem;
+      const int last = np == 0 ? o >> 7 : (np == 1 ? p0 : (np == 2 ? p1 : p2));
+      todo = !lds_cas(S.open[l], o, rem ? last << 7 | rem : -1);
+    }
+  } while (__any(todo));
+  if (l < kTypes && n > 0) {
+    int16_t *d = S.dest[w][l];
+    const bool have = o >= 0;
+    d[0] = (int16_t)(have ? o >> 7 : p0);
+    d[1] = (int16_t)(have ? p0 : p1);
+    d[2] = (int16_t)(have ? p1 : p2);
+    d[3] = (int16_t)p2;
+    // a page too many, when the open page changed in between
+    if (hv > np) {
+      const int pg = np == 0 ? p0 : (np == 1 ? p1 : p2);
+      ring_put(S.fr[lds_add(S.ftail, 1) & (kLP - 1)], pg);
     }
   }
-  if (l == 0) {
-    S.nfree = ok ? nfree - total : nfree;
-    S.need = S.need - task_need(task.type, task.n);
-    if (!ok) atomicOr(&cnt->overflow, 1);
-  }
-  sched_unlock(S);
+  // what the task did not take of its needs, and its own page
+  int took = np;
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) took += __shfl_xor(took, d, 64);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  if (l == 0) lds_add(S.avail, task.need + 1 - took);
   return f;
 }
 
@@ -213,28 +271,17 @@ __device__ __forceinline__ void commit(Sched &S, int f, int n) {
   const int w = (int)(threadIdx.x >> 6);
   // the tracks' stores before the other waves can see the pages
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  sched_lock(S);
   if (l < kTypes && n > 0) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    const int last = (f + n - 1) >> 6;
+    for (int j = 0; j <= last; ++j) {
       const int c = min(f + n, 64 * (j + 1)) - max(f, 64 * j);
       const int pg = S.dest[w][l][j];
-      if (c > 0 && pg >= 0) {
-        const int have = S.cnt[pg] + c;
-        S.cnt[pg] = (uint16_t)have;
-        if (have == kPageTracks) {
-          const int t = S.tail[l];
-          S.rq[l][t & (kLP - 1)] = (uint16_t)pg;
-          S.tail[l] = t + 1;
-        }
-      }
+      if (lds_add(S.cnt[pg], c) + c == kPageTracks)
+        ring_put(S.rq[l][lds_add(S.tail[l], 1) & (kLP - 1)], pg | (kPageTracks - 1) << 9);
     }
   }
-  if (l == 0) {
-    S.active = S.active - 1;
-    S.commits = S.commits + 1;
-  }
-  sched_unlock(S);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  if (l == 0) lds_add(S.busy, 256 - 1);
 }
 
 template <class R>
@@ -449,15 +496,12 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
     if (type == ty) rank = (int)__popcll(m & lt);
     if (lane() == ty) n = (int)__popcll(m);
   }
-  const int f = reserve(S, a.cnt, task, n);
+  const int f = reserve(S, task, n);
   const int e = __shfl(f, type >= 0 ? type : 0, 64) + rank;
   if (type >= 0) {
-    const int pg = S.dest[threadIdx.x >> 6][type][e >> 6];
-    if (pg >= 0) {
-      const PageSlot<R> p(page_at<R>(a, S, pg), e & 63);
-      store_track(p, t, trace);
-      if (trace && q >= 0 && q != kQueueAtRest) p.f64(kPtedep) = edep;
-    }
+    const PageSlot<R> p(page_at<R>(a, S, S.dest[threadIdx.x >> 6][type][e >> 6]), e & 63);
+    store_track(p, t, trace);
+    if (trace && q >= 0 && q != kQueueAtRest) p.f64(kPtedep) = edep;
   }
   commit(S, f, n);
   // what needs no answer
@@ -565,7 +609,7 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
   const int inclN = wave_incl_scan(outN), inclC = wave_incl_scan(outC);
   const int totN = __builtin_amdgcn_readlane(inclN, 63), totC = __builtin_amdgcn_readlane(inclC, 63);
   const int n = lane() == 0 ? totN : (lane() == 1 ? totC : 0);
-  const int f = reserve(S, a.cnt, task, n);
+  const int f = reserve(S, task, n);
   int kN = __builtin_amdgcn_readlane(f, 0) + inclN - outN;
   int kC = __builtin_amdgcn_readlane(f, 1) + inclC - outC;
   const int w = (int)(threadIdx.x >> 6);
@@ -602,8 +646,7 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
         substream_state(P, uid, rng);
         const int idx = species == 0 ? kN++ : kC++;
         const int pg = S.dest[w][species == 0 ? 0 : 1][idx >> 6];
-        if (pg >= 0)
-          store_new(PageSlot<R>(page_at<R>(a, S, pg), idx & 63), t, species, e, d0, d1, d2, uid, rng, trace);
+        store_new(PageSlot<R>(page_at<R>(a, S, pg), idx & 63), t, species, e, d0, d1, d2, uid, rng, trace);
         atomicAdd(&a.ev[t.event].nsec[species], 1ULL);
         spectrum(wh, species, (double)e);
         d0 = -d0;
@@ -615,7 +658,7 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
   if (survive) {
     const int idx = t.species == 0 ? kN : kC;
     const int pg = S.dest[w][t.species == 0 ? 0 : 1][idx >> 6];
-    if (pg >= 0) store_track(PageSlot<R>(page_at<R>(a, S, pg), idx & 63), t, trace);
+    store_track(PageSlot<R>(page_at<R>(a, S, pg), idx & 63), t, trace);
   }
   commit(S, f, n);
   if (a.prof) t_derive += wall_clock64() - t0;
@@ -639,7 +682,7 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
 // ------------------------------------------------------------------ the loop
 // kLds: the tables in LDS (LoopArgs::lds_tables).
 template <class R, int kMode, int kLds>
-__global__ __launch_bounds__(kLoopBlock, 2) void k_loop(LoopArgs a) {
+__global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a) {
   __shared__ Sched S;
   __shared__ DevParams sP;
   __shared__ Hist wh;
@@ -664,16 +707,17 @@ __global__ __launch_bounds__(kLoopBlock, 2) void k_loop(LoopArgs a) {
     int dyn = 0;
     if (kLds >= 1) dyn = stage_tables<R>(a.P, 0, dyn);
     if (kLds >= 2) (void)stage_tables<R>(a.P, 1, dyn);
-    if (tid < kTypes) {
+    if (tid < 16) {
       S.head[tid] = S.tail[tid] = 0;
       S.open[tid] = -1;
-      S.fill[tid] = 0;
+      S.stat[tid] = 0;
     }
-    if (tid < 16) S.stat[tid] = 0;
     if (tid == 0) {
-      S.lock = S.need = S.active = S.stop = S.ran = S.commits = 0;
-      S.nfree = nf;
+      S.busy = S.stop = S.ran = S.fhead = 0;
+      S.ftail = S.avail = nf;
     }
+    for (int j = tid; j < kTypes * kLP; j += kLoopBlock) S.rq[j / kLP][j % kLP] = kNone16;
+    for (int j = tid; j < kLP; j += kLoopBlock) S.fr[j] = kNone16;
     __syncthreads();
     // local pages: [0, nt) with tracks, [nt, nt + nf) free
     int start_live = 0;
@@ -682,18 +726,15 @@ __global__ __launch_bounds__(kLoopBlock, 2) void k_loop(LoopArgs a) {
         const uint32_t en = a.list[(uint32_t)(lhead + (unsigned)b + (unsigned long long)groups * j) & a.mask];
         const int type = (int)(en >> 6 & 15u), n = (int)(en & 63u) + 1;
         S.gpage[j] = en >> 10;
-        S.cnt[j] = (uint16_t)n;
+        S.cnt[j] = n;
         start_live += n;
         // the first partial page of a type is filled further, the others are
         // tasks as they are
-        if (n < kPageTracks && atomicCAS(&S.open[type], -1, j) == -1)
-          S.fill[type] = n;
-        else
-          S.rq[type][atomicAdd(&S.tail[type], 1)] = (uint16_t)j;
+        if (n == kPageTracks || !lds_cas(S.open[type], -1, j << 7 | n))
+          S.rq[type][lds_add(S.tail[type], 1)] = (uint16_t)(j | (n - 1) << 9);
       } else {
         S.gpage[j] = a.freel[(uint32_t)(fhead + (unsigned long long)b * nf + (j - nt)) & a.mask];
-        S.cnt[j] = 0;
-        S.freestk[j - nt] = (uint16_t)j;
+        S.fr[j - nt] = (uint16_t)j;
       }
     }
     __syncthreads();
@@ -732,11 +773,12 @@ __global__ __launch_bounds__(kLoopBlock, 2) void k_loop(LoopArgs a) {
     }
     __syncthreads();
     // hand back: pages with tracks (ready, then open ones) and free pages
+    const int fh = S.fhead, nfree = S.ftail - fh;
     if (tid == 0) {
       int np = 0;
-      for (int t = 0; t < kTypes; ++t) np += S.tail[t] - S.head[t] + (S.open[t] >= 0 && S.fill[t] > 0 ? 1 : 0);
+      for (int t = 0; t < kTypes; ++t) np += S.tail[t] - S.head[t] + (S.open[t] >= 0 ? 1 : 0);
       const unsigned long long lp = atomicAdd(&rg.lpush, (unsigned long long)np);
-      const unsigned long long fp = atomicAdd(&rg.fpush, (unsigned long long)S.nfree);
+      const unsigned long long fp = atomicAdd(&rg.fpush, (unsigned long long)nfree);
       S.base[0] = (uint32_t)(ltail + lp);
       S.base[1] = (uint32_t)(ftail + fp);
       if (S.ran) atomicAdd(&rg.ran, 1u);
@@ -747,21 +789,23 @@ __global__ __launch_bounds__(kLoopBlock, 2) void k_loop(LoopArgs a) {
     for (int t = 0; t < kTypes; ++t) {
       const int h = S.head[t], n = S.tail[t] - h;
       for (int j = tid; j < n; j += kLoopBlock) {
-        const int lp = S.rq[t][(h + j) & (kLP - 1)];
-        const int c = S.cnt[lp];
-        a.list[(at + (uint32_t)j) & a.mask] = page_entry(S.gpage[lp], t, c);
+        const int v = S.rq[t][(h + j) & (kLP - 1)];
+        const int c = (v >> 9) + 1;
+        a.list[(at + (uint32_t)j) & a.mask] = page_entry(S.gpage[v & (kLP - 1)], t, c);
         live += c;
       }
       at += (uint32_t)n;
-      if (S.open[t] >= 0 && S.fill[t] > 0) {
+      const int o = S.open[t];
+      if (o >= 0) {
         if (tid == 0) {
-          a.list[at & a.mask] = page_entry(S.gpage[S.open[t]], t, S.fill[t]);
-          live += S.fill[t];
+          a.list[at & a.mask] = page_entry(S.gpage[o >> 7], t, o & 127);
+          live += o & 127;
         }
         ++at;
       }
     }
-    for (int j = tid; j < S.nfree; j += kLoopBlock) a.freel[(S.base[1] + (uint32_t)j) & a.mask] = S.gpage[S.freestk[j]];
+    for (int j = tid; j < nfree; j += kLoopBlock)
+      a.freel[(S.base[1] + (uint32_t)j) & a.mask] = S.gpage[S.fr[(fh + j) & (kLP - 1)]];
     live = __builtin_amdgcn_readlane(wave_incl_scan(live), 63);
     if (lane() == 0 && live != 0) atomicAdd((unsigned long long *)&rg.live, (unsigned long long)(long long)live);
     hist_flush(a.rows, a.P, wh);
