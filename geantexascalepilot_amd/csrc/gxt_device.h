@@ -258,16 +258,6 @@ __device__ __forceinline__ uint32_t dot3_fold(uint32_t M0, uint32_t M1, uint32_t
   x = fold<c>(x);
   return (uint32_t)x + ((x >> 32) ? c : 0u);
 }
-// v = M v, congruent mod m (M row-major 3x3 of residues).
-template <uint32_t c>
-__device__ __forceinline__ void matvec_fold(const uint32_t M[9], uint32_t v[3]) {
-  const uint32_t r0 = dot3_fold<c>(M[0], M[1], M[2], v);
-  const uint32_t r1 = dot3_fold<c>(M[3], M[4], M[5], v);
-  const uint32_t r2 = dot3_fold<c>(M[6], M[7], M[8], v);
-  v[0] = r0;
-  v[1] = r1;
-  v[2] = r2;
-}
 // The residue of v <= 2^32 - 1 (m > 2^31: one subtraction).
 template <uint32_t c>
 __device__ __forceinline__ void reduce3(uint32_t v[3]) {
@@ -277,26 +267,28 @@ __device__ __forceinline__ void reduce3(uint32_t v[3]) {
 }
 constexpr uint32_t kC1 = 209u, kC2 = 22853u;  // 2^32 - m1, 2^32 - m2
 
-// One jump-table row: three 16-byte loads of a 48-byte aligned row.
-__device__ __forceinline__ void jump_row(const uint32_t *T, int c, int k, int d, uint32_t M[9]) {
-  const uint4 *row = reinterpret_cast<const uint4 *>(T + ((c * 8 + k) * 256 + d) * kJumpRow);
-  const uint4 a = row[0], b = row[1], e = row[2];
-  M[0] = a.x;
-  M[1] = a.y;
-  M[2] = a.z;
-  M[3] = a.w;
-  M[4] = b.x;
-  M[5] = b.y;
-  M[6] = b.z;
-  M[7] = b.w;
-  M[8] = e.x;
+// A state is three consecutive values x0 x1 x2 of its recurrence, and A^n maps
+// it to the values n further on.  Each of these is a combination of x0 x1 x2;
+// the coefficients of the first, c, are the first row of A^n, and the same
+// combination of x1 x2 x3 and x2 x3 x4 gives the next two: 3 words per matrix
+// in place of 9, which lets the whole table sit in LDS.  next1, next2: the
+// values after x (x3 = a12 x1 - a13n x0, x3 = a21 x2 - a23n x0), congruent and
+// <= 2^32 - 1 for such x; K = m (a + 1) or m (a + 8) keeps the difference >= 0.
+__device__ __forceinline__ uint32_t next1(uint32_t x0, uint32_t x1) {
+  constexpr uint64_t K = 4294967087ULL * 810729ULL;
+  const uint64_t t = fold<kC1>((uint64_t)x1 * 1403580u + (K - (uint64_t)x0 * 810728u));
+  return (uint32_t)t + ((t >> 32) ? kC1 : 0u);
+}
+__device__ __forceinline__ uint32_t next2(uint32_t x0, uint32_t x2) {
+  constexpr uint64_t K = 4294944443ULL * 1370597ULL;
+  const uint64_t t = fold<kC2>(fold<kC2>((uint64_t)x2 * 527612u + (K - (uint64_t)x0 * 1370589u)));
+  return (uint32_t)t + ((t >> 32) ? kC2 : 0u);
 }
 
 // Substream idx of the stream seeded with s: (A^(2^76))^idx s, as the
 // product over the 8 bytes d_k of idx of A^(d_k 2^(76+8k)) (powers of one
-// matrix commute).  T[((c * 8 + k) * 256 + d) * kJumpRow + i], i < 9, holds
-// A_c^(d 2^(76+8k)) mod m_c, the identity for d = 0.  The rows' loads depend
-// only on idx: two bytes' rows are in flight at a time.
+// matrix commute).  T: DevParams::jump8 or its LDS copy; a row is the identity
+// for d = 0.  The rows depend only on idx: two are in flight at a time.
 __device__ __forceinline__ void jump_substream(const uint32_t *T, const uint32_t s[6], uint64_t idx,
                                                uint32_t v1[3], uint32_t v2[3]) {
   v1[0] = s[0];
@@ -308,19 +300,25 @@ __device__ __forceinline__ void jump_substream(const uint32_t *T, const uint32_t
 #pragma unroll 2
   for (int k = 0; k < 8; ++k) {
     const int d = (int)((idx >> (8 * k)) & 255u);
-    uint32_t M1[9], M2[9];
-    jump_row(T, 0, k, d, M1);
-    jump_row(T, 1, k, d, M2);
-    matvec_fold<kC1>(M1, v1);
-    matvec_fold<kC2>(M2, v2);
+    const uint2 *row = reinterpret_cast<const uint2 *>(T + (k * 256 + d) * kJumpRow);
+    const uint2 a = row[0], b = row[1], e = row[2];
+    const uint32_t x1 = next1(v1[0], v1[1]), y1 = next1(v1[1], v1[2]);
+    const uint32_t x2 = next2(v2[0], v2[2]), y2 = next2(v2[1], x2);
+    const uint32_t w1[5] = {v1[0], v1[1], v1[2], x1, y1}, w2[5] = {v2[0], v2[1], v2[2], x2, y2};
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      v1[j] = dot3_fold<kC1>(a.x, a.y, b.x, w1 + j);
+      v2[j] = dot3_fold<kC2>(b.y, e.x, e.y, w2 + j);
+    }
   }
   reduce3<kC1>(v1);
   reduce3<kC2>(v2);
 }
 
-__device__ __forceinline__ void substream_state(const DevParams *P, uint64_t idx, uint32_t out[6]) {
+__device__ __forceinline__ void substream_state(const uint32_t *T, const uint32_t seed[6], uint64_t idx,
+                                                uint32_t out[6]) {
   uint32_t v1[3], v2[3];
-  jump_substream(P->jump8, P->seed, idx, v1, v2);
+  jump_substream(T, seed, idx, v1, v2);
   out[0] = v1[0];
   out[1] = v1[1];
   out[2] = v1[2];

@@ -1001,8 +1001,11 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
     const int nb = c->precision == GXT_FP32 ? (int)sizeof(Node32) : (int)sizeof(Node64);
     const int room = kLoopLds - kLoopLdsFixed;
     const int b0 = P.lds_nodes[0] * nb, b1 = P.lds_nodes[1] * nb;
-    c->lds_tables = b0 + b1 <= room ? 2 : (b0 <= room ? 1 : 0);
-    c->lds_bytes = c->lds_tables == 2 ? b0 + b1 : (c->lds_tables == 1 ? b0 : 0);
+    const int bj = kJumpWords * (int)sizeof(uint32_t);
+    // (two slots in FP32: all tables without the jump table would fit as well,
+    // and measured the same)
+    c->lds_tables = b0 + b1 + bj <= room ? kLdsAll : (b0 + bj <= room ? kLdsPhotons : kLdsNone);
+    c->lds_bytes = c->lds_tables == kLdsAll ? b0 + b1 + bj : (c->lds_tables == kLdsPhotons ? b0 + bj : 0);
   }
   // pages, counters, tallies: pages for the capacity, and for each workgroup
   // but one what it holds open or partly filled

@@ -17,7 +17,7 @@ __device__ __forceinline__ void inject_state(const DevParams *P, const LoopArgs 
   t.nil0 = t.nil1 = t.nil2 = R(-1);
   t.nsteps = 0;
   t.vol = geo_locate(P->geo, t.pos, p.dir);
-  if (t.vol >= 0) substream_state(P, t.uid, t.rng.s);
+  if (t.vol >= 0) substream_state(P->jump8, P->seed, t.uid, t.rng.s);
 }
 
 // A track in flight continues from its own interaction lengths, RNG state,

@@ -546,8 +546,8 @@ __device__ __forceinline__ int sec_fate(const DevParams *P, TrackRegs<R> &t, Dep
 // One page of queue q: sample the final states, write the survivors and the
 // tracks created, each with its RNG state.
 template <class R>
-__device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams *P, Sched &S, Hist &wh,
-                                              const Task &task, long long &t_derive) {
+__device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams *P, const uint32_t *jump, Sched &S,
+                                              Hist &wh, const Task &task, long long &t_derive) {
   const bool trace = P->trace_events > 0;
   const R mine = (R)P->tracking_cut;
   const int q = task.type - 2;
@@ -643,7 +643,7 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
       if (go) {
         const uint64_t uid = child_substream(t.rng);
         uint32_t rng[6];
-        substream_state(P, uid, rng);
+        substream_state(jump, P->seed, uid, rng);
         const int idx = species == 0 ? kN++ : kC++;
         const int pg = S.dest[w][species == 0 ? 0 : 1][idx >> 6];
         store_new(PageSlot<R>(page_at<R>(a, S, pg), idx & 63), t, species, e, d0, d1, d2, uid, rng, trace);
@@ -705,8 +705,11 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     hist_clear(wh);
     stage_params(a.P, sP);
     int dyn = 0;
-    if (kLds >= 1) dyn = stage_tables<R>(a.P, 0, dyn);
-    if (kLds >= 2) (void)stage_tables<R>(a.P, 1, dyn);
+    if (kLds != kLdsNone) dyn = stage_tables<R>(a.P, 0, dyn);
+    if (kLds == kLdsAll) dyn = stage_tables<R>(a.P, 1, dyn);
+    const int at_jump = dyn;
+    if (kLds != kLdsNone)
+      copy_words16(tab_lds + at_jump, reinterpret_cast<const uint4 *>(a.P->jump8), kJumpWords / 4);
     if (tid < 16) {
       S.head[tid] = S.tail[tid] = 0;
       S.open[tid] = -1;
@@ -741,17 +744,23 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     {
       const DevParams *P = &sP;
       using T = typename NodeType<R>::T;
-      const NodesT<R, (kLds >= 1)> N0 = [&] {
-        if constexpr (kLds >= 1)
+      const NodesT<R, (kLds != kLdsNone)> N0 = [&] {
+        if constexpr (kLds != kLdsNone)
           return NodesT<R, true>(reinterpret_cast<const T *>(tab_lds), P->hints);
         else
           return NodesT<R, false>(P);
       }();
-      const NodesT<R, (kLds >= 2)> N1 = [&] {
-        if constexpr (kLds >= 2)
+      const NodesT<R, (kLds == kLdsAll)> N1 = [&] {
+        if constexpr (kLds == kLdsAll)
           return NodesT<R, true>(reinterpret_cast<const T *>(tab_lds) + P->lds_nodes[0], P->hints);
         else
           return NodesT<R, false>(P);
+      }();
+      const uint32_t *jump = [&] {
+        if constexpr (kLds != kLdsNone)
+          return reinterpret_cast<const uint32_t *>(tab_lds + at_jump);
+        else
+          return P->jump8;
       }();
       for (;;) {
         const Task task = next_task(S, t_end);
@@ -763,7 +772,7 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
         else if (task.type == 1)
           transport_task<R, true, kMode>(a, P, N1, S, wh, task);
         else
-          interact_task<R>(a, P, S, wh, task, td);
+          interact_task<R>(a, P, jump, S, wh, task, td);
         if (a.prof && lane() == 0) {
           const int part = task.type < 2 ? kStatTimeN + task.type : (task.type < 5 ? kStatTimeIN : kStatTimeIC);
           atomicAdd(&S.stat[part], (unsigned long long)(wall_clock64() - t0 - td));
@@ -841,9 +850,11 @@ static hipError_t launch_one(const LoopArgs &a, hipStream_t st, hipEvent_t e0, h
 
 template <class R, int kMode>
 hipError_t launch_loop_mode(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  if (a.lds_tables == 2) return launch_one<R, kMode, 2>(a, st, e0, e1);
-  if (a.lds_tables == 1) return launch_one<R, kMode, 1>(a, st, e0, e1);
-  return launch_one<R, kMode, 0>(a, st, e0, e1);
+  switch (a.lds_tables) {
+    case kLdsAll: return launch_one<R, kMode, kLdsAll>(a, st, e0, e1);
+    case kLdsPhotons: return launch_one<R, kMode, kLdsPhotons>(a, st, e0, e1);
+    default: return launch_one<R, kMode, kLdsNone>(a, st, e0, e1);
+  }
 }
 
 }  // namespace gxt

@@ -21,8 +21,10 @@ constexpr int kMaxShells = 128;   // shell binding energies over the elements of
 // Statistics counters are spread over kStripes rows (workgroup b adds to row
 // b % kStripes).
 constexpr int kStripes = 16;
-// Words per row of the substream jump tables: a 3x3 matrix padded to 48 bytes.
-constexpr int kJumpRow = 12;
+// Words per row of the substream jump table: the first rows of both components'
+// matrices; 8 bytes of the index x 256 values x 24 bytes = 48 KB.
+constexpr int kJumpRow = 6;
+constexpr int kJumpWords = 8 * 256 * kJumpRow;
 
 // One node of a physics vector: abscissa (energy or range), value, second
 // derivative; a spline lookup reads two adjacent nodes, 64 B (32 B in FP32).
@@ -32,6 +34,10 @@ struct alignas(32) Node64 {
 struct alignas(16) Node32 {
   float x, y, d2, pad;
 };
+
+// What a step-loop launch stages in LDS: nothing; the photon tables and the
+// jump table; those and the e-/e+ tables.
+enum { kLdsNone = 0, kLdsPhotons, kLdsAll };
 
 // One physics vector inside the node array (nodes [off, off+n)).
 struct DevTable {
@@ -179,7 +185,7 @@ struct DevParams {
   int msc;            // e-/e+ multiple scattering
   uint32_t seed[6];
   int nsandia, nshells;     // doubles in the Sandia and shell arrays
-  const uint32_t *jump8;    // A_c^(d 2^(76+8k)) mod m_c at ((c * 8 + k) * 256 + d) * kJumpRow
+  const uint32_t *jump8;    // first row of A_c^(d 2^(76+8k)) mod m_c at (k * 256 + d) * kJumpRow + 3 c
   const Node64 *nd;             // physics-vector nodes, FP64
   const Node32 *nf;             // FP32 mirror
   const double *sbd;            // Seltzer-Berger grids, FP64
