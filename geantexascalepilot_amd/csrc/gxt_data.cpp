@@ -290,6 +290,14 @@ int load_material(const std::string &data, int which, double lar_density, HostDa
     e.sandia = (int)hd.sandia.size();
     e.nint = (int)rows.size() / 5;
     hd.sandia.insert(hd.sandia.end(), rows.begin(), rows.end());
+    // a sampler takes the first shell bound at most as strongly as the photon's
+    // energy; one not below all the shells before it is never the first
+    {
+      size_t k = 0;
+      for (double b : shells)
+        if (k == 0 || b < shells[k - 1]) shells[k++] = b;
+      shells.resize(k);
+    }
     e.shell = (int)hd.shells.size();
     e.nshell = (int)shells.size();
     hd.shells.insert(hd.shells.end(), shells.begin(), shells.end());

@@ -335,6 +335,23 @@ __device__ __forceinline__ uint64_t child_substream(Rng &r) {
 }
 
 // ------------------------------------------------------------------ tables
+// A load through a pointer that is known to point to device memory.  The
+// pointers in DevParams are read from its LDS copy, where the compiler
+// cannot tell what they point to, and would load flat: slower, and waited for
+// together with all LDS accesses.
+template <class T>
+__device__ __forceinline__ T gld(const T *p) {
+  return *(const __attribute__((address_space(1))) T *)p;
+}
+__device__ __forceinline__ Node64 gld(const Node64 *p) {
+  const double *q = &p->x;
+  return Node64{gld(q), gld(q + 1), gld(q + 2), gld(q + 3)};
+}
+__device__ __forceinline__ Node32 gld(const Node32 *p) {
+  const float *q = &p->x;
+  return Node32{gld(q), gld(q + 1), gld(q + 2), gld(q + 3)};
+}
+
 template <class R> struct NodeType;
 template <> struct NodeType<double> {
   using T = Node64;
@@ -344,16 +361,25 @@ template <> struct NodeType<float> {
   using T = Node32;
   __device__ static const Node32 *global(const DevParams *P) { return P->nf; }
 };
-// Where a kernel reads physics-vector nodes: the node array in device memory
-// (DevTable::off), or with kLds its LDS copy (DevTable::loff).
-template <class R, bool kLds = false>
+// Where a kernel reads the physics vectors' nodes, the search hints and the
+// merged Sandia rows: in device memory (DevTable::off), or from LDS copies
+// (kLds: nodes, at DevTable::loff; kSmall: hints and Sandia rows).
+template <class R, bool kLds = false, bool kSmall = false>
 struct NodesT {
   using T = typename NodeType<R>::T;
   const T *v;
   const int *hints;
-  __device__ NodesT(const DevParams *P) : v(NodeType<R>::global(P)), hints(P->hints) {}
-  __device__ NodesT(const T *lds, const int *h) : v(lds), hints(h) {}
-  __device__ __forceinline__ const T &at(const DevTable &t, int i) const { return v[(kLds ? t.loff : t.off) + i]; }
+  const double *sx;
+  __device__ NodesT(const DevParams *P) : v(NodeType<R>::global(P)), hints(P->hints), sx(P->sx) {}
+  __device__ NodesT(const T *nodes, const int *h, const double *s) : v(nodes), hints(h), sx(s) {}
+  __device__ __forceinline__ T at(const DevTable &t, int i) const {
+    if constexpr (kLds)
+      return v[t.loff + i];
+    else
+      return gld(v + t.off + i);
+  }
+  __device__ __forceinline__ int hint(int i) const { return kSmall ? hints[i] : gld(hints + i); }
+  __device__ __forceinline__ double sand(int i) const { return kSmall ? sx[i] : gld(sx + i); }
 };
 template <class R> using Nodes = NodesT<R, false>;
 
@@ -436,7 +462,7 @@ __device__ __forceinline__ R pvec_inv_value(const NS &N, const DevTable &t, R r)
   // next node is below r: about one dependent load instead of log2(n).
   int k = (int)floorf((__log2f((float)r) - t.hlog0) * t.hscale) - 1;
   k = k < 0 ? 0 : (k >= t.nhint ? t.nhint - 1 : k);
-  int j = N.hints[t.hint + k];
+  int j = N.hint(t.hint + k);
   while (j > 0 && !(N.at(t, j).x < r)) --j;
   while (j < n - 2 && N.at(t, j + 1).x < r) ++j;
   return spline<R>(N.at(t, j), N.at(t, j + 1), r);
@@ -503,8 +529,8 @@ __device__ __forceinline__ R sb_at(const DevParams *P, const SbRow<R> &r, R x) {
   else if (x > gx[31]) x = gx[31];
   const int ix = sb_bin(gx, 32, x);
   const R x1 = gx[ix], x2 = gx[ix + 1], y = r.y, y1 = r.y1, y2 = r.y2;
-  const R v11 = r.v1[ix], v12 = r.v1[ix + 1];
-  const R v21 = r.v2[ix], v22 = r.v2[ix + 1];
+  const R v11 = gld(r.v1 + ix), v12 = gld(r.v1 + ix + 1);
+  const R v21 = gld(r.v2 + ix), v22 = gld(r.v2 + ix + 1);
   return ((y2 - y) * (v11 * (x2 - x) + v12 * (x - x1)) + ((y - y1) * (v21 * (x2 - x) + v22 * (x - x1)))) /
          ((x2 - x1) * (y2 - y1));
 }
@@ -519,35 +545,38 @@ __device__ __forceinline__ R sb_value(const DevParams *P, const R *g, R x, R y) 
 // the hint of the log2 bin one below ek's (the FP32 log2 is off by far less
 // than a bin) and steps to the interval: one or two dependent loads, where a
 // walk over each element's rows took up to its number of intervals.
-__device__ __forceinline__ int sandia_interval(const DevParams *P, const DevMaterial &m, double ek) {
-  const double *B = P->sx + m.sx_b;
-  const int nb = m.sx_n;
+template <class NS>
+__device__ __forceinline__ int sandia_interval(const NS &N, const DevMaterial &m, double ek) {
+  const int B = m.sx_b, nb = m.sx_n;
   int k = (int)floorf((__log2f((float)ek) - m.sx_hlog0) * m.sx_hscale) - 1;
   k = k < 0 ? 0 : (k >= m.sx_nhint ? m.sx_nhint - 1 : k);
-  int j = P->hints[m.sx_hint + k];
-  while (j > 0 && B[j - 1] > ek) --j;
-  while (j < nb && B[j] <= ek) ++j;
+  int j = N.hint(m.sx_hint + k);
+  while (j > 0 && N.sand(B + j - 1) > ek) --j;
+  while (j < nb && N.sand(B + j) <= ek) ++j;
   return j;
 }
 
-// Sandia photo-absorption per atom (mm2) of an element with coefficients c
-// (a1..a4 of its row at ek, in keV).
-__device__ __forceinline__ double sandia_atom(const DevElement &el, const double *c, double ek) {
+// Sandia photo-absorption per atom (mm2) of an element with coefficients
+// a1..a4 at c (its row at ek, in keV).
+template <class NS>
+__device__ __forceinline__ double sandia_atom(const NS &N, const DevElement &el, int c, double ek) {
   const double inv = 1.0 / ek;
-  const double s = inv * (c[0] + inv * (c[1] + inv * (c[2] + inv * c[3])));
+  const double s = inv * (N.sand(c) + inv * (N.sand(c + 1) + inv * (N.sand(c + 2) + inv * N.sand(c + 3))));
   return (el.Z / el.zoa) / kAvogadro * s * 100.0;
 }
 
 // Coefficients of the elements of m at ek: element i's at the result + 4 i.
-__device__ __forceinline__ const double *sandia_coefs(const DevParams *P, const DevMaterial &m, double ek) {
-  return P->sx + m.sx_c + sandia_interval(P, m, ek) * m.nel * 4;
+template <class NS>
+__device__ __forceinline__ int sandia_coefs(const NS &N, const DevMaterial &m, double ek) {
+  return m.sx_c + sandia_interval(N, m, ek) * m.nel * 4;
 }
 
-__device__ __forceinline__ double sandia_macro(const DevParams *P, const DevMaterial &m, double ekin) {
+template <class NS>
+__device__ __forceinline__ double sandia_macro(const NS &N, const DevMaterial &m, double ekin) {
   const double ek = ekin * 1.0e3;
-  const double *c = sandia_coefs(P, m, ek);
+  const int c = sandia_coefs(N, m, ek);
   double s = 0;
-  for (int i = 0; i < m.nel; ++i) s += m.el[i].natoms * sandia_atom(m.el[i], c + 4 * i, ek);
+  for (int i = 0; i < m.nel; ++i) s += m.el[i].natoms * sandia_atom(N, m.el[i], c + 4 * i, ek);
   return s;
 }
 
@@ -576,7 +605,7 @@ __device__ __forceinline__ R macro_xs(const DevParams *P, const NS &N, const Dev
     }
     if (p == 1) return pvec_value(N, m.tab[GXT_TAB_LAMBDA_CONV], e, le);
     if ((double)e >= m.phot_emin) return pvec_value(N, m.tab[GXT_TAB_LAMBDAPRIM_PHOT], e, le) / e;
-    return (R)sandia_macro(P, m, (double)e);
+    return (R)sandia_macro(N, m, (double)e);
   }
   const bool pos = species == 2;
   if (p == 0) return pvec_value(N, m.tab[pos ? GXT_TAB_LAMBDA_BREM_EP : GXT_TAB_LAMBDA_BREM_EM], e, le);
@@ -647,14 +676,14 @@ __device__ __forceinline__ void ia_init(Interaction<R> &o, R e, const R d[3], R 
 }
 
 // Element choice for compounds (the reference hard-codes Z): kind 0 = n Z(Z+1), kind 1 = partial Sandia.
-template <class R>
-__device__ __forceinline__ int select_element(const DevParams *P, const DevMaterial &m, int kind, R e, Rng &rng) {
+template <class R, class NS>
+__device__ __forceinline__ int select_element(const NS &N, const DevMaterial &m, int kind, R e, Rng &rng) {
   if (m.nel == 1) return 0;
   double w[kMaxElem], tot = 0;
   const double ek = (double)e * 1.0e3;
-  const double *c = kind == 0 ? nullptr : sandia_coefs(P, m, ek);
+  const int c = kind == 0 ? 0 : sandia_coefs(N, m, ek);
   for (int i = 0; i < m.nel; ++i) {
-    w[i] = kind == 0 ? m.el[i].wbrem : m.el[i].natoms * sandia_atom(m.el[i], c + 4 * i, ek);
+    w[i] = kind == 0 ? m.el[i].wbrem : m.el[i].natoms * sandia_atom(N, m.el[i], c + 4 * i, ek);
     tot += w[i];
   }
   const double r = rng.uniform() * tot;
@@ -739,13 +768,13 @@ template <class R> __device__ __forceinline__ R coulomb_factor(R Z) {
 
 // Bethe-Heitler (proxy/ProxyBetheHeitler.hpp:64-182): element from the material, Tsai
 // angle used as an angle.
-template <class R>
-__device__ __forceinline__ void sample_pair(const DevParams *P, const DevMaterial &m, R e0, const R d0[3], Rng &rng,
+template <class R, class NS>
+__device__ __forceinline__ void sample_pair(const DevParams *P, const NS &N, const DevMaterial &m, R e0, const R d0[3], Rng &rng,
                                    Interaction<R> &o) {
   ia_init(o, e0, d0, e0);
   const R eps0 = R(kMe) / e0;
   if (eps0 > R(0.5)) return;
-  const int ie = select_element(P, m, 0, e0, rng);
+  const int ie = select_element(N, m, 0, e0, rng);
   const R Z = (R)m.el[ie].Z;
   R eps;
   if (e0 < R(2.0)) {
@@ -809,20 +838,24 @@ __device__ __forceinline__ void sample_pair(const DevParams *P, const DevMateria
 
 // Sauter-Gavrila (proxy/ProxySauterGavrila.hpp:66-130): element by partial Sandia
 // cross-section, first shell bound below E, binding energy deposited.
-template <class R>
-__device__ __forceinline__ void sample_photo(const DevParams *P, const DevMaterial &m, R e0, const R d0[3], Rng &rng,
+template <class R, class NS>
+__device__ __forceinline__ void sample_photo(const DevParams *P, const NS &N, const DevMaterial &m, R e0, const R d0[3], Rng &rng,
                                     Interaction<R> &o) {
   ia_init(o, e0, d0, R(0));
-  const int ie = select_element(P, m, 1, e0, rng);
+  const int ie = select_element(N, m, 1, e0, rng);
   const DevElement &el = m.el[ie];
-  R bind = R(0);
-  for (int i = 0; i < el.nshell; ++i) {
-    const R b = (R)P->shell_e[el.shell + i];
-    if (e0 >= b) {
-      bind = b;
-      break;
-    }
+  // the energies fall, so the first shell bound below e0 by bisection (a walk
+  // from the K shell was up to 23 dependent reads for a photon below all but
+  // the outer shells)
+  int s0 = 0, s1 = el.nshell;
+  while (s0 < s1) {
+    const int mid = (s0 + s1) >> 1;
+    if (e0 >= (R)P->shell_e[el.shell + mid])
+      s1 = mid;
+    else
+      s0 = mid + 1;
   }
+  const R bind = s0 < el.nshell ? (R)P->shell_e[el.shell + s0] : R(0);
   const R te = e0 - bind;
   const R tau = e0 / R(kMe);
   R cost;
@@ -858,14 +891,14 @@ __device__ __forceinline__ void sample_photo(const DevParams *P, const DevMateri
 
 // Seltzer-Berger (proxy/ProxySeltzerBerger.hpp:204-315): element from the material, its
 // own grid, Migdal factor, gamma cut of the couple, electron kinetic energy.
-template <class R>
-__device__ __forceinline__ void sample_brems(const DevParams *P, const DevMaterial &m, R t0, const R d0[3], Rng &rng,
+template <class R, class NS>
+__device__ __forceinline__ void sample_brems(const DevParams *P, const NS &N, const DevMaterial &m, R t0, const R d0[3], Rng &rng,
                                     Interaction<R> &o) {
   ia_init(o, t0, d0, t0);
   const R cut = rmin((R)m.cut_gamma, t0);
   const R emax = t0;
   if (cut >= emax) return;
-  const int ie = select_element(P, m, 0, t0, rng);
+  const int ie = select_element(N, m, 0, t0, rng);
   const R *sb = sb_base<R>(P, m.el[ie].sb);
   const R etot = t0 + R(kMe);
   const R dcorr = (R)m.migdal * etot * etot;
@@ -1042,15 +1075,15 @@ __device__ __forceinline__ void sample_annihil(R t0, const R d0[3], Rng &rng, In
   o.nsec = 2;
 }
 
-template <class R>
-__device__ __forceinline__ void sample_model(const DevParams *P, const DevMaterial &m, int model, R e, const R d[3], Rng &rng,
+template <class R, class NS>
+__device__ __forceinline__ void sample_model(const DevParams *P, const NS &N, const DevMaterial &m, int model, R e, const R d[3], Rng &rng,
                                     Interaction<R> &o) {
   switch (model) {
     case GXT_MODEL_KLEIN_NISHINA: sample_compton(e, d, rng, o); break;
-    case GXT_MODEL_BETHE_HEITLER: sample_pair(P, m, e, d, rng, o); break;
-    case GXT_MODEL_SAUTER_GAVRILA: sample_photo(P, m, e, d, rng, o); break;
+    case GXT_MODEL_BETHE_HEITLER: sample_pair(P, N, m, e, d, rng, o); break;
+    case GXT_MODEL_SAUTER_GAVRILA: sample_photo(P, N, m, e, d, rng, o); break;
     case GXT_MODEL_SELTZER_BERGER_EM:
-    case GXT_MODEL_SELTZER_BERGER_EP: sample_brems(P, m, e, d, rng, o); break;
+    case GXT_MODEL_SELTZER_BERGER_EP: sample_brems(P, N, m, e, d, rng, o); break;
     case GXT_MODEL_MOLLER: sample_ioni(m, false, e, d, rng, o); break;
     case GXT_MODEL_BHABHA: sample_ioni(m, true, e, d, rng, o); break;
     default: sample_annihil(e, d, rng, o); break;
@@ -1058,23 +1091,23 @@ __device__ __forceinline__ void sample_model(const DevParams *P, const DevMateri
 }
 
 // Samplers of the photon queues (0 Compton, 1 conversion, 2 photoelectric).
-template <class R>
-__device__ __forceinline__ void sample_neutral(const DevParams *P, const DevMaterial &m, int q, R e, const R d[3],
+template <class R, class NS>
+__device__ __forceinline__ void sample_neutral(const DevParams *P, const NS &N, const DevMaterial &m, int q, R e, const R d[3],
                                                Rng &rng, Interaction<R> &o) {
   if (q == 0)
     sample_compton(e, d, rng, o);
   else if (q == 1)
-    sample_pair(P, m, e, d, rng, o);
+    sample_pair(P, N, m, e, d, rng, o);
   else
-    sample_photo(P, m, e, d, rng, o);
+    sample_photo(P, N, m, e, d, rng, o);
 }
 
 // Samplers of the e-/e+ queues (3, 5 bremsstrahlung, 4 Moller, 6 Bhabha, 7 annihilation).
-template <class R>
-__device__ __forceinline__ void sample_charged(const DevParams *P, const DevMaterial &m, int q, R e, const R d[3],
+template <class R, class NS>
+__device__ __forceinline__ void sample_charged(const DevParams *P, const NS &N, const DevMaterial &m, int q, R e, const R d[3],
                                                Rng &rng, Interaction<R> &o) {
   if (q == 3 || q == 5)
-    sample_brems(P, m, e, d, rng, o);
+    sample_brems(P, N, m, e, d, rng, o);
   else if (q == 4)
     sample_ioni(m, false, e, d, rng, o);
   else if (q == 6)
@@ -1670,7 +1703,8 @@ __device__ __forceinline__ void map_field(const DevField &f, double x, double y,
   const double *q = p + (int64_t)f.nz * 3;
   double b[3];
 #pragma unroll
-  for (int c = 0; c < 3; ++c) b[c] = w00 * p[c] + w01 * p[3 + c] + w10 * q[c] + w11 * q[3 + c];
+  for (int c = 0; c < 3; ++c)
+    b[c] = w00 * gld(p + c) + w01 * gld(p + 3 + c) + w10 * gld(q + c) + w11 * gld(q + 3 + c);
   double cs = 1.0, sn = 0.0;
   if (r > 0.0) {
     cs = x / r;

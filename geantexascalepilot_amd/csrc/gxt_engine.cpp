@@ -154,6 +154,9 @@ int upload(HostData &hd, DeviceData &dd) {
     if (e != hipSuccess) return e;
     return hipMemcpy(*dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice);
   };
+  // (padded to whole 16-byte words, as the step loop copies them into LDS)
+  while (hd.sx.size() % 2) hd.sx.push_back(0.0);
+  while (hd.hints.size() % 4) hd.hints.push_back(0);
   std::vector<Node64> n64(hd.x.size());
   std::vector<Node32> n32(hd.x.size());
   for (size_t i = 0; i < hd.x.size(); ++i) {
@@ -175,6 +178,8 @@ int upload(HostData &hd, DeviceData &dd) {
   build_jump_tables(jump, j8);
   HIP_TRY(put(&dd.jump8, j8));
   p.nsandia = (int)hd.sandia.size();
+  p.nsx = (int)hd.sx.size();
+  p.nhints = (int)hd.hints.size();
   p.nshells = (int)hd.shells.size();
   if (hd.shells.size() > (size_t)kMaxShells) return set_err(GXT_EDATA, "more shell energies than DevParams holds");
   for (size_t i = 0; i < hd.shells.size(); ++i) p.shell_e[i] = hd.shells[i];
@@ -1001,7 +1006,7 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
     const int nb = c->precision == GXT_FP32 ? (int)sizeof(Node32) : (int)sizeof(Node64);
     const int room = kLoopLds - kLoopLdsFixed;
     const int b0 = P.lds_nodes[0] * nb, b1 = P.lds_nodes[1] * nb;
-    const int bj = kJumpWords * (int)sizeof(uint32_t);
+    const int bj = kJumpWords * (int)sizeof(uint32_t) + P.nsx * (int)sizeof(double) + P.nhints * (int)sizeof(int);
     // (two slots in FP32: all tables without the jump table would fit as well,
     // and measured the same)
     c->lds_tables = b0 + b1 + bj <= room ? kLdsAll : (b0 + bj <= room ? kLdsPhotons : kLdsNone);

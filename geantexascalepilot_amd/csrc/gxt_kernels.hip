@@ -189,7 +189,7 @@ __global__ void k_sample(const DevParams *P, int slot, int model, SampleArgs s) 
   for (int j = 0; j < 6; ++j) r.s[j] = s.rng[6 * i + j];
   const R d[3] = {(R)s.dir[i], (R)s.dir[n + i], (R)s.dir[2 * n + i]};
   Interaction<R> o;
-  sample_model<R>(P, P->mat[slot], model, (R)s.ekin[i], d, r, o);
+  sample_model<R>(P, Nodes<R>(P), P->mat[slot], model, (R)s.ekin[i], d, r, o);
   for (int j = 0; j < 6; ++j) s.rng[6 * i + j] = r.s[j];
   s.out_ekin[i] = (double)o.ekin;
   s.out_dir[i] = (double)o.d[0];

@@ -545,9 +545,9 @@ __device__ __forceinline__ int sec_fate(const DevParams *P, TrackRegs<R> &t, Dep
 
 // One page of queue q: sample the final states, write the survivors and the
 // tracks created, each with its RNG state.
-template <class R>
-__device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams *P, const uint32_t *jump, Sched &S,
-                                              Hist &wh, const Task &task, long long &t_derive) {
+template <class R, class NS>
+__device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams *P, const NS &N,
+                                              const uint32_t *jump, Sched &S, Hist &wh, const Task &task, long long &t_derive) {
   const bool trace = P->trace_events > 0;
   const R mine = (R)P->tracking_cut;
   const int q = task.type - 2;
@@ -572,9 +572,9 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
       // an interacting track is in a material (the tree form's vacuum has no physics)
       const DevMaterial &m = P->mat[max(P->geo.slot[geo_cell<2>(P->geo, t.vol)], 0)];
       if (q < 3)
-        sample_neutral<R>(P, m, q, t.e, t.dir, t.rng, o);
+        sample_neutral<R>(P, N, m, q, t.e, t.dir, t.rng, o);
       else
-        sample_charged<R>(P, m, q, t.e, t.dir, t.rng, o);
+        sample_charged<R>(P, N, m, q, t.e, t.dir, t.rng, o);
       pair = q == 1 && o.nsec == 2;
       if (q == 7) ++nannih;
       dp.add(P, t, (double)o.edep, t.pos, t.vol);
@@ -704,12 +704,17 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     const long long t_end = wall_clock64() + a.ticks;
     hist_clear(wh);
     stage_params(a.P, sP);
-    int dyn = 0;
-    if (kLds != kLdsNone) dyn = stage_tables<R>(a.P, 0, dyn);
-    if (kLds == kLdsAll) dyn = stage_tables<R>(a.P, 1, dyn);
-    const int at_jump = dyn;
-    if (kLds != kLdsNone)
+    // (in 16-byte words) photon tables, e-/e+ tables, jump table, Sandia rows, hints
+    int at_jump = 0, at_sx = 0, at_hints = 0;
+    if (kLds != kLdsNone) {
+      at_jump = stage_tables<R>(a.P, 0, 0);
+      if (kLds == kLdsAll) at_jump = stage_tables<R>(a.P, 1, at_jump);
+      at_sx = at_jump + kJumpWords / 4;
+      at_hints = at_sx + a.P->nsx / 2;
       copy_words16(tab_lds + at_jump, reinterpret_cast<const uint4 *>(a.P->jump8), kJumpWords / 4);
+      copy_words16(tab_lds + at_sx, reinterpret_cast<const uint4 *>(a.P->sx), a.P->nsx / 2);
+      copy_words16(tab_lds + at_hints, reinterpret_cast<const uint4 *>(a.P->hints), a.P->nhints / 4);
+    }
     if (tid < 16) {
       S.head[tid] = S.tail[tid] = 0;
       S.open[tid] = -1;
@@ -744,17 +749,22 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     {
       const DevParams *P = &sP;
       using T = typename NodeType<R>::T;
-      const NodesT<R, (kLds != kLdsNone)> N0 = [&] {
-        if constexpr (kLds != kLdsNone)
-          return NodesT<R, true>(reinterpret_cast<const T *>(tab_lds), P->hints);
+      constexpr bool kSmall = kLds != kLdsNone;
+      const int *hints = reinterpret_cast<const int *>(tab_lds + at_hints);
+      const double *sx = reinterpret_cast<const double *>(tab_lds + at_sx);
+      const NodesT<R, kSmall, kSmall> N0 = [&] {
+        if constexpr (kSmall)
+          return NodesT<R, true, true>(reinterpret_cast<const T *>(tab_lds), hints, sx);
         else
-          return NodesT<R, false>(P);
+          return NodesT<R>(P);
       }();
-      const NodesT<R, (kLds == kLdsAll)> N1 = [&] {
+      const NodesT<R, (kLds == kLdsAll), kSmall> N1 = [&] {
         if constexpr (kLds == kLdsAll)
-          return NodesT<R, true>(reinterpret_cast<const T *>(tab_lds) + P->lds_nodes[0], P->hints);
+          return NodesT<R, true, true>(reinterpret_cast<const T *>(tab_lds) + P->lds_nodes[0], hints, sx);
+        else if constexpr (kSmall)
+          return NodesT<R, false, true>(NodeType<R>::global(P), hints, sx);
         else
-          return NodesT<R, false>(P);
+          return NodesT<R>(P);
       }();
       const uint32_t *jump = [&] {
         if constexpr (kLds != kLdsNone)
@@ -772,7 +782,7 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
         else if (task.type == 1)
           transport_task<R, true, kMode>(a, P, N1, S, wh, task);
         else
-          interact_task<R>(a, P, jump, S, wh, task, td);
+          interact_task<R>(a, P, N0, jump, S, wh, task, td);
         if (a.prof && lane() == 0) {
           const int part = task.type < 2 ? kStatTimeN + task.type : (task.type < 5 ? kStatTimeIN : kStatTimeIC);
           atomicAdd(&S.stat[part], (unsigned long long)(wall_clock64() - t0 - td));

@@ -35,8 +35,8 @@ struct alignas(16) Node32 {
   float x, y, d2, pad;
 };
 
-// What a step-loop launch stages in LDS: nothing; the photon tables and the
-// jump table; those and the e-/e+ tables.
+// What a step-loop launch stages in LDS: nothing; the photon tables, the jump
+// table, the Sandia rows and the search hints; those and the e-/e+ tables.
 enum { kLdsNone = 0, kLdsPhotons, kLdsAll };
 
 // One physics vector inside the node array (nodes [off, off+n)).
@@ -185,6 +185,7 @@ struct DevParams {
   int msc;            // e-/e+ multiple scattering
   uint32_t seed[6];
   int nsandia, nshells;     // doubles in the Sandia and shell arrays
+  int nsx, nhints;          // entries of sx and hints, both to whole 16-byte words
   const uint32_t *jump8;    // first row of A_c^(d 2^(76+8k)) mod m_c at (k * 256 + d) * kJumpRow + 3 c
   const Node64 *nd;             // physics-vector nodes, FP64
   const Node32 *nf;             // FP32 mirror
@@ -198,8 +199,8 @@ struct DevParams {
   // read them from their LDS copy of DevParams
   double sbx[32], sby[57];
   float sbxf[32], sbyf[57];
-  // shell binding energies (MeV) of every element of the slots, innermost
-  // first (DevElement::shell, nshell), read where DevParams is
+  // shell binding energies (MeV) of every element of the slots, falling, the
+  // innermost first (DevElement::shell, nshell), read where DevParams is
   double shell_e[kMaxShells];
   // LDS copies of the physics vectors a transport kernel reads: layout 0 the
   // photon tables (GXT_TAB_LAMBDA_COMPT .. GXT_TAB_LAMBDAPRIM_PHOT), layout 1
