@@ -238,6 +238,7 @@ struct gxt_ctx {
   int npages = 0;
   uint32_t *list = nullptr;  // rings of the pages with tracks and of the free ones
   uint32_t *freel = nullptr;
+  PageSeg *seg = nullptr;    // each workgroup's part of the list, two arrays
   uint32_t ring_mask = 0;
   Counters *cnt = nullptr;
   Snapshot *hsnap = nullptr;  // pinned
@@ -272,6 +273,8 @@ struct gxt_ctx {
   std::vector<std::unique_ptr<Job>> done_unpolled;
   std::map<uint64_t, std::unique_ptr<Job>> finished;
   std::vector<char> ev_used;
+  int64_t events_in_flight = 0;     // at the last admission
+  bool waiting = false;             // events wait for admission
   double committed = 0;             // summed footprint of events in flight
   double tracks_per_gev = 300.0;    // estimated peak live tracks per GeV of an event (learned)
   double seen_sum = 0;              // summed peak per GeV of the events past their maximum
@@ -304,6 +307,7 @@ struct gxt_ctx {
     a.pages = pages;
     a.list = list;
     a.freel = freel;
+    a.seg = seg;
     a.mask = ring_mask;
     a.npages = npages;
     a.rows.bins = rows;
@@ -317,7 +321,20 @@ struct gxt_ctx {
     a.lds_tables = lds_tables;
     a.lds_bytes = lds_bytes;
     a.groups = groups;
+    // Pages stay with their workgroup once there are 8 events or more for each:
+    // the sums per event then find their place in LDS (10,000 e- of 10 GeV, FP32:
+    // 41 ms, shared out evenly 52 ms).  With fewer, an even share of every
+    // kind of page is worth more (257 e- in the calorimeter with msc 22.4 ms,
+    // kept 23.3 ms; 1,000 in the volume tree the same).
+    a.keep = events_in_flight >= 8 * (int64_t)groups;
+    // A launch ends after 1 ms, so that events waiting for admission or jobs
+    // being served get their turn (10,000 e- FP32: 41 ms, at 2 ms 44; a burst of
+    // 20 jobs 13.6 ms, at 2 ms 15.6), or after 2 ms when neither is the case and
+    // every workgroup has 512 tracks or more, past the growth of the showers
+    // (613 e- in the calorimeter: 21.6 -> 20.7 ms; 100 e- of 50 GeV would take
+    // 6.9 in place of 6.4 ms).
     a.ticks = 100000;
+    if (!waiting && !serving.load() && hsnap->live > 512 * (int64_t)groups) a.ticks = 200000;
     a.prof = prof ? 1 : 0;
     return a;
   }
@@ -388,12 +405,16 @@ int admit(gxt_ctx *c) {
   {
     std::lock_guard<std::mutex> lk(c->mu);
     int active = 0;
+    c->events_in_flight = 0;
+    c->waiting = false;
     for (auto &jp : c->jobs) {
       Job *j = jp.get();
       if (!j->started) {
+        c->waiting = true;
         if (active >= c->cfg.max_jobs) break;
         const int eb = alloc_events(c, j->n_events);
         if (eb < 0) break;
+        c->waiting = false;
         j->ev_base = eb;
         j->started = true;
         j->admit_ms = now_ms(c->t0);
@@ -420,7 +441,11 @@ int admit(gxt_ctx *c) {
         ranges.push_back(Range{j->dprims ? j->dprims + p0 : nullptr, j->dtracks ? j->dtracks + p0 : nullptr,
                                p1 - p0, j->ev_base});
       }
-      if (full) break;
+      c->events_in_flight += j->next_event - j->n_done;
+      if (full) {
+        c->waiting = true;
+        break;
+      }
     }
   }
   // everything below is queued on the stream behind the work in flight (the
@@ -654,6 +679,7 @@ void destroy_ctx(gxt_ctx *c) {
   (void)hipFree(c->pages);
   (void)hipFree(c->list);
   (void)hipFree(c->freel);
+  (void)hipFree(c->seg);
   (void)hipFree(c->cnt);
   (void)hipHostFree(c->hsnap);
   (void)hipFree(c->ev);
@@ -927,7 +953,7 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
   // a workgroup per CU, fewer for small pools (at least 4096 tracks each)
-  c->groups = (int)std::min<int64_t>(std::max(cus, 1), std::max<int64_t>(c->cap / 4096, 1));
+  c->groups = (int)std::min<int64_t>(std::min(std::max(cus, 1), kMaxGroups), std::max<int64_t>(c->cap / 4096, 1));
   // physics data
   DevParams &P = c->hd.params;
   std::memset(&P, 0, sizeof(P));
@@ -1024,6 +1050,7 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
   HIP_TRY(dalloc(&c->pages, (size_t)np * (c->precision == GXT_FP32 ? page_bytes<float>() : page_bytes<double>())));
   HIP_TRY(dalloc(&c->list, (size_t)ring));
   HIP_TRY(dalloc(&c->freel, (size_t)ring));
+  HIP_TRY(dalloc(&c->seg, (size_t)2 * c->groups));
   HIP_TRY(dalloc(&c->cnt, 1));
   HIP_TRY(hipMemset(c->cnt, 0, sizeof(Counters)));
   HIP_TRY(hipHostMalloc((void **)&c->hsnap, sizeof(Snapshot), hipHostMallocDefault));

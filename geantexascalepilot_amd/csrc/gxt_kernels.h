@@ -28,6 +28,7 @@ struct LoopArgs {
   char *pages;       // npages pages of page_bytes<R>()
   uint32_t *list;    // ring of the pages with tracks, mask + 1 entries (Rings)
   uint32_t *freel;   // ring of the free pages, mask + 1 entries
+  PageSeg *seg;      // two arrays of `groups` (Rings::parity)
   uint32_t mask;
   int npages;
   TallyRows rows;
@@ -39,6 +40,7 @@ struct LoopArgs {
   int lds_tables;    // staged in LDS (kLds*)
   int lds_bytes;     // dynamic LDS they take
   int groups;        // workgroups launched (at most)
+  int keep;          // workgroups keep their pages from launch to launch
   int ticks;         // 100 MHz ticks after which a workgroup starts no further task
   int prof;          // accumulate the time of the loop's parts (kStatTime*)
 };
@@ -60,7 +62,7 @@ struct SampleArgs {
 // One launch of the step loop (gxt_loop.h) on a.groups workgroups.  e0, e1 (may
 // be null) take the kernel's start and end.
 // LDS of a launch beside its dynamic tables, and all of a workgroup's.
-constexpr int kLoopLdsFixed = 31 * 1024;
+constexpr int kLoopLdsFixed = 39 * 1024;
 constexpr int kLoopLds = 160 * 1024;
 template <class R>
 hipError_t launch_loop(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);

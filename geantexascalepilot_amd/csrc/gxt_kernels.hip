@@ -2,6 +2,8 @@
 // snapshot) and of the component entry points.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "gxt_step.h"
 
 namespace gxt {
@@ -95,14 +97,18 @@ __global__ __launch_bounds__(kBlock) void k_inject(LoopArgs a, const In *prim, i
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_pages_init(Counters *cnt, uint32_t *freel, int npages) {
+__global__ __launch_bounds__(kBlock) void k_pages_init(Counters *cnt, uint32_t *freel, PageSeg *seg, int npages,
+                                                       int groups) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i < npages) freel[i] = (uint32_t)i;
+  if (i < 2 * groups) seg[i] = PageSeg{0u, 0u};
   if (i == 0) {
     Rings &r = cnt->rings;
     r.lhead = r.ltail = r.fhead = r.lpush = r.fpush = 0;
     r.ftail = (unsigned long long)npages;
     r.done = r.ran = r.ran_last = 0;
+    r.parity = 0;
+    r.seg_lo = r.seg_hi = 0;
     r.live = 0;
   }
 }
@@ -368,7 +374,8 @@ template hipError_t launch_inject<double, gxt_track>(const LoopArgs &, const gxt
 template hipError_t launch_inject<float, gxt_track>(const LoopArgs &, const gxt_track *, int, int, int, hipStream_t);
 
 hipError_t launch_pages_init(const LoopArgs &a, hipStream_t st) {
-  hipLaunchKernelGGL(k_pages_init, dim3(grid_for(a.npages)), dim3(kBlock), 0, st, a.cnt, a.freel, a.npages);
+  hipLaunchKernelGGL(k_pages_init, dim3(grid_for(std::max(a.npages, 2 * a.groups))), dim3(kBlock), 0, st, a.cnt,
+                     a.freel, a.seg, a.npages, a.groups);
   return hipGetLastError();
 }
 

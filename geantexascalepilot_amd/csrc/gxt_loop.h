@@ -284,6 +284,109 @@ __device__ __forceinline__ void commit(Sched &S, int f, int n) {
   if (l == 0) lds_add(S.busy, 256 - 1);
 }
 
+// ------------------------------------------------------------------ event tallies
+// The workgroup's sums per event, in LDS, added to the events' records when the
+// launch ends.  A workgroup keeps its pages from launch to launch, so its
+// tracks belong to few events; one that finds no place goes to its record
+// directly.  (With every death, secondary and live count an atomic in device
+// memory, 0.99e9 of them bounded the loop: 10,000 e- of 10 GeV in FP32 took
+// 55.5 ms with and 39.7 ms without them.)
+constexpr int kEvSlots = 128;
+constexpr int kEvProbe = 4;
+struct EventSums {
+  double edep[kEvSlots], visible[kEvSlots], leak[kEvSlots], clen[kEvSlots];
+  unsigned long long nsteps[kEvSlots];
+  int tag[kEvSlots];  // event slot, -1: none
+  int live[kEvSlots];
+  unsigned int nsec[3][kEvSlots], npairs[kEvSlots], nannihil[kEvSlots];
+};
+
+// Where the event's sums are kept, -1: in its record.
+__device__ __forceinline__ int event_slot(EventSums &E, int event) {
+  for (int k = 0; k < kEvProbe; ++k) {
+    const int s = (event + k) & (kEvSlots - 1);
+    const int tag = lds_ld(E.tag[s]);
+    if (tag == event) return s;
+    if (tag < 0 && (lds_cas(E.tag[s], -1, event) || lds_ld(E.tag[s]) == event)) return s;
+  }
+  return -1;
+}
+
+// A task's contribution to a track's event.
+struct EventAdd {
+  double edep = 0.0, visible = 0.0, leak = 0.0, clen = 0.0;
+  int nsteps = 0, live = 0;
+  unsigned int nsec0 = 0, nsec1 = 0, nsec2 = 0, npairs = 0, nannihil = 0;
+  // a track dies: its tallies go to its event
+  template <class R>
+  __device__ __forceinline__ void retire(const TrackRegs<R> &t) {
+    edep = t.aed;
+    visible = t.avis;
+    clen = t.alen;
+    nsteps = t.nsteps;
+  }
+};
+
+__device__ __forceinline__ void event_add(const LoopArgs &a, EventSums &S, int event, const EventAdd &c) {
+  const int s = event_slot(S, event);
+  if (s >= 0) {
+    if (c.edep != 0.0) unsafeAtomicAdd(&S.edep[s], c.edep);
+    if (c.visible != 0.0) unsafeAtomicAdd(&S.visible[s], c.visible);
+    if (c.leak != 0.0) unsafeAtomicAdd(&S.leak[s], c.leak);
+    if (c.clen != 0.0) unsafeAtomicAdd(&S.clen[s], c.clen);
+    if (c.nsteps) atomicAdd(&S.nsteps[s], (unsigned long long)c.nsteps);
+    if (c.live) atomicAdd(&S.live[s], c.live);
+    if (c.nsec0) atomicAdd(&S.nsec[0][s], c.nsec0);
+    if (c.nsec1) atomicAdd(&S.nsec[1][s], c.nsec1);
+    if (c.nsec2) atomicAdd(&S.nsec[2][s], c.nsec2);
+    if (c.npairs) atomicAdd(&S.npairs[s], c.npairs);
+    if (c.nannihil) atomicAdd(&S.nannihil[s], c.nannihil);
+  } else {
+    DevEvent &E = a.ev[event];
+    if (c.edep != 0.0) unsafeAtomicAdd(&E.edep, c.edep);
+    if (c.visible != 0.0) unsafeAtomicAdd(&E.visible, c.visible);
+    if (c.leak != 0.0) unsafeAtomicAdd(&E.leak, c.leak);
+    if (c.clen != 0.0) unsafeAtomicAdd(&E.clen, c.clen);
+    if (c.nsteps) atomicAdd(&E.nsteps, (unsigned long long)c.nsteps);
+    if (c.live) atomicAdd(&a.ev_live[(int64_t)event * kLiveStride], c.live);
+    if (c.nsec0) atomicAdd(&E.nsec[0], (unsigned long long)c.nsec0);
+    if (c.nsec1) atomicAdd(&E.nsec[1], (unsigned long long)c.nsec1);
+    if (c.nsec2) atomicAdd(&E.nsec[2], (unsigned long long)c.nsec2);
+    if (c.npairs) atomicAdd(&E.npairs, (unsigned long long)c.npairs);
+    if (c.nannihil) atomicAdd(&E.nannihil, (unsigned long long)c.nannihil);
+  }
+}
+
+__device__ __forceinline__ void events_clear(EventSums &S) {
+  for (int s = (int)threadIdx.x; s < kEvSlots; s += (int)blockDim.x) {
+    S.edep[s] = S.visible[s] = S.leak[s] = S.clen[s] = 0.0;
+    S.nsteps[s] = 0;
+    S.tag[s] = -1;
+    S.live[s] = 0;
+    for (int k = 0; k < 3; ++k) S.nsec[k][s] = 0;
+    S.npairs[s] = S.nannihil[s] = 0;
+  }
+}
+
+// By all threads of the workgroup, with a barrier before.
+__device__ __forceinline__ void events_flush(const LoopArgs &a, const EventSums &S) {
+  for (int s = (int)threadIdx.x; s < kEvSlots; s += (int)blockDim.x) {
+    const int event = S.tag[s];
+    if (event < 0) continue;
+    DevEvent &E = a.ev[event];
+    if (S.edep[s] != 0.0) unsafeAtomicAdd(&E.edep, S.edep[s]);
+    if (S.visible[s] != 0.0) unsafeAtomicAdd(&E.visible, S.visible[s]);
+    if (S.leak[s] != 0.0) unsafeAtomicAdd(&E.leak, S.leak[s]);
+    if (S.clen[s] != 0.0) unsafeAtomicAdd(&E.clen, S.clen[s]);
+    if (S.nsteps[s]) atomicAdd(&E.nsteps, S.nsteps[s]);
+    if (S.live[s]) atomicAdd(&a.ev_live[(int64_t)event * kLiveStride], S.live[s]);
+    for (int k = 0; k < 3; ++k)
+      if (S.nsec[k][s]) atomicAdd(&E.nsec[k], (unsigned long long)S.nsec[k][s]);
+    if (S.npairs[s]) atomicAdd(&E.npairs, (unsigned long long)S.npairs[s]);
+    if (S.nannihil[s]) atomicAdd(&E.nannihil, (unsigned long long)S.nannihil[s]);
+  }
+}
+
 template <class R>
 __device__ __forceinline__ char *page_at(const LoopArgs &a, const Sched &S, int lp) {
   return a.pages + (int64_t)S.gpage[lp] * page_bytes<R>();
@@ -351,7 +454,7 @@ __device__ __forceinline__ int stage_tables(const DevParams *P, int layout, int 
 // kMode as LoopArgs::mode.
 template <class R, bool kCharged, int kMode, class NS>
 __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParams *P, const NS &N, Sched &S,
-                                               Hist &wh, const Task &task) {
+                                               Hist &wh, EventSums &ES, const Task &task) {
   const bool trace = P->trace_events > 0;
   const R mine = (R)P->tracking_cut;
   constexpr int kG = kMode == 4 ? 1 : 0;  // geo_cell form
@@ -504,14 +607,13 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
     if (trace && q >= 0 && q != kQueueAtRest) p.f64(kPtedep) = edep;
   }
   commit(S, f, n);
-  // what needs no answer
-  if (active) {
-    if (escaped) unsafeAtomicAdd(&a.ev[t.event].leak, (double)t.e);
-    if (killed) atomicAdd(&S.stat[kStatKilled], 1ULL);
-    if (dies) {
-      retire(a, t);
-      atomicAdd(&a.ev_live[(int64_t)t.event * kLiveStride], -1);
-    }
+  if (killed) atomicAdd(&S.stat[kStatKilled], 1ULL);
+  if (dies) {
+    EventAdd c;
+    c.retire(t);
+    c.live = -1;
+    if (escaped) c.leak = (double)t.e;
+    event_add(a, ES, t.event, c);
   }
   const int steps = __builtin_amdgcn_readlane(wave_incl_scan(nsub), 63);
   if (lane() == 0) {
@@ -547,7 +649,8 @@ __device__ __forceinline__ int sec_fate(const DevParams *P, TrackRegs<R> &t, Dep
 // tracks created, each with its RNG state.
 template <class R, class NS>
 __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams *P, const NS &N,
-                                              const uint32_t *jump, Sched &S, Hist &wh, const Task &task, long long &t_derive) {
+                                              const uint32_t *jump, Sched &S, Hist &wh, EventSums &ES,
+                                              const Task &task, long long &t_derive) {
   const bool trace = P->trace_events > 0;
   const R mine = (R)P->tracking_cut;
   const int q = task.type - 2;
@@ -614,6 +717,7 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
   int kC = __builtin_amdgcn_readlane(f, 1) + inclC - outC;
   const int w = (int)(threadIdx.x >> 6);
   const long long t0 = a.prof ? wall_clock64() : 0;
+  EventAdd c;
   // new tracks in the oracle's draw order: secondary 0, secondary 1, then the
   // primary's annihilation at rest (two back-to-back 511 keV photons,
   // isotropic); the survivor last
@@ -647,7 +751,9 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
         const int idx = species == 0 ? kN++ : kC++;
         const int pg = S.dest[w][species == 0 ? 0 : 1][idx >> 6];
         store_new(PageSlot<R>(page_at<R>(a, S, pg), idx & 63), t, species, e, d0, d1, d2, uid, rng, trace);
-        atomicAdd(&a.ev[t.event].nsec[species], 1ULL);
+        c.nsec0 += species == 0;
+        c.nsec1 += species == 1;
+        c.nsec2 += species == 2;
         spectrum(wh, species, (double)e);
         d0 = -d0;
         d1 = -d1;
@@ -664,11 +770,12 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
   if (a.prof) t_derive += wall_clock64() - t0;
   if (active) {
     dp.flush(wh);
-    if (pair) atomicAdd(&a.ev[t.event].npairs, 1ULL);
-    if (nannih) atomicAdd(&a.ev[t.event].nannihil, (unsigned long long)nannih);
     if (killed) atomicAdd(&S.stat[kStatKilled], 1ULL);
-    if (!survive) retire(a, t);
-    if (outN + outC != 1) atomicAdd(&a.ev_live[(int64_t)t.event * kLiveStride], outN + outC - 1);
+    c.npairs = pair ? 1u : 0u;
+    c.nannihil = (unsigned int)nannih;
+    if (!survive) c.retire(t);
+    c.live = outN + outC - 1;
+    event_add(a, ES, t.event, c);
   }
   const int made = totN + totC - (int)__popcll(__ballot(survive));
   if (lane() == 0) {
@@ -679,6 +786,90 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
   }
 }
 
+// ------------------------------------------------------------------ sharing out
+// With many events in flight (LoopArgs::keep) a workgroup keeps its pages from
+// launch to launch, so that an event stays with few workgroups; what it has
+// beyond the average goes to those with less, after the pages that belong to
+// none (injected since).  The workgroups' counts n of the last launch give
+// each its own part: with q = ceil(pages / G), s = max(n - q, 0) and d = max(q
+// - n, 0), the surplus is the sequence of the pages of none and the s pages of
+// each workgroup in order, and a workgroup takes from it d pages behind those
+// the workgroups before it take (all find one: the sum of d is at least the sum
+// of s and none, as q G is at least the number of pages).
+struct Shares {
+  uint32_t first[kMaxGroups];  // PageSeg::first
+  int sur[kMaxGroups];         // surplus pages of the workgroups before, + none
+  int wave[8][3];
+  int q, none, own, nt, take0;  // of this workgroup: its own pages, all, its first place in the surplus
+  int rank, groups;             // workgroups with pages: before it, all
+};
+
+__device__ __forceinline__ void share_out(Shares &sh, const PageSeg *seg, int none, int q, int b, int G) {
+  const int tid = (int)threadIdx.x, w = tid >> 6;
+  const PageSeg e = tid < G ? seg[tid] : PageSeg{0u, 0u};
+  const int n = (int)e.count;
+  const int s = max(n - q, 0), d = tid < G ? max(q - n, 0) : 0;
+  const int is = wave_incl_scan(s), id = wave_incl_scan(d);
+  if (lane() == 63 && w < 8) {
+    sh.wave[w][0] = is;
+    sh.wave[w][1] = id;
+  }
+  __syncthreads();
+  int bs = none, bd = 0, total = none;
+  for (int k = 0; k < 8; ++k) {
+    if (k < w) {
+      bs += sh.wave[k][0];
+      bd += sh.wave[k][1];
+    }
+    total += sh.wave[k][0];
+  }
+  const int take0 = bd + id - d;
+  const int nt = tid < G ? min(n, q) + min(max(total - take0, 0), d) : 0;
+  const int ia = wave_incl_scan(nt > 0 ? 1 : 0);
+  if (lane() == 63 && w < 8) sh.wave[w][2] = ia;
+  if (tid < G) {
+    sh.first[tid] = e.first;
+    sh.sur[tid] = bs + is - s;
+  }
+  __syncthreads();
+  if (tid == b) {
+    int r = 0, all = 0;
+    for (int k = 0; k < 8; ++k) {
+      if (k < w) r += sh.wave[k][2];
+      all += sh.wave[k][2];
+    }
+    sh.q = q;
+    sh.none = none;
+    sh.own = min(n, q);
+    sh.nt = nt;
+    sh.take0 = take0;
+    sh.rank = r + ia - (nt > 0 ? 1 : 0);
+    sh.groups = all;
+  }
+  __syncthreads();
+}
+
+// Ring position of page j of the workgroup.
+__device__ __forceinline__ unsigned long long share_entry(const Shares &sh, int j, unsigned long long lhead,
+                                                          unsigned long long seg_lo, unsigned long long seg_hi) {
+  if (j < sh.own) return seg_lo + sh.first[blockIdx.x] + (unsigned)j;
+  const int p = sh.take0 + j - sh.own;
+  if (p < sh.none) {
+    const unsigned long long front = seg_lo - lhead;
+    return (unsigned long long)p < front ? lhead + (unsigned)p : seg_hi + ((unsigned long long)p - front);
+  }
+  // the workgroup whose surplus holds place p: the last with sur <= p
+  int lo = 0, hi = (int)gridDim.x;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (sh.sur[mid] <= p)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  return seg_lo + sh.first[lo] + (unsigned)(sh.q + p - sh.sur[lo]);
+}
+
 // ------------------------------------------------------------------ the loop
 // kLds: the tables in LDS (LoopArgs::lds_tables).
 template <class R, int kMode, int kLds>
@@ -686,20 +877,42 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
   __shared__ Sched S;
   __shared__ DevParams sP;
   __shared__ Hist wh;
-  static_assert(sizeof(Sched) + sizeof(DevParams) + sizeof(Hist) <= kLoopLdsFixed, "LDS beside the tables");
+  __shared__ union {
+    Shares sh;  // until the pages are taken
+    EventSums es;
+  } un;
+  Shares &sh = un.sh;
+  EventSums &ES = un.es;
+  static_assert(sizeof(Sched) + sizeof(DevParams) + sizeof(Hist) + sizeof(un) <= kLoopLdsFixed,
+                "LDS beside the tables");
   const int tid = (int)threadIdx.x;
   Rings &rg = a.cnt->rings;
   // what the launch shares out (the heads and tails move when its last
-  // workgroup ends): workgroup b of `groups` takes pages with tracks lhead +
-  // b + groups j, j < kTake, and `nf` free pages from fhead + b nf on
+  // workgroup ends)
   const unsigned long long lhead = rg.lhead, ltail = rg.ltail, fhead = rg.fhead, ftail = rg.ftail;
+  const unsigned long long seg_lo = rg.seg_lo, seg_hi = rg.seg_hi;
+  const int parity = rg.parity;
   const long long have = (long long)(ltail - lhead);
-  const int b = (int)blockIdx.x;
   const long long spare = (long long)(ftail - fhead);
-  const int groups = (int)max(min(min((long long)gridDim.x, have), spare / kMinFree), 1LL);
-  const long long taken = min(have, (long long)groups * kTake);
-  const int nt = b < groups ? (int)((taken - b + groups - 1) / groups) : 0;
+  const int b = (int)blockIdx.x, G = (int)gridDim.x;
+  // by rank: one of `groups` workgroups takes entries lhead + b + groups j
+  const bool by_rank = !a.keep || have > (long long)G * kTake || spare < (long long)G * kMinFree;
+  int groups = 1, nt = 0, at_free = 0;
+  long long taken = have;
+  if (by_rank) {
+    groups = (int)max(min(min((long long)G, have), spare / kMinFree), 1LL);
+    taken = min(have, (long long)groups * kTake);
+    nt = b < groups ? (int)((taken - b + groups - 1) / groups) : 0;
+    at_free = b;
+  } else if (have > 0) {
+    share_out(sh, a.seg + (int64_t)parity * G, (int)(have - (long long)(seg_hi - seg_lo)), (int)((have + G - 1) / G),
+              b, G);
+    groups = max(sh.groups, 1);
+    nt = sh.nt;
+    at_free = sh.rank;
+  }
   const int nf = have > 0 ? (int)min(spare / groups, (long long)(kLP - kTake)) : 0;
+  PageSeg my_seg = {0u, 0u};
   if (nt > 0) {
     const long long t_end = wall_clock64() + a.ticks;
     hist_clear(wh);
@@ -731,7 +944,9 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     int start_live = 0;
     for (int j = tid; j < nt + nf; j += kLoopBlock) {
       if (j < nt) {
-        const uint32_t en = a.list[(uint32_t)(lhead + (unsigned)b + (unsigned long long)groups * j) & a.mask];
+        const unsigned long long at = by_rank ? lhead + (unsigned)b + (unsigned long long)groups * j
+                                              : share_entry(sh, j, lhead, seg_lo, seg_hi);
+        const uint32_t en = a.list[(uint32_t)at & a.mask];
         const int type = (int)(en >> 6 & 15u), n = (int)(en & 63u) + 1;
         S.gpage[j] = en >> 10;
         S.cnt[j] = n;
@@ -741,10 +956,12 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
         if (n == kPageTracks || !lds_cas(S.open[type], -1, j << 7 | n))
           S.rq[type][lds_add(S.tail[type], 1)] = (uint16_t)(j | (n - 1) << 9);
       } else {
-        S.gpage[j] = a.freel[(uint32_t)(fhead + (unsigned long long)b * nf + (j - nt)) & a.mask];
+        S.gpage[j] = a.freel[(uint32_t)(fhead + (unsigned long long)at_free * nf + (j - nt)) & a.mask];
         S.fr[j - nt] = (uint16_t)j;
       }
     }
+    __syncthreads();
+    events_clear(ES);
     __syncthreads();
     {
       const DevParams *P = &sP;
@@ -778,11 +995,11 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
         const long long t0 = a.prof ? wall_clock64() : 0;
         long long td = 0;
         if (task.type == 0)
-          transport_task<R, false, (kMode == 4 ? 4 : 0)>(a, P, N0, S, wh, task);
+          transport_task<R, false, (kMode == 4 ? 4 : 0)>(a, P, N0, S, wh, ES, task);
         else if (task.type == 1)
-          transport_task<R, true, kMode>(a, P, N1, S, wh, task);
+          transport_task<R, true, kMode>(a, P, N1, S, wh, ES, task);
         else
-          interact_task<R>(a, P, N0, jump, S, wh, task, td);
+          interact_task<R>(a, P, N0, jump, S, wh, ES, task, td);
         if (a.prof && lane() == 0) {
           const int part = task.type < 2 ? kStatTimeN + task.type : (task.type < 5 ? kStatTimeIN : kStatTimeIC);
           atomicAdd(&S.stat[part], (unsigned long long)(wall_clock64() - t0 - td));
@@ -799,6 +1016,7 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
       const unsigned long long lp = atomicAdd(&rg.lpush, (unsigned long long)np);
       const unsigned long long fp = atomicAdd(&rg.fpush, (unsigned long long)nfree);
       S.base[0] = (uint32_t)(ltail + lp);
+      my_seg = PageSeg{(uint32_t)lp, (uint32_t)np};
       S.base[1] = (uint32_t)(ftail + fp);
       if (S.ran) atomicAdd(&rg.ran, 1u);
     }
@@ -828,8 +1046,10 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     live = __builtin_amdgcn_readlane(wave_incl_scan(live), 63);
     if (lane() == 0 && live != 0) atomicAdd((unsigned long long *)&rg.live, (unsigned long long)(long long)live);
     hist_flush(a.rows, a.P, wh);
+    events_flush(a, ES);
     if (tid < kNumStats && S.stat[tid]) atomicAdd(&a.cnt->stat[b % kStripes][tid], S.stat[tid]);
   }
+  if (tid == 0) a.seg[(int64_t)(1 - parity) * G + b] = my_seg;
   // the last workgroup to end moves the rings on
   __threadfence();
   __syncthreads();
@@ -837,6 +1057,9 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     const unsigned long long lp = atomicExch(&rg.lpush, 0ULL), fp = atomicExch(&rg.fpush, 0ULL);
     rg.lhead = lhead + (unsigned long long)taken;
     rg.ltail = ltail + lp;
+    rg.seg_lo = ltail;
+    rg.seg_hi = ltail + lp;
+    rg.parity = 1 - parity;
     rg.fhead = fhead + (unsigned long long)groups * nf;
     rg.ftail = ftail + fp;
     rg.ran_last = atomicExch(&rg.ran, 0u);

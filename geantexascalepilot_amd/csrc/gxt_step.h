@@ -216,16 +216,6 @@ struct Dep {
   }
 };
 
-// A track dies: its tallies go to its event (one set of atomics per track).
-template <class R>
-__device__ __forceinline__ void retire(const LoopArgs &a, const TrackRegs<R> &t) {
-  DevEvent &E = a.ev[t.event];
-  if (t.aed != 0.0) unsafeAtomicAdd(&E.edep, t.aed);
-  if (t.avis != 0.0) unsafeAtomicAdd(&E.visible, t.avis);
-  if (t.alen != 0.0) unsafeAtomicAdd(&E.clen, t.alen);
-  atomicAdd(&E.nsteps, (unsigned long long)t.nsteps);
-}
-
 template <class R>
 __device__ __forceinline__ void trace_rec(const LoopArgs &a, const TrackRegs<R> &t, int proc, double edep) {
   if (t.event >= a.P->trace_events || t.nsteps > a.P->trace_steps) return;

@@ -239,19 +239,27 @@ constexpr uint32_t kMaxPages = 1u << 22;
 
 // The step loop's page lists in device memory, two rings of `mask + 1` entries
 // (at least twice the pages, so that what a launch writes never reaches what it
-// has still to read):
-// list (page_entry of the pages with tracks, [lhead, ltail)) and free pages
-// ([fhead, ftail)).  A launch of the loop takes entries from the heads and
-// writes behind the tails (counted by lpush, fpush); its last workgroup to end
-// moves the heads and tails, so that a launch reads only what was written
-// before it began.
+// has still to read): list (page_entry of the pages with tracks, [lhead,
+// ltail)) and free pages ([fhead, ftail)).  A launch of the loop takes entries
+// from the heads and writes behind the tails (counted by lpush, fpush); its
+// last workgroup to end moves the heads and tails, so that a launch reads only
+// what was written before it began.  Each workgroup's entries are contiguous
+// within [seg_lo, seg_hi), what the last launch wrote: PageSeg of the
+// workgroup in the array of `parity`; the entries before (left over) and
+// behind (injected) belong to none.
 struct alignas(128) Rings {
   unsigned long long lhead, ltail, fhead, ftail;
   unsigned long long lpush, fpush;
   unsigned int done;        // workgroups of the launch that have ended
   unsigned int ran, ran_last;  // workgroups that ran a task in this launch, in the last one
+  int parity;
+  unsigned long long seg_lo, seg_hi;
   long long live;           // tracks in pages
 };
+struct PageSeg {
+  uint32_t first, count;    // entries [seg_lo + first, + count)
+};
+constexpr int kMaxGroups = 512;
 
 enum StatKind { kStatSteps = 0, kStatStepsCharged, kStatKilled, kStatInteractions, kStatCreated, kStatLoaded0,
                 kStatLoaded1, kStatInteractions0, kStatCreated0,
