@@ -126,9 +126,7 @@ __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
       else if (o >= 0 && lds_ld(S.cnt[o >> 7]) == (o & 127))
         key = ((o & 127) << 4) | l;
     }
-#pragma unroll
-    for (int d = 1; d < 16; d <<= 1) key = max(key, __shfl_xor(key, d, 64));
-    key = __builtin_amdgcn_readfirstlane(key);
+    key = row0_max(key);
     // (a launch runs a task wherever it can, so that one that ran none is short of pages)
     if (__builtin_amdgcn_readfirstlane(lds_ld(S.stop)) != 0 ||
         (over && __builtin_amdgcn_readfirstlane(lds_ld(S.ran)) != 0))
@@ -215,12 +213,7 @@ __device__ __forceinline__ int reserve(Sched &S, const Task &task, int n) {
       np = ((f + n + 63) >> 6) - (o >= 0 ? 1 : 0);
       ex = max(np - hv, 0);
     }
-    int incl = ex;
-#pragma unroll
-    for (int d = 1; d < 16; d <<= 1) {
-      const int t = __shfl_up(incl, d, 64);
-      if (l >= d) incl += t;
-    }
+    const int incl = row_incl_scan(ex);
     const int total = __builtin_amdgcn_readlane(incl, kTypes - 1);
     if (total > 0) {
       int tk = 0;
@@ -256,9 +249,7 @@ __device__ __forceinline__ int reserve(Sched &S, const Task &task, int n) {
     }
   }
   // what the task did not take of its needs, and its own page
-  int took = np;
-#pragma unroll
-  for (int d = 1; d < 16; d <<= 1) took += __shfl_xor(took, d, 64);
+  const int took = __builtin_amdgcn_readlane(row_incl_scan(np), kTypes - 1);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   if (l == 0) lds_add(S.avail, task.need + 1 - took);
   return f;

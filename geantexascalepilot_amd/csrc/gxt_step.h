@@ -12,13 +12,35 @@ namespace gxt {
 // ------------------------------------------------------------------ wave helpers
 __device__ __forceinline__ int lane() { return (int)__lane_id(); }
 
+// Scans by DPP moves: VALU instructions, where a shuffle is an LDS access of
+// over 100 cycles in a chain of six.  All 64 lanes must be active.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ int dpp_or(int other, int v) {
+  return __builtin_amdgcn_update_dpp(other, v, kCtrl, kRows, 0xf, false);
+}
+
+// Inclusive sum within each row of 16 lanes.
+__device__ __forceinline__ int row_incl_scan(int v) {
+  v += dpp_or<0x111, 0xf>(0, v);  // row_shr 1, 2, 4, 8
+  v += dpp_or<0x112, 0xf>(0, v);
+  v += dpp_or<0x114, 0xf>(0, v);
+  v += dpp_or<0x118, 0xf>(0, v);
+  return v;
+}
+
+// Largest of lanes 0 .. 15, in every lane.
+__device__ __forceinline__ int row0_max(int v) {
+  v = max(v, dpp_or<0x111, 0xf>(v, v));
+  v = max(v, dpp_or<0x112, 0xf>(v, v));
+  v = max(v, dpp_or<0x114, 0xf>(v, v));
+  v = max(v, dpp_or<0x118, 0xf>(v, v));
+  return __builtin_amdgcn_readlane(v, 15);
+}
+
 __device__ __forceinline__ int wave_incl_scan(int v) {
-  const int l = lane();
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int t = __shfl_up(v, d, 64);
-    if (l >= d) v += t;
-  }
+  v = row_incl_scan(v);
+  v += dpp_or<0x142, 0xa>(0, v);  // row_bcast 15: the sum of rows 0, 2 to rows 1, 3
+  v += dpp_or<0x143, 0xc>(0, v);  // row_bcast 31: the sum of rows 0, 1 to rows 2, 3
   return v;
 }
 
