@@ -340,6 +340,8 @@ int load_material(const std::string &data, int which, double lar_density, HostDa
     dt.base = std::log(v.x[0]) / dt.dl;
     dt.dlf = (float)dt.dl;
     dt.basef = (float)dt.base;
+    dt.idl = 1.0 / dt.dl;
+    dt.idlf = 1.0f / dt.dlf;
     dt.x0 = v.x.front();
     dt.y0 = v.y.front();
     dt.xn = v.x.back();

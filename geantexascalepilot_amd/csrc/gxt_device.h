@@ -24,6 +24,31 @@ constexpr double kHuge = 1.0e300;
 constexpr double kAvogadro = 6.02214179e+23;
 constexpr double kClassicRe = 2.8179402894e-12;
 
+// ------------------------------------------------------------------ division
+// n / d, correctly rounded, from the correctly rounded reciprocal y of d: a
+// quotient within an ulp by one correction with the exact remainder, then
+// Markstein's theorem for a second.  5 operations where a division takes 11;
+// for normal d, n and quotients away from under- and overflow (or n = 0).
+__device__ __forceinline__ double div_by(double n, double d, double y) {
+  double q = n * y;
+  q = fma(fma(-d, q, n), y, q);
+  return fma(fma(-d, q, n), y, q);
+}
+__device__ __forceinline__ float div_by(float n, float d, float y) {
+  float q = n * y;
+  q = fmaf(fmaf(-d, q, n), y, q);
+  return fmaf(fmaf(-d, q, n), y, q);
+}
+// The same for a d without a known reciprocal: the steps of a division without
+// the scaling for extreme exponents (8 operations).
+__device__ __forceinline__ double div_normal(double n, double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma(fma(-d, y, 1.0), y, y);
+  y = fma(fma(-d, y, 1.0), y, y);
+  const double q = n * y;
+  return fma(fma(-d, q, n), y, q);
+}
+
 // ------------------------------------------------------------------ math
 // FP64 log and exp, and what is built on them, computed the same way by the
 // CPU oracle so that both give the same bits (samplers, table bins and
@@ -53,7 +78,7 @@ __device__ __forceinline__ double log_cw(double x) {
     m *= 2.0;
     e -= 1;
   }
-  const double f = (m - 1.0) / (m + 1.0);
+  const double f = div_normal(m - 1.0, m + 1.0);
   const double w = f * f;
   const double t =
       w * (2.0 / 3.0 +
@@ -157,21 +182,15 @@ __device__ __forceinline__ void sincos_cw(double x, double &s, double &c) {
                 z * (-1.0 / 3628800.0 + z * (1.0 / 479001600.0 + z * (-1.0 / 87178291200.0 + z * (1.0 / 20922789888000.0))))));
   const double sr = r + r * z * ps;
   const double cr = (1.0 - 0.5 * z) + z * z * pc;
-  double q = fmod(k, 4.0);
-  if (q < 0.0) q += 4.0;
-  if (q == 0.0) {
-    s = sr;
-    c = cr;
-  } else if (q == 1.0) {
-    s = cr;
-    c = -sr;
-  } else if (q == 2.0) {
-    s = -sr;
-    c = -cr;
-  } else {
-    s = -cr;
-    c = sr;
-  }
+  // k mod 4, from the low bits of the integer (|k| < 2^50: k + 1.5 2^52 holds k's
+  // two's complement in its last bits, exactly)
+  const double kb = k + 0x1.8p52;
+  uint64_t bits;
+  __builtin_memcpy(&bits, &kb, 8);
+  const int q = (int)bits & 3;
+  const double as = (q & 1) ? cr : sr, ac = (q & 1) ? sr : cr;
+  s = (q & 2) ? -as : as;
+  c = (q == 1 || q == 2) ? -ac : ac;
 }
 __device__ __forceinline__ double m_sin(double x) {
   double s, c;
@@ -193,49 +212,6 @@ template <class R> __device__ __forceinline__ R rmin(R a, R b) { return a < b ? 
 template <class R> __device__ __forceinline__ R rmax(R a, R b) { return a > b ? a : b; }
 
 // ------------------------------------------------------------------ MRG32k3a
-// L'Ecuyer's recurrence (random/MRG.hpp:35-45, random/src/MRG32k3a.cpp:123-163)
-// in FP64 arithmetic; the state is held as 32-bit integers (half the registers
-// of doubles; each use converts exactly). a*s < 2^53 is exact; q = floor(p *
-// (1/m)) is exact up to one unit, which the two fix-ups absorb, so the residue
-// is the exact integer residue and the output (one FP64 multiply by norm) is
-// bit-identical to the reference's host branch.
-constexpr double kM1 = 4294967087.0, kM2 = 4294944443.0;
-constexpr double kInvM1 = 1.0 / 4294967087.0, kInvM2 = 1.0 / 4294944443.0;
-constexpr double kA12 = 1403580.0, kA13n = 810728.0, kA21 = 527612.0, kA23n = 1370589.0;
-constexpr double kNorm = 1.0 / (4294967087.0 + 1.0);
-
-struct Rng {
-  uint32_t s[6];
-  __device__ __forceinline__ void load(const uint32_t *plane, int64_t cap, int64_t i) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) s[k] = plane[k * cap + i];
-  }
-  __device__ __forceinline__ void store(uint32_t *plane, int64_t cap, int64_t i) const {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) plane[k * cap + i] = s[k];
-  }
-  __device__ __forceinline__ double uniform() {
-    double p1 = kA12 * (double)s[1] - kA13n * (double)s[0];
-    double k1 = floor(p1 * kInvM1);
-    p1 -= k1 * kM1;
-    if (p1 < 0.0) p1 += kM1;
-    if (p1 >= kM1) p1 -= kM1;
-    s[0] = s[1];
-    s[1] = s[2];
-    s[2] = (uint32_t)p1;
-    double p2 = kA21 * (double)s[5] - kA23n * (double)s[3];
-    double k2 = floor(p2 * kInvM2);
-    p2 -= k2 * kM2;
-    if (p2 < 0.0) p2 += kM2;
-    if (p2 >= kM2) p2 -= kM2;
-    s[3] = s[4];
-    s[4] = s[5];
-    s[5] = (uint32_t)p2;
-    return (p1 > p2) ? (p1 - p2) * kNorm : (p1 - p2 + kM1) * kNorm;
-  }
-  template <class R> __device__ __forceinline__ R u() { return (R)uniform(); }
-};
-
 // Products modulo m = 2^32 - c (c = 209 and 22853 for the two components) need
 // no division: 2^32 = c (mod m), so a 64-bit value x folds to (x >> 32) c +
 // (x & (2^32 - 1)) <= (c + 1)(2^32 - 1).  A row of a matrix times a vector is
@@ -265,7 +241,45 @@ __device__ __forceinline__ void reduce3(uint32_t v[3]) {
 #pragma unroll
   for (int k = 0; k < 3; ++k) v[k] = v[k] >= m ? v[k] - m : v[k];
 }
+// The residue of t < 2^33 for t >> 32 <= 1: 2^32 = c again, then one subtraction,
+// x - m = x + c where that carries.
+template <uint32_t c>
+__device__ __forceinline__ uint32_t reduce33(uint64_t t) {
+  const uint32_t x = (uint32_t)t + ((t >> 32) ? c : 0u);
+  const uint32_t y = x + c;
+  return y < c ? y : x;
+}
 constexpr uint32_t kC1 = 209u, kC2 = 22853u;  // 2^32 - m1, 2^32 - m2
+
+// L'Ecuyer's recurrence (random/MRG.hpp:35-45, random/src/MRG32k3a.cpp:123-163)
+// in 32-bit integers with 64-bit products and the folds above: the exact
+// residues, and (p1 - p2) or (p1 - p2 + m1) exact in 32 bits, so the output
+// (one FP64 multiply by norm) is bit-identical to the reference's host
+// branch.  24 vector instructions; the recurrence in FP64 with floor
+// and two fix-ups per component took 46.
+constexpr double kNorm = 1.0 / (4294967087.0 + 1.0);
+
+struct Rng {
+  uint32_t s[6];
+  __device__ __forceinline__ double uniform() {
+    constexpr uint32_t m1 = 0u - kC1, m2 = 0u - kC2;
+    // a12 s1 - a13n s0 = a12 s1 + a13n (m1 - s0) < 2^54: a fold leaves less than 2^33
+    uint64_t t = fold<kC1>((uint64_t)s[1] * 1403580u + (uint64_t)(m1 - s[0]) * 810728u);
+    const uint32_t p1 = reduce33<kC1>(t);
+    s[0] = s[1];
+    s[1] = s[2];
+    s[2] = p1;
+    // a21 s5 - a23n s3 likewise; two folds
+    t = fold<kC2>(fold<kC2>((uint64_t)s[5] * 527612u + (uint64_t)(m2 - s[3]) * 1370589u));
+    const uint32_t p2 = reduce33<kC2>(t);
+    s[3] = s[4];
+    s[4] = s[5];
+    s[5] = p2;
+    const uint32_t d = p1 - p2;
+    return (double)(p1 > p2 ? d : d + m1) * kNorm;
+  }
+  template <class R> __device__ __forceinline__ R u() { return (R)uniform(); }
+};
 
 // A state is three consecutive values x0 x1 x2 of its recurrence, and A^n maps
 // it to the values n further on.  Each of these is a combination of x0 x1 x2;
@@ -386,6 +400,9 @@ template <class R> using Nodes = NodesT<R, false>;
 template <class R> __device__ __forceinline__ R tdl(const DevTable &t);
 template <> __device__ __forceinline__ double tdl<double>(const DevTable &t) { return t.dl; }
 template <> __device__ __forceinline__ float tdl<float>(const DevTable &t) { return t.dlf; }
+template <class R> __device__ __forceinline__ R tidl(const DevTable &t);
+template <> __device__ __forceinline__ double tidl<double>(const DevTable &t) { return t.idl; }
+template <> __device__ __forceinline__ float tidl<float>(const DevTable &t) { return t.idlf; }
 template <class R> __device__ __forceinline__ R tbase(const DevTable &t);
 template <> __device__ __forceinline__ double tbase<double>(const DevTable &t) { return t.base; }
 template <> __device__ __forceinline__ float tbase<float>(const DevTable &t) { return t.basef; }
@@ -411,9 +428,10 @@ template <class R, class V>
 __device__ __forceinline__ R spline(const V &lo, const V &hi, R e) {
   const R x1 = lo.x, x2 = hi.x;
   const R delta = x2 - x1;
-  const R a = (x2 - e) / delta;
-  const R b = (e - x1) / delta;
-  return a * lo.y + b * hi.y + ((a * a * a - a) * lo.d2 + (b * b * b - b) * hi.d2) * delta * delta / R(6.0);
+  const R a = div_by(x2 - e, delta, lo.idx);
+  const R b = div_by(e - x1, delta, lo.idx);
+  return a * lo.y + b * hi.y +
+         div_by(((a * a * a - a) * lo.d2 + (b * b * b - b) * hi.d2) * delta * delta, R(6.0), R(1.0) / R(6.0));
 }
 
 // ProxyPhysicsVector::Value on a log-binned vector (ProxyPhysicsVector.cu:388-394,469-483).
@@ -424,7 +442,7 @@ __device__ __forceinline__ R pvec_value(const NS &N, const DevTable &t, R e, R l
   tends<R>(t, x0, y0, xn, yn);
   if (e <= x0) return y0;
   if (e >= xn) return yn;
-  int bin = (int)(le / tdl<R>(t) - tbase<R>(t));
+  int bin = (int)(div_by(le, tdl<R>(t), tidl<R>(t)) - tbase<R>(t));
   if (bin > n - 2) bin = n - 2;
   if (bin < 0) bin = 0;
   auto lo = N.at(t, bin);

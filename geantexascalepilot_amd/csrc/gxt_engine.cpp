@@ -160,8 +160,12 @@ int upload(HostData &hd, DeviceData &dd) {
   std::vector<Node64> n64(hd.x.size());
   std::vector<Node32> n32(hd.x.size());
   for (size_t i = 0; i < hd.x.size(); ++i) {
-    n64[i] = Node64{hd.x[i], hd.y[i], hd.d2[i], 0.0};
-    n32[i] = Node32{(float)hd.x[i], (float)hd.y[i], (float)hd.d2[i], 0.0f};
+    // (the last node of a vector has no next: its reciprocal is not used)
+    const double x1 = i + 1 < hd.x.size() ? hd.x[i + 1] : hd.x[i];
+    const double w = x1 - hd.x[i];
+    const float wf = (float)x1 - (float)hd.x[i];
+    n64[i] = Node64{hd.x[i], hd.y[i], hd.d2[i], w != 0.0 ? 1.0 / w : 0.0};
+    n32[i] = Node32{(float)hd.x[i], (float)hd.y[i], (float)hd.d2[i], wf != 0.0f ? 1.0f / wf : 0.0f};
   }
   HIP_TRY(put(&dd.nd, n64));
   HIP_TRY(put(&dd.nf, n32));

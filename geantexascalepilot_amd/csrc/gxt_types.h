@@ -27,12 +27,13 @@ constexpr int kJumpRow = 6;
 constexpr int kJumpWords = 8 * 256 * kJumpRow;
 
 // One node of a physics vector: abscissa (energy or range), value, second
-// derivative; a spline lookup reads two adjacent nodes, 64 B (32 B in FP32).
+// derivative, 1 / (distance to the next node); a spline lookup reads two
+// adjacent nodes, 64 B (32 B in FP32).
 struct alignas(32) Node64 {
-  double x, y, d2, pad;
+  double x, y, d2, idx;
 };
 struct alignas(16) Node32 {
-  float x, y, d2, pad;
+  float x, y, d2, idx;
 };
 
 // What a step-loop launch stages in LDS: nothing; the photon tables, the jump
@@ -47,7 +48,9 @@ struct DevTable {
   int lpad;
   double dl, base;  // log-binning: bin = log(E)/dl - base
   double x0, xn, y0, yn;  // first and last node (the clamps of a lookup)
-  float dlf, basef;
+  double idl;             // 1 / dl
+  float dlf, basef, idlf;
+  float fpad;
   float x0f, xnf, y0f, ynf;
   // search hints of a non-log vector (inverse range): hints[hint + k] is the
   // last node below x[0] 2^(k / hscale), k < nhint (hint < 0: none)
