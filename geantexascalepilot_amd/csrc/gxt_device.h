@@ -1481,25 +1481,29 @@ __device__ __forceinline__ int propagate(const DevParams *P, int species, R e, d
   const R ub[3] = {(R)(P->B[0] / P->bmag), (R)(P->B[1] / P->bmag), (R)(P->B[2] / P->bmag)};
   double remaining = pstep;
   step = 0.0;
+  // one helix step per sub-step, whatever ends it, so that a wave's lanes take
+  // it together (and its code is there once)
   for (int it = 0; it < 64; ++it) {
     const double saf = safety(g, vol, pos);
-    if (remaining <= saf) {
-      helix_step<R>(P->B, P->bmag, q, mom, (R)remaining, pos, dir);
-      step += remaining;
-      return kPhysics;
+    const bool within = remaining <= saf;  // the whole rest is within the safety
+    bool aimed = false;
+    int face = -1;
+    double s = remaining;
+    if (!within) {
+      const double slin = dist_out(g, vol, pos, (double)dir[0], (double)dir[1], (double)dir[2], face);
+      const R pl = mom * (dir[0] * ub[0] + dir[1] * ub[1] + dir[2] * ub[2]);
+      R pt2 = mom * mom - pl * pl;
+      if (pt2 < R(0)) pt2 = R(0);
+      const R pt = m_sqrt(pt2);
+      const double sl = pt > R(0) ? (double)(R(2) * m_sqrt(R(0.1) / (R(0.299792458) * (R)P->bmag / pt))) : kHuge;
+      // aimed step: crosses the aimed face by construction, on its plane
+      aimed = slin <= sl && slin <= remaining;
+      s = aimed ? fmax(slin, 1.0e-6) : fmin(remaining, fmax(sl, saf));
     }
-    int face;
-    const double slin = dist_out(g, vol, pos, (double)dir[0], (double)dir[1], (double)dir[2], face);
-    const R pl = mom * (dir[0] * ub[0] + dir[1] * ub[1] + dir[2] * ub[2]);
-    R pt2 = mom * mom - pl * pl;
-    if (pt2 < R(0)) pt2 = R(0);
-    const R pt = m_sqrt(pt2);
-    const double sl = pt > R(0) ? (double)(R(2) * m_sqrt(R(0.1) / (R(0.299792458) * (R)P->bmag / pt))) : kHuge;
-    if (slin <= sl && slin <= remaining) {
-      // aimed step: cross the aimed face by construction, on its plane
-      const double s = fmax(slin, 1.0e-6);
-      helix_step<R>(P->B, P->bmag, q, mom, (R)s, pos, dir);
-      step += s;
+    helix_step<R>(P->B, P->bmag, q, mom, (R)s, pos, dir);
+    step += s;
+    if (within) return kPhysics;
+    if (aimed) {
       if (face == 0 || face == 1) {
         const int nv = face == 1 ? vol + 1 : vol - 1;
         pos[2] = g.z[face == 1 ? vol + 1 : vol];
@@ -1509,9 +1513,6 @@ __device__ __forceinline__ int propagate(const DevParams *P, int species, R e, d
       }
       return kEscaped;
     }
-    const double s = fmin(remaining, fmax(sl, saf));
-    helix_step<R>(P->B, P->bmag, q, mom, (R)s, pos, dir);
-    step += s;
     remaining -= s;
     const int v2 = locate(g, pos, (double)dir[0], (double)dir[1], (double)dir[2]);
     if (v2 != vol) {
@@ -1577,24 +1578,24 @@ __device__ __forceinline__ int propagate_tree(const DevParams *P, int species, R
   step = 0.0;
   for (int it = 0; it < 64; ++it) {
     const double saf = nav_safety(g, vol, pos);
-    if (remaining <= saf) {
-      helix_step<R>(P->B, P->bmag, q, mom, (R)remaining, pos, dir);
-      step += remaining;
-      return kPhysics;
+    const bool within = remaining <= saf;
+    double s = remaining;
+    if (!within) {
+      int enter;
+      const double v[3] = {(double)dir[0], (double)dir[1], (double)dir[2]};
+      const double slin = nav_boundary(g, vol, pos, v, enter);
+      const R pl = mom * (dir[0] * ub[0] + dir[1] * ub[1] + dir[2] * ub[2]);
+      R pt2 = mom * mom - pl * pl;
+      if (pt2 < R(0)) pt2 = R(0);
+      const R pt = m_sqrt(pt2);
+      const double sl = pt > R(0) ? (double)(R(2) * m_sqrt(R(0.1) / (R(0.299792458) * (R)P->bmag / pt))) : kHuge;
+      // aimed at the boundary when the straight line reaches it within the
+      // sagitta-limited length
+      s = (slin <= sl && slin <= remaining) ? fmax(slin, 1.0e-6) : fmin(remaining, fmax(sl, saf));
     }
-    int enter;
-    const double v[3] = {(double)dir[0], (double)dir[1], (double)dir[2]};
-    const double slin = nav_boundary(g, vol, pos, v, enter);
-    const R pl = mom * (dir[0] * ub[0] + dir[1] * ub[1] + dir[2] * ub[2]);
-    R pt2 = mom * mom - pl * pl;
-    if (pt2 < R(0)) pt2 = R(0);
-    const R pt = m_sqrt(pt2);
-    const double sl = pt > R(0) ? (double)(R(2) * m_sqrt(R(0.1) / (R(0.299792458) * (R)P->bmag / pt))) : kHuge;
-    // aimed at the boundary when the straight line reaches it within the
-    // sagitta-limited length
-    const double s = (slin <= sl && slin <= remaining) ? fmax(slin, 1.0e-6) : fmin(remaining, fmax(sl, saf));
     helix_step<R>(P->B, P->bmag, q, mom, (R)s, pos, dir);
     step += s;
+    if (within) return kPhysics;
     remaining -= s;
     const double w[3] = {(double)dir[0], (double)dir[1], (double)dir[2]};
     const int v2 = nav_relocate(g, vol, pos, w);
@@ -1889,32 +1890,35 @@ __device__ __forceinline__ int propagate_general(const DevParams *P, int species
   double ex = 0.0, eu = 0.0;
   double remaining = pstep;
   step = 0.0;
+  // one stepper call per sub-step, as in propagate
   for (int it = 0; it < 64; ++it) {
     const double saf = safety(g, vol, pos);
     double B[3];
     field_at(F, pos, B);
     const double bm = sqrt(B[0] * B[0] + B[1] * B[1] + B[2] * B[2]);
     const double smax = rk && bm > 0.0 ? kRkMaxSub * GXT_RK_ANGLE * (double)mom / ((-kB2C) * bm) : kHuge;
-    if (remaining <= saf && remaining <= smax) {
-      field_advance<R, kStep>(F, B, bm, q, mom, remaining, pos, dir, ex, eu);
-      step += remaining;
-      return kPhysics;
+    const bool within = remaining <= saf && remaining <= smax;
+    bool aimed = false;
+    int face = -1;
+    double s = remaining;
+    if (!within) {
+      const double slin = dist_out(g, vol, pos, (double)dir[0], (double)dir[1], (double)dir[2], face);
+      double sl = kHuge;
+      if (bm > 0.0) {
+        const R pl = mom * (dir[0] * (R)(B[0] / bm) + dir[1] * (R)(B[1] / bm) + dir[2] * (R)(B[2] / bm));
+        R pt2 = mom * mom - pl * pl;
+        if (pt2 < R(0)) pt2 = R(0);
+        const R pt = m_sqrt(pt2);
+        if (pt > R(0)) sl = (double)(R(2) * m_sqrt(R(0.1) / (R(0.299792458) * (R)bm / pt)));
+      }
+      // aimed step: crosses the aimed face by construction, on its plane
+      aimed = slin <= sl && slin <= remaining && slin <= smax;
+      s = aimed ? fmax(slin, 1.0e-6) : fmin(fmin(remaining, fmax(sl, saf)), smax);
     }
-    int face;
-    const double slin = dist_out(g, vol, pos, (double)dir[0], (double)dir[1], (double)dir[2], face);
-    double sl = kHuge;
-    if (bm > 0.0) {
-      const R pl = mom * (dir[0] * (R)(B[0] / bm) + dir[1] * (R)(B[1] / bm) + dir[2] * (R)(B[2] / bm));
-      R pt2 = mom * mom - pl * pl;
-      if (pt2 < R(0)) pt2 = R(0);
-      const R pt = m_sqrt(pt2);
-      if (pt > R(0)) sl = (double)(R(2) * m_sqrt(R(0.1) / (R(0.299792458) * (R)bm / pt)));
-    }
-    if (slin <= sl && slin <= remaining && slin <= smax) {
-      // aimed step: cross the aimed face by construction, on its plane
-      const double s = fmax(slin, 1.0e-6);
-      field_advance<R, kStep>(F, B, bm, q, mom, s, pos, dir, ex, eu);
-      step += s;
+    field_advance<R, kStep>(F, B, bm, q, mom, s, pos, dir, ex, eu);
+    step += s;
+    if (within) return kPhysics;
+    if (aimed) {
       if (face == 0 || face == 1) {
         const int nv = face == 1 ? vol + 1 : vol - 1;
         pos[2] = g.z[face == 1 ? vol + 1 : vol];
@@ -1924,9 +1928,6 @@ __device__ __forceinline__ int propagate_general(const DevParams *P, int species
       }
       return kEscaped;
     }
-    const double s = fmin(fmin(remaining, fmax(sl, saf)), smax);
-    field_advance<R, kStep>(F, B, bm, q, mom, s, pos, dir, ex, eu);
-    step += s;
     remaining -= s;
     const int v2 = locate(g, pos, (double)dir[0], (double)dir[1], (double)dir[2]);
     if (v2 != vol) {
