@@ -40,14 +40,18 @@ __device__ __forceinline__ float div_by(float n, float d, float y) {
   return fmaf(fmaf(-d, q, n), y, q);
 }
 // The same for a d without a known reciprocal: the steps of a division without
-// the scaling for extreme exponents (8 operations).
-__device__ __forceinline__ double div_normal(double n, double d) {
+// the scaling for extreme exponents (8 operations, 3 more for each further n).
+__device__ __forceinline__ double rcp_normal(double d) {
   double y = __builtin_amdgcn_rcp(d);
   y = fma(fma(-d, y, 1.0), y, y);
-  y = fma(fma(-d, y, 1.0), y, y);
+  return fma(fma(-d, y, 1.0), y, y);
+}
+__device__ __forceinline__ double div_rcp(double n, double d, double y) {
   const double q = n * y;
   return fma(fma(-d, q, n), y, q);
 }
+__device__ __forceinline__ double div_normal(double n, double d) { return div_rcp(n, d, rcp_normal(d)); }
+__device__ __forceinline__ float div_normal(float n, float d) { return n / d; }
 
 // ------------------------------------------------------------------ math
 // FP64 log and exp, and what is built on them, computed the same way by the
@@ -1420,19 +1424,22 @@ __device__ __forceinline__ int nav_find_next_boundary(const DevNav &g, int t, co
 
 // ConstFieldHelixStepper::DoStep (magneticfield/ConstFieldHelixStepper.hpp:164-239)
 // in mm/MeV/tesla; the direction is renormalised (FieldPropagationHandler.cpp:323-330).
-// The arithmetic is in R; the position update is accumulated in FP64.
+// The quotients take div_normal (momenta and fields are normal numbers): with
+// those of the field map they were 8 % of a map's step loop (100 events of 10
+// GeV in a solenoid map, Runge-Kutta: 21.1 -> 19.4 ms).
+// ub: the field's unit vector.  The arithmetic is in R; the position update is
+// accumulated in FP64.
 template <class R>
-__device__ __forceinline__ void helix_step(const double B[3], double bmag, R charge, R mom, R step, double pos[3], R dir[3]) {
-  const R ub[3] = {(R)(B[0] / bmag), (R)(B[1] / bmag), (R)(B[2] / bmag)};
+__device__ __forceinline__ void helix_step(const R ub[3], double bmag, R charge, R mom, R step, double pos[3], R dir[3]) {
   const R uvb = dir[0] * ub[0] + dir[1] * ub[1] + dir[2] * ub[2];
   R dt2 = dir[0] * dir[0] + dir[1] * dir[1] + dir[2] * dir[2] - uvb * uvb;
   if (dt2 < R(0)) dt2 = R(0);
   const R sinvb = m_sqrt(dt2) + R(1.0e-30);
-  const R Rad = mom * sinvb / (R(kB2C) * charge * (R)bmag);
+  const R Rad = div_normal(mom * sinvb, R(kB2C) * charge * (R)bmag);
   R vx[3] = {dir[0] - uvb * ub[0], dir[1] - uvb * ub[1], dir[2] - uvb * ub[2]};
   unit3(vx[0], vx[1], vx[2]);
   const R cvb[3] = {vx[1] * ub[2] - vx[2] * ub[1], vx[2] * ub[0] - vx[0] * ub[2], vx[0] * ub[1] - vx[1] * ub[0]};
-  const R phi = -step * charge * (R)bmag * R(kB2C) / mom;
+  const R phi = div_normal(-step * charge * (R)bmag * R(kB2C), mom);
   const R sphi = m_sin(phi), cphi = m_cos(phi);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
@@ -1478,7 +1485,7 @@ __device__ __forceinline__ int propagate(const DevParams *P, int species, R e, d
   }
   const R q = species == 1 ? R(-1) : R(1);
   const R mom = m_sqrt(e * (e + R(2) * R(kMe)));
-  const R ub[3] = {(R)(P->B[0] / P->bmag), (R)(P->B[1] / P->bmag), (R)(P->B[2] / P->bmag)};
+  const R ub[3] = {(R)P->ub[0], (R)P->ub[1], (R)P->ub[2]};
   double remaining = pstep;
   step = 0.0;
   // one helix step per sub-step, whatever ends it, so that a wave's lanes take
@@ -1500,7 +1507,7 @@ __device__ __forceinline__ int propagate(const DevParams *P, int species, R e, d
       aimed = slin <= sl && slin <= remaining;
       s = aimed ? fmax(slin, 1.0e-6) : fmin(remaining, fmax(sl, saf));
     }
-    helix_step<R>(P->B, P->bmag, q, mom, (R)s, pos, dir);
+    helix_step<R>(ub, P->bmag, q, mom, (R)s, pos, dir);
     step += s;
     if (within) return kPhysics;
     if (aimed) {
@@ -1573,7 +1580,7 @@ __device__ __forceinline__ int propagate_tree(const DevParams *P, int species, R
   }
   const R q = species == 1 ? R(-1) : R(1);
   const R mom = m_sqrt(e * (e + R(2) * R(kMe)));
-  const R ub[3] = {(R)(P->B[0] / P->bmag), (R)(P->B[1] / P->bmag), (R)(P->B[2] / P->bmag)};
+  const R ub[3] = {(R)P->ub[0], (R)P->ub[1], (R)P->ub[2]};
   double remaining = pstep;
   step = 0.0;
   for (int it = 0; it < 64; ++it) {
@@ -1593,7 +1600,7 @@ __device__ __forceinline__ int propagate_tree(const DevParams *P, int species, R
       // sagitta-limited length
       s = (slin <= sl && slin <= remaining) ? fmax(slin, 1.0e-6) : fmin(remaining, fmax(sl, saf));
     }
-    helix_step<R>(P->B, P->bmag, q, mom, (R)s, pos, dir);
+    helix_step<R>(ub, P->bmag, q, mom, (R)s, pos, dir);
     step += s;
     if (within) return kPhysics;
     remaining -= s;
@@ -1711,8 +1718,8 @@ __device__ __forceinline__ void map_field(const DevField &f, double x, double y,
   const double zmax = f.z0 + (double)(f.nz - 1) * f.dz;
   const double rc = fmin(fmax(r, f.r0), rmax);
   const double zc = fmin(fmax(z, f.z0), zmax);
-  const double fr = (rc - f.r0) / f.dr;
-  const double fz = (zc - f.z0) / f.dz;
+  const double fr = div_by(rc - f.r0, f.dr, f.idr);
+  const double fz = div_by(zc - f.z0, f.dz, f.idz);
   const int ir = min((int)fr, f.nr - 2);
   const int iz = min((int)fz, f.nz - 2);
   const double tr = fr - (double)ir, tz = fz - (double)iz;
@@ -1725,7 +1732,11 @@ __device__ __forceinline__ void map_field(const DevField &f, double x, double y,
   for (int c = 0; c < 3; ++c)
     b[c] = w00 * gld(p + c) + w01 * gld(p + 3 + c) + w10 * gld(q + c) + w11 * gld(q + 3 + c);
   double cs = 1.0, sn = 0.0;
-  if (r > 0.0) {
+  if (r > 0.0 && r < 1e150) {
+    const double inv = rcp_normal(r);
+    cs = div_rcp(x, r, inv);
+    sn = div_rcp(y, r, inv);
+  } else if (r > 0.0) {  // squares that overflowed
     cs = x / r;
     sn = y / r;
   }
@@ -1865,7 +1876,8 @@ __device__ __forceinline__ void field_advance(const DevField &F, const double B[
       ck45_step<R>(F, kq, h, f1, pos, dir, ex, eu);
     }
   } else if (bm > 0.0) {
-    helix_step<R>(B, bm, q, mom, (R)s, pos, dir);
+    const R ub[3] = {(R)(B[0] / bm), (R)(B[1] / bm), (R)(B[2] / bm)};
+    helix_step<R>(ub, bm, q, mom, (R)s, pos, dir);
   } else {
 #pragma unroll
     for (int c = 0; c < 3; ++c) pos[c] += s * (double)dir[c];

@@ -977,6 +977,7 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
   P.B[1] = cfg->field[1];
   P.B[2] = cfg->field[2];
   P.bmag = std::sqrt(P.B[0] * P.B[0] + P.B[1] * P.B[1] + P.B[2] * P.B[2]);
+  for (int k = 0; k < 3; ++k) P.ub[k] = P.B[k] / P.bmag;
   if (cfg->field_map) {
     c->fmap_path = cfg->field_map;
     c->cfg.field_map = c->fmap_path.c_str();

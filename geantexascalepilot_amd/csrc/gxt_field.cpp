@@ -128,6 +128,8 @@ DevField dev_field(const gxt_field_map *m, const double b[3], const double origi
     f.z0 = m->z0;
     f.dr = m->dr;
     f.dz = m->dz;
+    f.idr = 1.0 / f.dr;
+    f.idz = 1.0 / f.dz;
   }
   for (int k = 0; k < 3; ++k) {
     f.b[k] = b ? b[k] : 0.0;

@@ -220,7 +220,8 @@ __global__ void k_helix(double b0, double b1, double b2, const double *charge, c
   const double bmag = sqrt(b0 * b0 + b1 * b1 + b2 * b2);
   double p[3] = {pos[i], pos[n + i], pos[2 * n + i]};
   R d[3] = {(R)dir[i], (R)dir[n + i], (R)dir[2 * n + i]};
-  helix_step<R>(B, bmag, (R)charge[i], (R)mom[i], (R)step[i], p, d);
+  const R ub[3] = {(R)(B[0] / bmag), (R)(B[1] / bmag), (R)(B[2] / bmag)};
+  helix_step<R>(ub, bmag, (R)charge[i], (R)mom[i], (R)step[i], p, d);
   for (int k = 0; k < 3; ++k) {
     pos[k * n + i] = p[k];
     dir[k * n + i] = (double)d[k];

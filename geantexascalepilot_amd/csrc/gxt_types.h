@@ -127,6 +127,7 @@ struct DevField {
   const double *v;         // (Br, Bphi, Bz) in tesla at (ir * nz + iz) * 3; null: uniform b
   int nr, nz;
   double r0, z0, dr, dz;   // first node and spacing (mm)
+  double idr, idz;         // 1 / spacing
   double origin[3];        // setup origin in the map frame (mm)
   double b[3];             // uniform field (tesla) when v is null
   int stepper;             // GXT_STEPPER_*
@@ -176,7 +177,7 @@ constexpr int kNavLdsMax = 48 * 1024;
 struct DevParams {
   DevMaterial mat[kMaxSlots];
   DevGeometry geo;
-  double B[3];
+  double B[3], ub[3];  // uniform field and its unit vector
   double bmag;
   DevField field;
   double tracking_cut;
