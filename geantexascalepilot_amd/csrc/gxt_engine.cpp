@@ -269,7 +269,6 @@ struct gxt_ctx {
   gxt_navigator *nav = nullptr;
   int32_t *cell = nullptr;
   int transport_mode = 0;  // LoopArgs::mode
-  int inner_steps = 4;     // LoopArgs::inner_steps
   int lds_tables = 0, lds_bytes = 0;  // LoopArgs
   // jobs
   std::mutex mu;
@@ -321,7 +320,6 @@ struct gxt_ctx {
     a.trace = trace_buf;
     a.trace_cap = trace_cap;
     a.mode = transport_mode;
-    a.inner_steps = inner_steps;
     a.lds_tables = lds_tables;
     a.lds_bytes = lds_bytes;
     a.groups = groups;
@@ -994,12 +992,6 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
   c->transport_mode = cfg->geometry == GXT_GEOM_TREE
                            ? 4
                            : (P.field.general ? (P.field.stepper == GXT_STEPPER_RK45 ? 3 : 2) : (P.msc ? 1 : 0));
-  // Steps per transport launch for tracks that neither interact nor end (a
-  // track's results do not depend on it).  Measured: in the block 2 is
-  // fastest (10 GeV e- in PbWO4; 1: -2 %, 3: -1 %, 4: -2 %, 6: -4 %); in the
-  // layered calorimeter, where most steps end on a thin layer's face, 4 is
-  // 12 % faster than 2.
-  c->inner_steps = cfg->geometry == GXT_GEOM_BOX ? 2 : 4;
   P.tracking_cut = cfg->tracking_cut;
   P.zbin = cfg->zbin_mm;
   P.rbin = cfg->rbin_mm;

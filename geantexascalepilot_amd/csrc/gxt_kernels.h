@@ -36,7 +36,6 @@ struct LoopArgs {
   int64_t trace_cap;
   int mode;          // transport: 0 plain, 1 with e-/e+ multiple scattering, 2 e-/e+ in a field map with
                      // the local helix, 3 with the RK45 stepper, 4 the volume tree
-  int inner_steps;   // steps a track may take in one task while it neither interacts nor ends (>= 1)
   int lds_tables;    // staged in LDS (kLds*)
   int lds_bytes;     // dynamic LDS they take
   int groups;        // workgroups launched (at most)
