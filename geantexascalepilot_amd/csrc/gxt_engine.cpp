@@ -269,7 +269,7 @@ struct gxt_ctx {
   gxt_navigator *nav = nullptr;
   int32_t *cell = nullptr;
   int transport_mode = 0;  // LoopArgs::mode
-  int lds_tables = 0, lds_bytes = 0;  // LoopArgs
+  int lds_tables = 0, lds_tab_bytes = 0, lds_bytes = 0, ev_slots = 0;  // LoopArgs
   // jobs
   std::mutex mu;
   std::deque<std::unique_ptr<Job>> jobs;   // submitted, not finished (FIFO)
@@ -321,7 +321,9 @@ struct gxt_ctx {
     a.trace_cap = trace_cap;
     a.mode = transport_mode;
     a.lds_tables = lds_tables;
+    a.lds_tab_bytes = lds_tab_bytes;
     a.lds_bytes = lds_bytes;
+    a.ev_slots = ev_slots;
     a.groups = groups;
     // Pages stay with their workgroup once there are 8 events or more for each:
     // the sums per event then find their place in LDS (10,000 e- of 10 GeV, FP32:
@@ -1027,13 +1029,16 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
   if (rc) return rc;
   {
     const int nb = c->precision == GXT_FP32 ? (int)sizeof(Node32) : (int)sizeof(Node64);
-    const int room = kLoopLds - kLoopLdsFixed;
+    const int all = kLoopLds - kLoopLdsFixed, room = all - kMinEvSlots * kEventSumBytes;
     const int b0 = P.lds_nodes[0] * nb, b1 = P.lds_nodes[1] * nb;
     const int bj = kJumpWords * (int)sizeof(uint32_t) + P.nsx * (int)sizeof(double) + P.nhints * (int)sizeof(int);
     // (two slots in FP32: all tables without the jump table would fit as well,
     // and measured the same)
     c->lds_tables = b0 + b1 + bj <= room ? kLdsAll : (b0 + bj <= room ? kLdsPhotons : kLdsNone);
-    c->lds_bytes = c->lds_tables == kLdsAll ? b0 + b1 + bj : (c->lds_tables == kLdsPhotons ? b0 + bj : 0);
+    c->lds_tab_bytes = c->lds_tables == kLdsAll ? b0 + b1 + bj : (c->lds_tables == kLdsPhotons ? b0 + bj : 0);
+    c->ev_slots = kMinEvSlots;
+    while (c->ev_slots < kMaxEvSlots && c->lds_tab_bytes + 2 * c->ev_slots * kEventSumBytes <= all) c->ev_slots *= 2;
+    c->lds_bytes = c->lds_tab_bytes + c->ev_slots * kEventSumBytes;
   }
   // pages, counters, tallies: pages for the capacity, and for each workgroup
   // but one what it holds open or partly filled

@@ -37,7 +37,9 @@ struct LoopArgs {
   int mode;          // transport: 0 plain, 1 with e-/e+ multiple scattering, 2 e-/e+ in a field map with
                      // the local helix, 3 with the RK45 stepper, 4 the volume tree
   int lds_tables;    // staged in LDS (kLds*)
-  int lds_bytes;     // dynamic LDS they take
+  int lds_tab_bytes; // dynamic LDS they take
+  int lds_bytes;     // dynamic LDS with the event sums
+  int ev_slots;      // events with sums in LDS
   int groups;        // workgroups launched (at most)
   int keep;          // workgroups keep their pages from launch to launch
   int ticks;         // 100 MHz ticks after which a workgroup starts no further task
@@ -60,8 +62,10 @@ struct SampleArgs {
 
 // One launch of the step loop (gxt_loop.h) on a.groups workgroups.  e0, e1 (may
 // be null) take the kernel's start and end.
-// LDS of a launch beside its dynamic tables, and all of a workgroup's.
-constexpr int kLoopLdsFixed = 39 * 1024;
+// LDS of a launch beside its tables and event sums, and all of a workgroup's.
+constexpr int kLoopLdsFixed = 31 * 1024;
+constexpr int kEventSumBytes = 72;
+constexpr int kMinEvSlots = 128, kMaxEvSlots = 512;
 constexpr int kLoopLds = 160 * 1024;
 template <class R>
 hipError_t launch_loop(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);

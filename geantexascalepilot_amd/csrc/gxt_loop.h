@@ -307,23 +307,31 @@ __device__ __forceinline__ void commit(Sched &S, int f, int n) {
 // directly.  (With every death, secondary and live count an atomic in device
 // memory, 0.99e9 of them bounded the loop: 10,000 e- of 10 GeV in FP32 took
 // 55.5 ms with and 39.7 ms without them.)
-constexpr int kEvSlots = 128;
+// The slots (LoopArgs::ev_slots, a power of two) are what the tables leave of
+// the LDS, 128 at least: a burst of requests has more events in flight than a
+// batch (with 128 of them 13.7 ms per 100 events, with 512 11.9).
 constexpr int kEvProbe = 4;
+struct EventSum {
+  double edep, visible, leak, clen;
+  unsigned long long nsteps;
+  int tag;  // event slot, -1: none
+  int live;
+  unsigned int nsec[3], npairs, nannihil, pad;
+};
+static_assert(sizeof(EventSum) == kEventSumBytes, "LDS of the event sums");
 struct EventSums {
-  double edep[kEvSlots], visible[kEvSlots], leak[kEvSlots], clen[kEvSlots];
-  unsigned long long nsteps[kEvSlots];
-  int tag[kEvSlots];  // event slot, -1: none
-  int live[kEvSlots];
-  unsigned int nsec[3][kEvSlots], npairs[kEvSlots], nannihil[kEvSlots];
+  EventSum *slot;
+  int n;
 };
 
 // Where the event's sums are kept, -1: in its record.
-__device__ __forceinline__ int event_slot(EventSums &E, int event) {
+__device__ __forceinline__ int event_slot(const EventSums &E, int event) {
   for (int k = 0; k < kEvProbe; ++k) {
-    const int s = (event + k) & (kEvSlots - 1);
-    const int tag = lds_ld(E.tag[s]);
+    const int s = (event + k) & (E.n - 1);
+    int &tag_s = E.slot[s].tag;
+    const int tag = lds_ld(tag_s);
     if (tag == event) return s;
-    if (tag < 0 && (lds_cas(E.tag[s], -1, event) || lds_ld(E.tag[s]) == event)) return s;
+    if (tag < 0 && (lds_cas(tag_s, -1, event) || lds_ld(tag_s) == event)) return s;
   }
   return -1;
 }
@@ -343,20 +351,21 @@ struct EventAdd {
   }
 };
 
-__device__ __forceinline__ void event_add(const LoopArgs &a, EventSums &S, int event, const EventAdd &c) {
+__device__ __forceinline__ void event_add(const LoopArgs &a, const EventSums &S, int event, const EventAdd &c) {
   const int s = event_slot(S, event);
   if (s >= 0) {
-    if (c.edep != 0.0) unsafeAtomicAdd(&S.edep[s], c.edep);
-    if (c.visible != 0.0) unsafeAtomicAdd(&S.visible[s], c.visible);
-    if (c.leak != 0.0) unsafeAtomicAdd(&S.leak[s], c.leak);
-    if (c.clen != 0.0) unsafeAtomicAdd(&S.clen[s], c.clen);
-    if (c.nsteps) atomicAdd(&S.nsteps[s], (unsigned long long)c.nsteps);
-    if (c.live) atomicAdd(&S.live[s], c.live);
-    if (c.nsec0) atomicAdd(&S.nsec[0][s], c.nsec0);
-    if (c.nsec1) atomicAdd(&S.nsec[1][s], c.nsec1);
-    if (c.nsec2) atomicAdd(&S.nsec[2][s], c.nsec2);
-    if (c.npairs) atomicAdd(&S.npairs[s], c.npairs);
-    if (c.nannihil) atomicAdd(&S.nannihil[s], c.nannihil);
+    EventSum &E = S.slot[s];
+    if (c.edep != 0.0) unsafeAtomicAdd(&E.edep, c.edep);
+    if (c.visible != 0.0) unsafeAtomicAdd(&E.visible, c.visible);
+    if (c.leak != 0.0) unsafeAtomicAdd(&E.leak, c.leak);
+    if (c.clen != 0.0) unsafeAtomicAdd(&E.clen, c.clen);
+    if (c.nsteps) atomicAdd(&E.nsteps, (unsigned long long)c.nsteps);
+    if (c.live) atomicAdd(&E.live, c.live);
+    if (c.nsec0) atomicAdd(&E.nsec[0], c.nsec0);
+    if (c.nsec1) atomicAdd(&E.nsec[1], c.nsec1);
+    if (c.nsec2) atomicAdd(&E.nsec[2], c.nsec2);
+    if (c.npairs) atomicAdd(&E.npairs, c.npairs);
+    if (c.nannihil) atomicAdd(&E.nannihil, c.nannihil);
   } else {
     DevEvent &E = a.ev[event];
     if (c.edep != 0.0) unsafeAtomicAdd(&E.edep, c.edep);
@@ -373,33 +382,34 @@ __device__ __forceinline__ void event_add(const LoopArgs &a, EventSums &S, int e
   }
 }
 
-__device__ __forceinline__ void events_clear(EventSums &S) {
-  for (int s = (int)threadIdx.x; s < kEvSlots; s += (int)blockDim.x) {
-    S.edep[s] = S.visible[s] = S.leak[s] = S.clen[s] = 0.0;
-    S.nsteps[s] = 0;
-    S.tag[s] = -1;
-    S.live[s] = 0;
-    for (int k = 0; k < 3; ++k) S.nsec[k][s] = 0;
-    S.npairs[s] = S.nannihil[s] = 0;
+__device__ __forceinline__ void events_clear(const EventSums &S) {
+  for (int s = (int)threadIdx.x; s < S.n; s += (int)blockDim.x) {
+    EventSum &E = S.slot[s];
+    E.edep = E.visible = E.leak = E.clen = 0.0;
+    E.nsteps = 0;
+    E.tag = -1;
+    E.live = 0;
+    E.nsec[0] = E.nsec[1] = E.nsec[2] = E.npairs = E.nannihil = 0;
   }
 }
 
 // By all threads of the workgroup, with a barrier before.
 __device__ __forceinline__ void events_flush(const LoopArgs &a, const EventSums &S) {
-  for (int s = (int)threadIdx.x; s < kEvSlots; s += (int)blockDim.x) {
-    const int event = S.tag[s];
+  for (int s = (int)threadIdx.x; s < S.n; s += (int)blockDim.x) {
+    const EventSum &L = S.slot[s];
+    const int event = L.tag;
     if (event < 0) continue;
     DevEvent &E = a.ev[event];
-    if (S.edep[s] != 0.0) unsafeAtomicAdd(&E.edep, S.edep[s]);
-    if (S.visible[s] != 0.0) unsafeAtomicAdd(&E.visible, S.visible[s]);
-    if (S.leak[s] != 0.0) unsafeAtomicAdd(&E.leak, S.leak[s]);
-    if (S.clen[s] != 0.0) unsafeAtomicAdd(&E.clen, S.clen[s]);
-    if (S.nsteps[s]) atomicAdd(&E.nsteps, S.nsteps[s]);
-    if (S.live[s]) atomicAdd(&a.ev_live[(int64_t)event * kLiveStride], S.live[s]);
+    if (L.edep != 0.0) unsafeAtomicAdd(&E.edep, L.edep);
+    if (L.visible != 0.0) unsafeAtomicAdd(&E.visible, L.visible);
+    if (L.leak != 0.0) unsafeAtomicAdd(&E.leak, L.leak);
+    if (L.clen != 0.0) unsafeAtomicAdd(&E.clen, L.clen);
+    if (L.nsteps) atomicAdd(&E.nsteps, L.nsteps);
+    if (L.live) atomicAdd(&a.ev_live[(int64_t)event * kLiveStride], L.live);
     for (int k = 0; k < 3; ++k)
-      if (S.nsec[k][s]) atomicAdd(&E.nsec[k], (unsigned long long)S.nsec[k][s]);
-    if (S.npairs[s]) atomicAdd(&E.npairs, (unsigned long long)S.npairs[s]);
-    if (S.nannihil[s]) atomicAdd(&E.nannihil, (unsigned long long)S.nannihil[s]);
+      if (L.nsec[k]) atomicAdd(&E.nsec[k], (unsigned long long)L.nsec[k]);
+    if (L.npairs) atomicAdd(&E.npairs, (unsigned long long)L.npairs);
+    if (L.nannihil) atomicAdd(&E.nannihil, (unsigned long long)L.nannihil);
   }
 }
 
@@ -472,7 +482,7 @@ constexpr int kPhotonSteps = 8;  // most steps of a photon in one task
 // kMode as LoopArgs::mode.
 template <class R, bool kCharged, int kMode, class NS>
 __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParams *P, const NS &N, Sched &S,
-                                               Hist &wh, EventSums &ES, const Task &task) {
+                                               Hist &wh, const EventSums &ES, const Task &task) {
   const bool trace = P->trace_events > 0;
   const R mine = (R)P->tracking_cut;
   constexpr int kG = kMode == 4 ? 1 : 0;  // geo_cell form
@@ -675,7 +685,7 @@ __device__ __forceinline__ int sec_fate(const DevParams *P, TrackRegs<R> &t, Dep
 // tracks created, each with its RNG state.
 template <class R, class NS>
 __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams *P, const NS &N,
-                                              const uint32_t *jump, Sched &S, Hist &wh, EventSums &ES,
+                                              const uint32_t *jump, Sched &S, Hist &wh, const EventSums &ES,
                                               const Task &task, long long &t_derive) {
   const bool trace = P->trace_events > 0;
   const R mine = (R)P->tracking_cut;
@@ -903,13 +913,12 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
   __shared__ Sched S;
   __shared__ DevParams sP;
   __shared__ Hist wh;
-  __shared__ union {
-    Shares sh;  // until the pages are taken
-    EventSums es;
-  } un;
-  Shares &sh = un.sh;
-  EventSums &ES = un.es;
-  static_assert(sizeof(Sched) + sizeof(DevParams) + sizeof(Hist) + sizeof(un) <= kLoopLdsFixed,
+  // behind the tables: the event sums, and where they will be, until the
+  // pages are taken, the shares
+  const EventSums ES = {reinterpret_cast<EventSum *>(tab_lds + a.lds_tab_bytes / 16), a.ev_slots};
+  Shares &sh = *reinterpret_cast<Shares *>(ES.slot);
+  static_assert(sizeof(Shares) <= kMinEvSlots * sizeof(EventSum), "the shares and the event sums");
+  static_assert(sizeof(Sched) + sizeof(DevParams) + sizeof(Hist) <= kLoopLdsFixed,
                 "LDS beside the tables");
   const int tid = (int)threadIdx.x;
   Rings &rg = a.cnt->rings;
