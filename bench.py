@@ -549,9 +549,9 @@ def main():
     ks = r64["ks"]
     steps_per_s = ks.track_steps / r64["seconds"]
     # Algorithmic bytes of the dominant kernel: one read and one write of the
-    # pool's track record (140 B in the FP64 form: position 24, direction 24,
+    # pool's track record (116 B in the FP64 form: position 24, direction 24,
     # energy 8, 3 interaction lengths 24, RNG 24, event, volume|species, step
-    # count 4 each, 3 per-track tallies 24) for every track a launch loads.  A
+    # count 4 each) for every track a launch loads.  A
     # track takes up to inner_steps steps in one launch while it neither
     # interacts nor ends, with one load and one store, so the unit is the
     # track loaded, not the track-step.  (The per-track-step figure of 2 x 148 B,

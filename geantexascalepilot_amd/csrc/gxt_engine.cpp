@@ -1312,7 +1312,7 @@ int gxt_get_kernel_stats(gxt_ctx *c, gxt_kernel_stats *o) {
   // x, y, z (FP64) + dir, E, 3 interaction lengths (R) + 6 RNG words + event, meta, nsteps
   // + 3 FP64 per-track tallies
   const int r = c->precision == GXT_FP32 ? 4 : 8;
-  o->record_bytes = 3 * 8 + 7 * r + 6 * 4 + 3 * 4 + 3 * 8;
+  o->record_bytes = 3 * 8 + 7 * r + 6 * 4 + 3 * 4;
   return GXT_OK;
 }
 

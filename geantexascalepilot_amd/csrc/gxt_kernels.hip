@@ -62,7 +62,6 @@ __global__ __launch_bounds__(kBlock) void k_inject(LoopArgs a, const In *prim, i
       t.pos[k] = p.pos[k];
       t.dir[k] = (R)p.dir[k];
     }
-    t.aed = t.avis = t.alen = 0.0;
     t.uid = p.substream;
     inject_state(P, a, p, t);
     if (t.vol < 0) {

@@ -341,13 +341,9 @@ struct EventAdd {
   double edep = 0.0, visible = 0.0, leak = 0.0, clen = 0.0;
   int nsteps = 0, live = 0;
   unsigned int nsec0 = 0, nsec1 = 0, nsec2 = 0, npairs = 0, nannihil = 0;
-  // a track dies: its tallies go to its event
-  template <class R>
-  __device__ __forceinline__ void retire(const TrackRegs<R> &t) {
-    edep = t.aed;
-    visible = t.avis;
-    clen = t.alen;
-    nsteps = t.nsteps;
+  __device__ __forceinline__ void deposit(const Dep &d) {
+    edep += d.e;
+    visible += d.visible;
   }
 };
 
@@ -491,6 +487,7 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
   int q = -1;
   bool survive = false, annihilate = false, dies = false, killed = false, escaped = false;
   int nsub = 0;  // steps taken in this task
+  EventAdd add;
   double edep = 0.0;
   if (active) {
     load_track(PageSlot<R>(page_at<R>(a, S, task.lp), lane()), t, trace);
@@ -577,11 +574,11 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
       if (xs2 > R(0)) t.nil2 -= (R)step * xs2;
       t.nsteps++;
       if (charged && !vac) {
-        t.alen += step;
+        add.clen = step;
         R loss = R(0);
         t.e = along_doit(N, m, t.species == 2, t.e, le, range, (R)step, mine, loss);
         const double mid[3] = {0.5 * (pre[0] + t.pos[0]), 0.5 * (pre[1] + t.pos[1]), 0.5 * (pre[2] + t.pos[2])};
-        dA.add<kG>(P, t, (double)loss, mid, prevol);
+        dA.add<kG>(P, (double)loss, mid, prevol);
         edep += (double)loss;
         if constexpr (kMode != 0) {
           if (lam1 < kMscNone && status != kEscaped && t.e > R(0) && step > 0.0)
@@ -604,11 +601,11 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
       } else {
         if (trace) trace_rec(a, t, tproc, edep);
         if (t.e < mine) {
-          dB.add<kG>(P, t, (double)t.e, t.pos, t.vol);
+          dB.add<kG>(P, (double)t.e, t.pos, t.vol);
           annihilate = t.species == 2;
           dies = !annihilate;
         } else if (t.nsteps >= P->max_steps) {
-          dB.add<kG>(P, t, (double)t.e, t.pos, t.vol);
+          dB.add<kG>(P, (double)t.e, t.pos, t.vol);
           killed = true;
           dies = true;
         } else {
@@ -619,6 +616,8 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
       if (annihilate) q = kQueueAtRest;
       dA.flush(wh);
       dB.flush(wh);
+      add.deposit(dA);
+      add.deposit(dB);
       ++nsub;
       if (kCharged || !survive || nsub >= kPhotonSteps || 2 * (int)__popcll(__ballot(survive)) < task.n) break;
     }
@@ -645,12 +644,11 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
   commit(S, f, n);
   if (killed) atomicAdd(&S.stat[kStatKilled], 1ULL);
   if (dies) {
-    EventAdd c;
-    c.retire(t);
-    c.live = -1;
-    if (escaped) c.leak = (double)t.e;
-    event_add(a, ES, t.event, c);
+    add.nsteps = t.nsteps;
+    add.live = -1;
+    if (escaped) add.leak = (double)t.e;
   }
+  if (active && (dies || add.clen != 0.0 || add.edep != 0.0)) event_add(a, ES, t.event, add);
   const int steps = __builtin_amdgcn_readlane(wave_incl_scan(nsub), 63);
   if (lane() == 0) {
     atomicAdd(&S.stat[kStatSteps], (unsigned long long)steps);
@@ -663,10 +661,10 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
 // Fate of a secondary: 1 pushed (>= tracking cut), 0 deposited, 2 deposited
 // and, a positron, annihilated at rest.
 template <class R>
-__device__ __forceinline__ int sec_fate(const DevParams *P, TrackRegs<R> &t, Dep &dp, const Sec<R> &s, R mine,
+__device__ __forceinline__ int sec_fate(const DevParams *P, const TrackRegs<R> &t, Dep &dp, const Sec<R> &s, R mine,
                                         int &outN, int &outC, int &nannih) {
   if (s.e < mine) {
-    dp.add(P, t, (double)s.e, t.pos, t.vol);
+    dp.add(P, (double)s.e, t.pos, t.vol);
     if (s.species == 2) {
       ++nannih;
       outN += 2;
@@ -716,7 +714,7 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
         sample_charged<R>(P, N, m, q, t.e, t.dir, t.rng, o);
       pair = q == 1 && o.nsec == 2;
       if (q == 7) ++nannih;
-      dp.add(P, t, (double)o.edep, t.pos, t.vol);
+      dp.add(P, (double)o.edep, t.pos, t.vol);
       t.e = o.ekin;
       t.dir[0] = o.d[0];
       t.dir[1] = o.d[1];
@@ -727,14 +725,14 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
     }
     if (t.e > R(0)) {
       if (t.e < mine) {
-        dp.add(P, t, (double)t.e, t.pos, t.vol);
+        dp.add(P, (double)t.e, t.pos, t.vol);
         if (t.species == 2) {
           ++nannih;
           prim_rest = true;
           outN += 2;
         }
       } else if (t.nsteps >= P->max_steps) {
-        dp.add(P, t, (double)t.e, t.pos, t.vol);
+        dp.add(P, (double)t.e, t.pos, t.vol);
         killed = true;
       } else {
         survive = true;
@@ -807,9 +805,10 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
   if (active) {
     dp.flush(wh);
     if (killed) atomicAdd(&S.stat[kStatKilled], 1ULL);
+    c.deposit(dp);
     c.npairs = pair ? 1u : 0u;
     c.nannihil = (unsigned int)nannih;
-    if (!survive) c.retire(t);
+    if (!survive) c.nsteps = t.nsteps;
     c.live = outN + outC - 1;
     event_add(a, ES, t.event, c);
   }

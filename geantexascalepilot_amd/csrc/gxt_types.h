@@ -225,8 +225,8 @@ struct DevParams {
 // tallies stay FP64.
 constexpr int kPageTracks = 64;
 constexpr int kTypes = 2 + kNumQueues;
-enum PageF64 { kPx = 0, kPy, kPz, kPaed, kPavis, kPalen,  // deposit, visible deposit, charged length of the track
-               kPtedep, kPuid,                            // tracing only: step deposit, substream index
+enum PageF64 { kPx = 0, kPy, kPz,
+               kPtedep, kPuid,  // tracing only: step deposit, substream index
                kPageF64 };
 enum PageR { kPdx = 0, kPdy, kPdz, kPe, kPnil0, kPnil1, kPnil2, kPageR };
 enum PageU32 { kPrng = 0, kPevent = 6, kPmeta, kPnsteps, kPageU32 };  // meta: volume | species << 16
