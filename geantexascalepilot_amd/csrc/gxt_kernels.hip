@@ -243,24 +243,28 @@ __global__ void k_field_value(DevField F, const double *pos, double *b, int n) {
 extern __shared__ uint4 nav_lds[];
 
 template <bool kLds>
-__device__ __forceinline__ DevNav nav_view(const DevNav &g, int lds_bytes) {
-  if (!kLds) return g;
-  const uint4 *src = reinterpret_cast<const uint4 *>(g.node);
-  for (int k = threadIdx.x; k < lds_bytes / 16; k += blockDim.x) nav_lds[k] = src[k];
-  __syncthreads();
-  const char *base = reinterpret_cast<const char *>(g.node);
-  const char *lds = reinterpret_cast<const char *>(nav_lds);
-  DevNav l = g;
-  l.node = reinterpret_cast<const NavNode *>(lds);
-  l.grid = reinterpret_cast<const NavGrid *>(lds + (reinterpret_cast<const char *>(g.grid) - base));
-  l.idx = reinterpret_cast<const int32_t *>(lds + (reinterpret_cast<const char *>(g.idx) - base));
-  return l;
+__device__ __forceinline__ auto nav_view(const DevNav &g, int lds_bytes) {
+  if constexpr (!kLds) {
+    return g;
+  } else {
+    constexpr int w = kNavLdsNode / 16;
+    const uint4 *src = reinterpret_cast<const uint4 *>(g.node);
+    const int nodes = 4 * g.ntouch;
+    for (int k = threadIdx.x; k < lds_bytes / 16; k += blockDim.x)
+      nav_lds[k < nodes ? (k >> 2) * w + (k & 3) : k + (w - 4) * g.ntouch] = src[k];
+    __syncthreads();
+    const char *lds = reinterpret_cast<const char *>(nav_lds);
+    const char *rest = lds + (kNavLdsNode - 64) * g.ntouch;
+    const char *base = reinterpret_cast<const char *>(g.node);
+    return NavLds{lds, reinterpret_cast<const NavGrid *>(rest + (reinterpret_cast<const char *>(g.grid) - base)),
+                  reinterpret_cast<const int32_t *>(rest + (reinterpret_cast<const char *>(g.idx) - base)), g.ntouch};
+  }
 }
 
 template <bool kLds>
 __global__ __launch_bounds__(kBlock) void k_nav_locate(DevNav g0, int lds_bytes, const double *pos, const double *dir,
                                                        int32_t *out, int n) {
-  const DevNav g = nav_view<kLds>(g0, lds_bytes);
+  const auto g = nav_view<kLds>(g0, lds_bytes);
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const double p[3] = {pos[i], pos[n + i], pos[2 * n + i]};
     const double v[3] = {dir[i], dir[n + i], dir[2 * n + i]};
@@ -273,7 +277,7 @@ template <bool kLds>
 __global__ __launch_bounds__(kBlock) void k_nav_step(DevNav g0, int lds_bytes, const int32_t *touchable,
                                                      const double *pos, const double *dir, double *snext,
                                                      int32_t *next, double *safety, int n) {
-  const DevNav g = nav_view<kLds>(g0, lds_bytes);
+  const auto g = nav_view<kLds>(g0, lds_bytes);
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int t = touchable[i];
     if (t < 0 || t >= g.ntouch) {
@@ -298,7 +302,7 @@ __global__ __launch_bounds__(kBlock) void k_nav_find_next_boundary(DevNav g0, in
                                                                    const double *pos, const double *dir,
                                                                    const double *pstep, double *snext, int32_t *next,
                                                                    double *safety, int32_t *boundary, int n) {
-  const DevNav g = nav_view<kLds>(g0, lds_bytes);
+  const auto g = nav_view<kLds>(g0, lds_bytes);
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int t = touchable[i];
     const double ps = pstep[i];
@@ -462,9 +466,9 @@ hipError_t launch_field_value(const DevField &F, const double *pos, double *b, i
 
 // LDS form (trees of at most kNavLdsMax bytes): as many workgroups as the
 // CUs hold at once, striding over the queries (one copy of the tree each and
-// no partial second round: for the step, 6 per CU when resident, 8 per CU
-// ran 10 % slower, 12 to 32 per CU tied with 6); otherwise one thread per
-// query.
+// no partial second round: the step's registers leave 6 per CU, held to 8 they
+// spill, 192 us for 86; loading the next query ahead changes nothing);
+// otherwise one thread per query.
 template <class K>
 static dim3 nav_grid(K kernel, int n, int lds_bytes) {
   const int g = grid_for(n);
@@ -482,11 +486,14 @@ static dim3 nav_grid(K kernel, int n, int lds_bytes) {
   return dim3(g < r ? g : r);
 }
 
+// LDS of a workgroup's copy of a tree of lds_bytes.
+static int nav_lds_size(const DevNav &g, int lds_bytes) { return lds_bytes + (kNavLdsNode - 64) * g.ntouch; }
+
 hipError_t launch_nav_locate(const DevNav &g, int lds_bytes, const double *pos, const double *dir, int32_t *out,
                              int n, hipStream_t st) {
   if (lds_bytes > 0)
-    hipLaunchKernelGGL(k_nav_locate<true>, nav_grid(k_nav_locate<true>, n, lds_bytes), dim3(kBlock), lds_bytes, st, g,
-                       lds_bytes, pos, dir, out, n);
+    hipLaunchKernelGGL(k_nav_locate<true>, nav_grid(k_nav_locate<true>, n, nav_lds_size(g, lds_bytes)), dim3(kBlock),
+                       nav_lds_size(g, lds_bytes), st, g, lds_bytes, pos, dir, out, n);
   else
     hipLaunchKernelGGL(k_nav_locate<false>, dim3(grid_for(n)), dim3(kBlock), 0, st, g, 0, pos, dir, out, n);
   return hipGetLastError();
@@ -495,8 +502,8 @@ hipError_t launch_nav_locate(const DevNav &g, int lds_bytes, const double *pos, 
 hipError_t launch_nav_step(const DevNav &g, int lds_bytes, const int32_t *touchable, const double *pos,
                            const double *dir, double *snext, int32_t *next, double *safety, int n, hipStream_t st) {
   if (lds_bytes > 0)
-    hipLaunchKernelGGL(k_nav_step<true>, nav_grid(k_nav_step<true>, n, lds_bytes), dim3(kBlock), lds_bytes, st, g,
-                       lds_bytes, touchable, pos, dir, snext, next, safety, n);
+    hipLaunchKernelGGL(k_nav_step<true>, nav_grid(k_nav_step<true>, n, nav_lds_size(g, lds_bytes)), dim3(kBlock),
+                       nav_lds_size(g, lds_bytes), st, g, lds_bytes, touchable, pos, dir, snext, next, safety, n);
   else
     hipLaunchKernelGGL(k_nav_step<false>, dim3(grid_for(n)), dim3(kBlock), 0, st, g, 0, touchable, pos, dir, snext, next,
                        safety, n);
@@ -507,8 +514,9 @@ hipError_t launch_nav_find_next_boundary(const DevNav &g, int lds_bytes, const i
                                         const double *dir, const double *pstep, double *snext, int32_t *next,
                                         double *safety, int32_t *boundary, int n, hipStream_t st) {
   if (lds_bytes > 0)
-    hipLaunchKernelGGL(k_nav_find_next_boundary<true>, nav_grid(k_nav_find_next_boundary<true>, n, lds_bytes),
-                       dim3(kBlock), lds_bytes, st, g, lds_bytes, touchable, pos, dir, pstep, snext, next, safety,
+    hipLaunchKernelGGL(k_nav_find_next_boundary<true>,
+                       nav_grid(k_nav_find_next_boundary<true>, n, nav_lds_size(g, lds_bytes)), dim3(kBlock),
+                       nav_lds_size(g, lds_bytes), st, g, lds_bytes, touchable, pos, dir, pstep, snext, next, safety,
                        boundary, n);
   else
     hipLaunchKernelGGL(k_nav_find_next_boundary<false>, dim3(grid_for(n)), dim3(kBlock), 0, st, g, 0, touchable, pos,

@@ -539,7 +539,7 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
           if (charged && P->msc) {
             lam1 = msc_lambda1<R>(Nodes<R>(P), m, sp == 2, t.e, le);
             if (lam1 < kMscNone) {
-              const double saf = kMode == 4 ? nav_safety(P->geo.nav, t.vol, t.pos) : safety(P->geo, t.vol, t.pos);
+              const double saf = kMode == 4 ? nav_safety(P->geo.nav, nav_box(P->geo.nav, t.vol), t.pos) : safety(P->geo, t.vol, t.pos);
               const double tlim = fmax(fmax(kMscFacRange * fmax((double)range, lam1), kMscFacSafety * saf), kMscTmin);
               if (tlim < bestd) {
                 bestd = tlim;

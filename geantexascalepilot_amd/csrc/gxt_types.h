@@ -137,7 +137,7 @@ struct DevField {
 // One placed box of a volume tree (a touchable), in global coordinates: boxes
 // are placed by translations only.  Touchables are numbered breadth-first, so
 // the daughters of a touchable are [first, first + count).
-struct alignas(64) NavNode {
+struct alignas(16) NavBox {
   double c[3];     // centre (mm)
   double h[3];     // half-lengths (mm)
   int32_t parent;  // -1 for the world
@@ -145,6 +145,7 @@ struct alignas(64) NavNode {
   int32_t count;
   int32_t volume;  // index into the caller's volume array
 };
+struct alignas(64) NavNode : NavBox {};
 
 // Daughter index of a volume with many daughters: nb bins of its extent
 // along axis ax (mother frame, bin = (x + h) inv); the daughters that may hold
