@@ -325,12 +325,13 @@ struct gxt_ctx {
     a.lds_bytes = lds_bytes;
     a.ev_slots = ev_slots;
     a.groups = groups;
-    // Pages stay with their workgroup once there are 8 events or more for each:
+    // Pages stay with their workgroup once there are 2 events or more for each:
     // the sums per event then find their place in LDS (10,000 e- of 10 GeV, FP32:
-    // 41 ms, shared out evenly 52 ms).  With fewer, an even share of every
-    // kind of page is worth more (257 e- in the calorimeter with msc 22.4 ms,
-    // kept 23.3 ms; 1,000 in the volume tree the same).
-    a.keep = events_in_flight >= 8 * (int64_t)groups;
+    // 35.2 ms, shared out evenly 44.7; 3,000: 11.3 and 14.7; 1,000 in the volume
+    // tree 8.5 and 9.0; from 8 events on, 8.9).  With fewer, an even share of
+    // every kind of page is worth as much or more (257 e- in the calorimeter
+    // with msc 13.5 ms, kept 13.8).
+    a.keep = events_in_flight >= 2 * (int64_t)groups;
     // A launch ends after 1 ms, so that events waiting for admission or jobs
     // being served get their turn (10,000 e- FP32: 41 ms, at 2 ms 44; a burst of
     // 20 jobs 13.6 ms, at 2 ms 15.6), or after 2 ms when neither is the case and
