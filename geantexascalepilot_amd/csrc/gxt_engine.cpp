@@ -277,7 +277,6 @@ struct gxt_ctx {
   std::map<uint64_t, std::unique_ptr<Job>> finished;
   std::vector<char> ev_used;
   int64_t events_in_flight = 0;     // at the last admission
-  bool waiting = false;             // events wait for admission
   double committed = 0;             // summed footprint of events in flight
   double tracks_per_gev = 300.0;    // estimated peak live tracks per GeV of an event (learned)
   double seen_sum = 0;              // summed peak per GeV of the events past their maximum
@@ -333,13 +332,11 @@ struct gxt_ctx {
     // with msc 13.5 ms, kept 13.8).
     a.keep = events_in_flight >= 2 * (int64_t)groups;
     // A launch ends after 1 ms, so that events waiting for admission or jobs
-    // being served get their turn (10,000 e- FP32: 41 ms, at 2 ms 44; a burst of
-    // 20 jobs 13.6 ms, at 2 ms 15.6), or after 2 ms when neither is the case and
-    // every workgroup has 512 tracks or more, past the growth of the showers
-    // (613 e- in the calorimeter: 21.6 -> 20.7 ms; 100 e- of 50 GeV would take
-    // 6.9 in place of 6.4 ms).
+    // being served get their turn and the tracks are shared out again (10,000
+    // e- of 10 GeV, FP32: 35.5 ms, at 1.5 ms 38.1; a burst of 20 jobs 11.3, at
+    // 1.5 ms 11.8; 10 e- of 50 GeV 4.5, at 2 ms 5.1; 0.7 ms: all the same, and so
+    // are 2 ms where nothing waits and every workgroup has 512 tracks or more).
     a.ticks = 100000;
-    if (!waiting && !serving.load() && hsnap->live > 512 * (int64_t)groups) a.ticks = 200000;
     a.prof = prof ? 1 : 0;
     return a;
   }
@@ -411,15 +408,12 @@ int admit(gxt_ctx *c) {
     std::lock_guard<std::mutex> lk(c->mu);
     int active = 0;
     c->events_in_flight = 0;
-    c->waiting = false;
     for (auto &jp : c->jobs) {
       Job *j = jp.get();
       if (!j->started) {
-        c->waiting = true;
         if (active >= c->cfg.max_jobs) break;
         const int eb = alloc_events(c, j->n_events);
         if (eb < 0) break;
-        c->waiting = false;
         j->ev_base = eb;
         j->started = true;
         j->admit_ms = now_ms(c->t0);
@@ -447,10 +441,7 @@ int admit(gxt_ctx *c) {
                                p1 - p0, j->ev_base});
       }
       c->events_in_flight += j->next_event - j->n_done;
-      if (full) {
-        c->waiting = true;
-        break;
-      }
+      if (full) break;
     }
   }
   // everything below is queued on the stream behind the work in flight (the
