@@ -548,49 +548,36 @@ def main():
     value = a.steps * n / r64["seconds"]
     ks = r64["ks"]
     steps_per_s = ks.track_steps / r64["seconds"]
-    # Algorithmic bytes of the dominant kernel: one read and one write of the
-    # pool's track record (116 B in the FP64 form: position 24, direction 24,
-    # energy 8, 3 interaction lengths 24, RNG 24, event, volume|species, step
-    # count 4 each) for every track a launch loads.  A
-    # track takes up to inner_steps steps in one launch while it neither
-    # interacts nor ends, with one load and one store, so the unit is the
-    # track loaded, not the track-step.  (The per-track-step figure of 2 x 148 B,
+    # Algorithmic bytes of the step loop's kernel: one read and one write of a
+    # track record (116 B in the FP64 form: position 24, direction 24, energy 8,
+    # 3 interaction lengths 24, RNG 24, event, volume|species, step count 4
+    # each) for every track a transport or an interaction task loads, and one
+    # write for every track created.  (The per-track-step figure of 2 x 148 B,
     # a nominal record with inverse mean free paths and safety, is reported
     # beside it.)
     rec = int(ks.record_bytes)
-    # The dominant kernel (the rocprofv3 summary in profiles/kernels_c1_fp64.md)
-    # is the photon interaction kernel, then the e-/e+ transport; only their
-    # launches carry HIP events during the timed batches (profile_kernels = 2,
-    # the events taken from the kernels' own dispatches), which keeps the
-    # instrumentation out of the measured throughput.
+    # The launches carry HIP events during the timed batches, taken from the
+    # kernel's own dispatches (profile_kernels = 2); the parts share a launch's
+    # duration out by the waves' time in them.
     launches = max(ks.launches, 1)
-    name = "k_interact<f64,photon>"
-    ms, units, made = ks.interact_neutral_ms, ks.neutral_interactions, ks.neutral_created
-    # a sampled photon's record read and written back (or its slot left:
-    # the record is read whole either way, and a survivor is written whole to
-    # the next pool), plus each created track's record written
-    nbytes = units * 2 * rec + made * rec
-    per_unit = ("2 x %d B per photon sampled (its record read, the survivor written) + %d B per track it "
-                "creates; %d photons sampled, %d tracks created" % (rec, rec, units, made))
+    name = "k_loop<f64>"
+    parts = dict(photon_transport_ms=ks.transport_neutral_ms, charged_transport_ms=ks.transport_charged_ms,
+                 photon_interactions_ms=ks.interact_neutral_ms, charged_interactions_ms=ks.interact_charged_ms,
+                 new_tracks_ms=ks.derive_ms)
+    ms = sum(parts.values())
+    loaded = ks.neutral_loaded + ks.charged_loaded + ks.interactions
+    nbytes = loaded * 2 * rec + ks.created * rec
+    per_unit = ("2 x %d B per track a task loads (its record read and written) + %d B per track created; "
+                "%d + %d tracks loaded by photon and e-/e+ transport, %d by interactions, %d created"
+                % (rec, rec, ks.neutral_loaded, ks.charged_loaded, ks.interactions, ks.created))
     avg_us = 1e3 * ms / launches
     achieved = (nbytes / launches) / (avg_us * 1e-6) / 1e9
-    # the e-/e+ transport, the dominant kernel of earlier builds, for continuity
-    tname = "k_transport<f64,e-/e+>"
-    tms, tunits = ks.transport_charged_ms, ks.charged_loaded
-    tbytes = tunits * 2 * rec
-    tavg = 1e3 * tms / launches
-    tach = (tbytes / launches) / (tavg * 1e-6) / 1e9
-    transport = dict(kernel=tname, achieved=tach, frac=tach / PEAK_HBM_GBS, traffic=profiled_traffic(tname),
-                     avg_launch_us=tavg, bytes_per_launch=tbytes / launches, kernel_ms=tms,
-                     per_unit="2 x %d B per e-/e+ track loaded by a launch (one read and one write of its record), "
-                              "%d tracks loaded for %d e-/e+ steps" % (rec, tunits, ks.charged_steps),
-                     per_track_step_296b_gbs=(ks.charged_steps * 2 * 148 / launches) / (tavg * 1e-6) / 1e9)
     roofline = dict(bound="hbm", achieved=achieved, peak=PEAK_HBM_GBS, unit="GB/s", frac=achieved / PEAK_HBM_GBS,
                     traffic=profiled_traffic(name), kernel=name, launches=int(ks.launches), avg_launch_us=avg_us,
                     bytes_per_launch=nbytes / launches, per_unit=per_unit, record_bytes_in_pool=rec,
-                    kernel_ms=ms, e_transport=transport,
-                    # every track loaded by a transport launch (photons included) over the wall time
-                    whole_run_gbs=(ks.charged_loaded + ks.neutral_loaded) * 2 * rec / r64["seconds"] / 1e9)
+                    kernel_ms=ms, parts=parts,
+                    per_track_step_296b_gbs=ks.track_steps * 2 * 148 / (ms * 1e-3) / 1e9,
+                    whole_run_gbs=nbytes / r64["seconds"] / 1e9)
     e64 = r64["edep"]["edep"]
     out = dict(metric="events/s and track-steps/s, FP32 vs FP64 on 1 MI355X; p99 job latency", value=value,
                unit="events/s", n_gpus=1, steps=a.steps, warmup=a.warmup,
