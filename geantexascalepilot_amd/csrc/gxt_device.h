@@ -521,7 +521,7 @@ template <> __device__ __forceinline__ const float *sb_ygrid<float>(const DevPar
 // Proxy2DVector::Value (Proxy2DVector.cpp:37-67), split in two: the part that
 // depends only on y (its bin and the two value rows), which a rejection loop
 // over x at fixed electron energy computes once, and the lookup at x.  The
-// grid comes from DevParams (an LDS copy in the step kernels); the values
+// grid comes from DevParams (an LDS copy in the step loop); the values
 // from the element's table g (x[32], y[57], v[57][32]).
 template <class R>
 struct SbRow {
@@ -1263,9 +1263,9 @@ constexpr int kNavGridMin = 8;  // daughters from which a volume has a daughter 
 // into 4 groups of banks: the copy was busy for 84 % of the step kernel's time,
 // three quarters of it conflicts.  With 80 bytes (16 groups), each box read
 // once and the quotients by NavRay, 4.2 M steps in the reference's calorimeter
-// went from 161 to 86 us (3.5 TB/s; their arrays alone take 59 us at the rate of
+// went from 161 to 81 us (3.7 TB/s; their arrays alone take 59 us at the rate of
 // a copy), and a step loop in that tree, which reads it in device memory with
-// global instead of flat loads, from 9.7 to 8.9 ms (1,000 e- of 10 GeV).
+// global instead of flat loads, from 9.7 to 8.6 ms (1,000 e- of 10 GeV).
 constexpr int kNavLdsNode = 80;
 struct NavLds {
   const char *node;
@@ -1274,7 +1274,8 @@ struct NavLds {
   int ntouch;
 };
 __device__ __forceinline__ NavBox nav_box(const NavLds &g, int t) {
-  return *reinterpret_cast<const NavBox *>(g.node + t * kNavLdsNode);
+  const NavBox *n = reinterpret_cast<const NavBox *>(g.node + t * kNavLdsNode);
+  return NavBox{{n->c[0], n->c[1], n->c[2]}, {n->h[0], n->h[1], n->h[2]}, n->parent, n->first, n->count, n->volume};
 }
 __device__ __forceinline__ NavBox nav_box(const DevNav &g, int t) {
   const NavNode *n = g.node + t;
@@ -1290,7 +1291,10 @@ __device__ __forceinline__ NavBox nav_box(const DevNav &g, int t) {
   b.volume = gld(&n->volume);
   return b;
 }
-__device__ __forceinline__ NavGrid nav_grid_of(const NavLds &g, int volume) { return g.grid[volume]; }
+__device__ __forceinline__ NavGrid nav_grid_of(const NavLds &g, int volume) {
+  const NavGrid *p = g.grid + volume;
+  return NavGrid{p->inv, p->ax, p->nb, p->off, 0};
+}
 __device__ __forceinline__ NavGrid nav_grid_of(const DevNav &g, int volume) {
   const NavGrid *p = g.grid + volume;
   return NavGrid{gld(&p->inv), gld(&p->ax), gld(&p->nb), gld(&p->off), 0};
@@ -1338,10 +1342,11 @@ __device__ __forceinline__ int nav_descend(const G &g, int t, NavBox m, const do
     if (m.count >= kNavGridMin) {
       const NavGrid gr = nav_grid_of(g, m.volume);
       if (gr.nb > 0) {
-        const double pa = gr.ax == 0 ? p[0] : (gr.ax == 1 ? p[1] : p[2]);
-        const double ca = gr.ax == 0 ? m.c[0] : (gr.ax == 1 ? m.c[1] : m.c[2]);
-        const double ha = gr.ax == 0 ? m.h[0] : (gr.ax == 1 ? m.h[1] : m.h[2]);
-        const int b = nav_bin(pa - ca, ha, gr.inv, gr.nb);
+        // the coordinate plus the half-length of each axis, then one of the
+        // three (a select among array elements keeps the arrays in private
+        // memory, 22 B more written per query: 86 us)
+        const double u0 = (p[0] - m.c[0]) + m.h[0], u1 = (p[1] - m.c[1]) + m.h[1], u2 = (p[2] - m.c[2]) + m.h[2];
+        const int b = nav_bin(gr.ax == 0 ? u0 : (gr.ax == 1 ? u1 : u2), 0.0, gr.inv, gr.nb);
         k = nav_index(g, gr.off + b);
         end = nav_index(g, gr.off + b + 1);
         indexed = true;

@@ -467,7 +467,7 @@ hipError_t launch_field_value(const DevField &F, const double *pos, double *b, i
 // LDS form (trees of at most kNavLdsMax bytes): as many workgroups as the
 // CUs hold at once, striding over the queries (one copy of the tree each and
 // no partial second round: the step's registers leave 6 per CU, held to 8 they
-// spill, 192 us for 86; loading the next query ahead changes nothing);
+// spill, 192 us for 81; loading the next query ahead changes nothing);
 // otherwise one thread per query.
 template <class K>
 static dim3 nav_grid(K kernel, int n, int lds_bytes) {

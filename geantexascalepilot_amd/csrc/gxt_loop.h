@@ -1,6 +1,6 @@
 // gxt_loop.h -- the step loop as one persistent kernel.
 //
-// A launch runs on one workgroup of 8 waves per CU.  Each workgroup takes a
+// A launch runs on one workgroup of 8 or 12 waves per CU.  Each workgroup takes a
 // share of the pages with tracks (64 tracks that wait for the same task:
 // photon transport, e-/e+ transport, or one of the interactions) and of the
 // free pages, and its waves work on their own: a wave takes a page, runs its

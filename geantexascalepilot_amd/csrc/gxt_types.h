@@ -200,8 +200,8 @@ struct DevParams {
   const double *sx;             // merged Sandia breakpoints and coefficients (DevMaterial::sx_*)
   const int *hints;             // search hints of the inverse-range vectors
   // the Seltzer-Berger grid every element shares: reduced photon energy k / T
-  // (32 nodes) and ln(T / MeV) (57 nodes), FP64 and FP32; the step kernels
-  // read them from their LDS copy of DevParams
+  // (32 nodes) and ln(T / MeV) (57 nodes), FP64 and FP32; the step loop
+  // reads them from its LDS copy of DevParams
   double sbx[32], sby[57];
   float sbxf[32], sbyf[57];
   // shell binding energies (MeV) of every element of the slots, falling, the
