@@ -48,7 +48,7 @@ def log(msg):
 
 
 def run_batch(g, abi, precision, n_events, steps, warmup, seed=777, pool=2_000_000):
-    cfg = abi.config_pbwo4_block(max_events=n_events, precision=precision, profile_kernels=2,
+    cfg = abi.config_pbwo4_block(max_events=n_events, precision=precision, profile_kernels=1,
                                  pool_capacity=pool, seed=seed)
     prims = g.make_primaries(seed, abi.ELECTRON, 10000.0, 10000.0, 0.0, n_events)
     import torch
@@ -141,8 +141,8 @@ def field_forms(g, abi, n_events=20000, seed=2468, cpu=False):
             ev = t.event_tallies(1, n_events)
             st = t.stats()
             ks = t.kernel_stats()
-        # the e-/e+ transport against the HBM roofline, as for the headline
-        # (2 x 148 B per e-/e+ step over its HIP-event-timed launches)
+        # the e-/e+ transport against the HBM roofline: 2 x 148 B per e-/e+
+        # step over its part of the launches' time
         gbs = 2 * 148 * ks.charged_steps / max(ks.transport_charged_ms * 1e-3, 1e-12) / 1e9
         out[name] = dict(events_per_s=n_events / dt, seconds=dt, track_steps=int(st.track_steps),
                          ns_per_track_step=1e9 * dt / max(int(st.track_steps), 1),
@@ -557,7 +557,7 @@ def main():
     # beside it.)
     rec = int(ks.record_bytes)
     # The launches carry HIP events during the timed batches, taken from the
-    # kernel's own dispatches (profile_kernels = 2); the parts share a launch's
+    # kernel's own dispatches (profile_kernels); the parts share a launch's
     # duration out by the waves' time in them.
     launches = max(ks.launches, 1)
     name = "k_loop<f64>"
