@@ -482,6 +482,7 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
   const bool trace = P->trace_events > 0;
   const R mine = (R)P->tracking_cut;
   constexpr int kG = kMode == 4 ? 1 : 0;  // geo_cell form
+  const bool volumes = P->geo.nvol > 1;
   const bool active = lane() < task.n;
   TrackRegs<R> t;
   int q = -1;
@@ -614,8 +615,8 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
       }
       // positron at rest: its two photons are made by the interaction task
       if (annihilate) q = kQueueAtRest;
-      dA.flush(wh);
-      dB.flush(wh);
+      dA.flush(wh, volumes);
+      dB.flush(wh, volumes);
       add.deposit(dA);
       add.deposit(dB);
       ++nsub;
@@ -803,7 +804,7 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
   commit(S, f, n);
   if (a.prof) t_derive += wall_clock64() - t0;
   if (active) {
-    dp.flush(wh);
+    dp.flush(wh, P->geo.nvol > 1);
     if (killed) atomicAdd(&S.stat[kStatKilled], 1ULL);
     c.deposit(dp);
     c.npairs = pair ? 1u : 0u;

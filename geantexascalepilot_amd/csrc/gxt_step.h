@@ -74,7 +74,14 @@ __device__ __forceinline__ void hist_clear(Hist &h) {
 __device__ __forceinline__ void hist_flush(const TallyRows &rows, const DevParams *P, const Hist &h) {
   const int nz = P->nz, nr = P->nr, nv = P->geo.nvol;
   double *row = tally_row(rows);
-  for (int i = (int)threadIdx.x; i < nz + nr + nv; i += (int)blockDim.x) {
+  if (nv == 1 && threadIdx.x < 64) {
+    // the one volume's deposit: that of all z bins (Dep::flush)
+    static_assert(kMaxZBins == 64, "a z bin per lane");
+    double s = (int)threadIdx.x < nz ? h.z[threadIdx.x] : 0.0;
+    for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d, 64);
+    if (threadIdx.x == 0 && s != 0.0) unsafeAtomicAdd(&row[nz + nr], s);
+  }
+  for (int i = (int)threadIdx.x; i < nz + nr + (nv == 1 ? 0 : nv); i += (int)blockDim.x) {
     const double v = i < nz ? h.z[i] : (i < nz + nr ? h.r[i - nz] : h.v[i - nz - nr]);
     if (v != 0.0) unsafeAtomicAdd(&row[i], v);
   }
@@ -222,9 +229,12 @@ struct Dep {
     }
     e += de;
   }
-  __device__ __forceinline__ void flush(Hist &h) const {
+  // volumes: more than one.  A single volume takes its sum from the z bins: 64
+  // lanes adding to one word were 2 % of the time (10,000 e- of 10 GeV in
+  // PbWO4: 39.7 -> 39.0 ms in FP64, 34.7 -> 34.0 in FP32).
+  __device__ __forceinline__ void flush(Hist &h, bool volumes) const {
     if (e <= 0.0) return;
-    unsafeAtomicAdd(&h.v[vol], e);
+    if (volumes) unsafeAtomicAdd(&h.v[vol], e);
     unsafeAtomicAdd(&h.z[iz], e);
     unsafeAtomicAdd(&h.r[ir], e);
   }
