@@ -256,7 +256,8 @@ __device__ __forceinline__ uint32_t reduce33(uint64_t t) {
 constexpr uint32_t kC1 = 209u, kC2 = 22853u;  // 2^32 - m1, 2^32 - m2
 
 // L'Ecuyer's recurrence (random/MRG.hpp:35-45, random/src/MRG32k3a.cpp:123-163)
-// in 32-bit integers with 64-bit products and the folds above: the exact
+// in 32-bit integers with 64-bit products and the folds above, for a state of
+// residues (words below m, as every draw and jump leaves them): the exact
 // residues, and (p1 - p2) or (p1 - p2 + m1) exact in 32 bits, so the output
 // (one FP64 multiply by norm) is bit-identical to the reference's host
 // branch.  24 vector instructions; the recurrence in FP64 with floor

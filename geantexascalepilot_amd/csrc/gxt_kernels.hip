@@ -126,13 +126,23 @@ __global__ void k_rng_init(const DevParams *P, const uint32_t *seed, const uint6
   out[6 * i + 5] = v2[2];
 }
 
+// Takes any 32-bit words: the recurrence (Rng) holds residues, so a word of 2^32 -
+// c or more enters as its residue; given back are the last three values of each
+// component, of which those before the draws are the caller's words as they were.
 __global__ void k_rng_draw(uint32_t *states, int n, int k, double *out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  uint32_t in[6];
   Rng r;
-  for (int j = 0; j < 6; ++j) r.s[j] = states[6 * i + j];
+  for (int j = 0; j < 6; ++j) r.s[j] = in[j] = states[6 * i + j];
+  reduce3<kC1>(r.s);
+  reduce3<kC2>(r.s + 3);
   for (int j = 0; j < k; ++j) out[(int64_t)i * k + j] = r.uniform();
-  for (int j = 0; j < 6; ++j) states[6 * i + j] = r.s[j];
+  for (int c = 0; c < 6; c += 3) {
+    states[6 * i + c] = k == 0 ? in[c] : (k == 1 ? in[c + 1] : (k == 2 ? in[c + 2] : r.s[c]));
+    states[6 * i + c + 1] = k == 0 ? in[c + 1] : (k == 1 ? in[c + 2] : r.s[c + 1]);
+    states[6 * i + c + 2] = k == 0 ? in[c + 2] : r.s[c + 2];
+  }
 }
 
 // Straight-line navigation of the analytic geometry for n points (the
