@@ -210,6 +210,7 @@ struct Job {
   std::vector<gxt_track> tracks;    // sorted by event (a job of tracks in flight)
   gxt_track *dtracks = nullptr;     // device copy of tracks
   std::vector<int> ev_first;        // entries [ev_first[e] .. ev_first[e+1]) belong to event e
+  std::vector<int> ev_photons;      // of the entries before ev_first[e], photons
   std::vector<double> ev_gev;       // summed primary energy of each event (GeV)
   std::vector<int> ev_max;          // highest live-track count seen for an event in flight
   std::vector<char> ev_state;       // 0 pending, 1 in flight, 2 finished
@@ -377,6 +378,9 @@ double event_footprint(const gxt_ctx *c, const Job *j, int e, int live) {
   return std::max(peak, 1.25 * live);
 }
 
+// Entries of an injection of several jobs, at most (one job may have more).
+constexpr int64_t kMaxInject = 1 << 30;
+
 int alloc_events(gxt_ctx *c, int n) {
   const int m = (int)c->ev_used.size();
   int run = 0;
@@ -392,17 +396,17 @@ int alloc_events(gxt_ctx *c, int n) {
 }
 
 // Admit events, oldest job first, while their estimated footprint fits the
-// pool budget; inject their primaries from the job's device copy, one kernel
-// launch per job.  Events are admitted whole (all primaries of an event
-// together) and in order, so a job's admitted primaries are contiguous.
+// pool budget; inject their primaries from the jobs' device copies, up to
+// kInjectRanges jobs in one kernel launch, so that they share pages.  Events are
+// admitted whole (all primaries of an event together) and in order, so a job's
+// admitted primaries are contiguous.
 int admit(gxt_ctx *c) {
   const double budget = 0.8 * (double)c->cap;
   struct Range {
-    const gxt_primary *prim;  // a job of primaries, or
-    const gxt_track *trk;     // of tracks in flight
-    int n, event_base;
+    const void *src;
+    int n, photons, event_base;
   };
-  std::vector<Range> ranges;
+  std::vector<Range> ranges[2];  // jobs of primaries, of tracks in flight
   std::vector<std::pair<int, int>> zero_ranges;
   {
     std::lock_guard<std::mutex> lk(c->mu);
@@ -437,8 +441,11 @@ int admit(gxt_ctx *c) {
       }
       if (j->next_event > e0) {
         const int p0 = j->ev_first[e0], p1 = j->ev_first[j->next_event];
-        ranges.push_back(Range{j->dprims ? j->dprims + p0 : nullptr, j->dtracks ? j->dtracks + p0 : nullptr,
-                               p1 - p0, j->ev_base});
+        const int photons = j->ev_photons[j->next_event] - j->ev_photons[e0];
+        if (j->dprims)
+          ranges[0].push_back(Range{j->dprims + p0, p1 - p0, photons, j->ev_base});
+        else
+          ranges[1].push_back(Range{j->dtracks + p0, p1 - p0, photons, j->ev_base});
       }
       c->events_in_flight += j->next_event - j->n_done;
       if (full) break;
@@ -454,18 +461,32 @@ int admit(gxt_ctx *c) {
                            c->stream));
   }
   const LoopArgs a = c->args();
-  for (const Range &r : ranges) {
-    hipError_t e;
-    // spread over the workgroups: pages of 64 once there are that many for each
-    const int fill = std::min(kPageTracks, (r.n + c->groups - 1) / c->groups);
-    if (c->precision == GXT_FP32)
-      e = r.prim ? launch_inject<float>(a, r.prim, r.n, fill, r.event_base, c->stream)
-                 : launch_inject<float>(a, r.trk, r.n, fill, r.event_base, c->stream);
-    else
-      e = r.prim ? launch_inject<double>(a, r.prim, r.n, fill, r.event_base, c->stream)
-                 : launch_inject<double>(a, r.trk, r.n, fill, r.event_base, c->stream);
-    if (e != hipSuccess) return c->fail(GXT_EHIP, std::string("inject: ") + hipGetErrorString(e));
-  }
+  for (int kind = 0; kind < 2; ++kind)
+    for (size_t k = 0; k < ranges[kind].size();) {
+      InjectArgs in{};
+      int64_t n = 0;
+      // (entries are counted in an int: the launch ends before they would not fit)
+      for (; k < ranges[kind].size() && in.nr < kInjectRanges; ++k) {
+        const Range &r = ranges[kind][k];
+        if (in.nr > 0 && n + r.n > kMaxInject) break;
+        in.src[in.nr] = r.src;
+        in.base[in.nr] = r.event_base;
+        n += r.n;
+        in.n[0] += r.photons;
+        in.n[1] += r.n - r.photons;
+        in.first[++in.nr] = (int)n;
+      }
+      // spread over the workgroups: pages of 64 once there are that many for each
+      in.fill = (int)std::min<int64_t>(kPageTracks, (n + c->groups - 1) / c->groups);
+      hipError_t e;
+      if (c->precision == GXT_FP32)
+        e = kind == 0 ? launch_inject<float, gxt_primary>(a, in, c->stream)
+                      : launch_inject<float, gxt_track>(a, in, c->stream);
+      else
+        e = kind == 0 ? launch_inject<double, gxt_primary>(a, in, c->stream)
+                      : launch_inject<double, gxt_track>(a, in, c->stream);
+      if (e != hipSuccess) return c->fail(GXT_EHIP, std::string("inject: ") + hipGetErrorString(e));
+    }
   return GXT_OK;
 }
 
@@ -803,8 +824,15 @@ int queue_job(gxt_ctx *c, std::vector<In> &host, In *&dev, std::unique_ptr<Job> 
   j->n_events = n_events;
   std::stable_sort(host.begin(), host.end(), [](const In &a, const In &b) { return a.event < b.event; });
   j->ev_first.assign(j->n_events + 1, 0);
-  for (const In &p : host) j->ev_first[p.event + 1]++;
-  for (int e = 0; e < j->n_events; ++e) j->ev_first[e + 1] += j->ev_first[e];
+  j->ev_photons.assign(j->n_events + 1, 0);
+  for (const In &p : host) {
+    j->ev_first[p.event + 1]++;
+    j->ev_photons[p.event + 1] += p.species == 0;
+  }
+  for (int e = 0; e < j->n_events; ++e) {
+    j->ev_first[e + 1] += j->ev_first[e];
+    j->ev_photons[e + 1] += j->ev_photons[e];
+  }
   j->ev_gev.assign(j->n_events, 0.0);
   j->ev_max.assign(j->n_events, 0);
   for (const In &p : host) j->ev_gev[p.event] += p.ekin * 1.0e-3;
@@ -1034,7 +1062,7 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
   }
   // pages, counters, tallies: pages for the capacity, and for each workgroup
   // but one what it holds open or partly filled
-  const int64_t np = (c->cap + kPageTracks - 1) / kPageTracks + (int64_t)(c->groups - 1) * 96;
+  const int64_t np = (c->cap + kPageTracks - 1) / kPageTracks + (int64_t)(c->groups - 1) * kMinFree;
   c->npages = (int)np;
   // (a launch reads a ring's entries while workgroups that have ended write
   // behind them: twice the pages)

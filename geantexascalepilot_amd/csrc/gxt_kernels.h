@@ -72,11 +72,20 @@ hipError_t launch_loop(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEven
 // The launch of one transport mode (each mode is compiled in a unit of its own).
 template <class R, int kMode>
 hipError_t launch_loop_mode(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
-// Injects n primaries or tracks in flight (In = gxt_primary, gxt_track) from
-// device memory as pages of up to `fill` tracks; event slots are
-// prim[i].event + event_base.
+// Primaries or tracks in flight (gxt_primary, gxt_track) of up to kInjectRanges
+// jobs, injected together: entry i, first[r] <= i < first[r + 1], is src[r][i -
+// first[r]] and its event slot .event + base[r].
+constexpr int kInjectRanges = 64;
+struct InjectArgs {
+  const void *src[kInjectRanges];
+  int first[kInjectRanges + 1];
+  int base[kInjectRanges];
+  int nr;
+  int n[2];  // of the entries, photons and e-/e+
+  int fill;  // tracks per page, if there are free pages enough
+};
 template <class R, class In>
-hipError_t launch_inject(const LoopArgs &a, const In *prim, int n, int fill, int event_base, hipStream_t st);
+hipError_t launch_inject(const LoopArgs &a, const InjectArgs &in, hipStream_t st);
 // Clears the rings and makes all pages free.
 hipError_t launch_pages_init(const LoopArgs &a, hipStream_t st);
 

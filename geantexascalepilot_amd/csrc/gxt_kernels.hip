@@ -42,21 +42,41 @@ __device__ __forceinline__ void inject_state(const DevParams *P, const LoopArgs 
 }
 
 // Entries In (gxt_primary or gxt_track) become tracks that wait for their
-// transport: each wave takes `fill` entries and writes their photons and
-// their e-/e+ to a free page each.
+// transport.  Photons and e-/e+ fill free pages one after the other, `fill`
+// tracks each, so that an injection takes no more pages than its tracks need,
+// however many jobs they come from (a page or more for each job, and for each
+// wave of it and species class, were 98,000 pages for 400 jobs of 256 photons
+// where 1,600 do).  Fewer than 64 per page, to spread few tracks over the
+// workgroups, only where the free pages leave every workgroup its share.  The
+// last workgroup to end puts the pages on the list.
 template <class R, class In>
-__global__ __launch_bounds__(kBlock) void k_inject(LoopArgs a, const In *prim, int n, int fill, int event_base) {
+__global__ __launch_bounds__(kBlock) void k_inject(LoopArgs a, InjectArgs in) {
   const DevParams *P = a.P;
   Rings &rg = a.cnt->rings;
+  const unsigned long long fhead = rg.fhead, ftail = rg.ftail, ltail = rg.ltail;
+  const long long spare = (long long)(ftail - fhead);
+  int fill = in.fill;
+  if ((in.n[0] + fill - 1) / fill + (in.n[1] + fill - 1) / fill + (long long)a.groups * kMinFree > spare)
+    fill = kPageTracks;
+  const int np[2] = {(in.n[0] + fill - 1) / fill, (in.n[1] + fill - 1) / fill};  // pages set aside for each class
   const bool trace = P->trace_events > 0;
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * fill + lane();
-  const bool active = lane() < fill && i < n;
+  const int n = in.n[0] + in.n[1];
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   TrackRegs<R> t;
   int region = -1;
-  if (active) {
-    const In &p = prim[i];
+  if (i < n) {
+    // the job whose entries hold i
+    int lo = 0, hi = in.nr;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (in.first[mid] <= i)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    const In &p = static_cast<const In *>(in.src[lo])[i - in.first[lo]];
     t.species = p.species;
-    t.event = p.event + event_base;
+    t.event = p.event + in.base[lo];
     t.e = (R)p.ekin;
     for (int k = 0; k < 3; ++k) {
       t.pos[k] = p.pos[k];
@@ -75,24 +95,55 @@ __global__ __launch_bounds__(kBlock) void k_inject(LoopArgs a, const In *prim, i
   for (int r = 0; r < 2; ++r) {
     const unsigned long long m = __ballot(region == r);
     if (!m) continue;
-    const int cnt = (int)__popcll(m);
-    unsigned int page = kMaxPages;
-    if (lane() == 0) {
-      // a launch of the loop moves the free head; here only injections do
-      const unsigned long long at = atomicAdd(&rg.fhead, 1ULL);
-      if (at < rg.ftail) {
-        page = a.freel[(uint32_t)at & a.mask];
-        a.list[(uint32_t)atomicAdd(&rg.ltail, 1ULL) & a.mask] = page_entry(page, r, cnt);
-        atomicAdd((unsigned long long *)&rg.live, (unsigned long long)cnt);
+    unsigned int at = 0;
+    if (lane() == 0) at = atomicAdd(&rg.inj[r], (unsigned int)__popcll(m));
+    at = __builtin_amdgcn_readfirstlane(at);
+    if (region == r) {
+      const unsigned int slot = at + (unsigned int)__popcll(m & ((1ULL << lane()) - 1));
+      const long long k = (long long)(slot / (unsigned int)fill) + (r == 0 ? 0 : np[0]);
+      if (k < spare) {
+        const unsigned int page = a.freel[(uint32_t)(fhead + (unsigned long long)k) & a.mask];
+        store_track(PageSlot<R>(a.pages + (int64_t)page * page_bytes<R>(), (int)(slot % (unsigned int)fill)), t, trace);
       } else {
-        atomicAdd(&rg.fhead, ~0ULL);
         atomicOr(&a.cnt->overflow, 1);
       }
     }
-    page = __builtin_amdgcn_readfirstlane(page);
-    if (page < (unsigned int)a.npages && region == r)
-      store_track(PageSlot<R>(a.pages + (int64_t)page * page_bytes<R>(), (int)__popcll(m & ((1ULL << lane()) - 1))), t,
-                  trace);
+  }
+  __shared__ unsigned int placed[2];
+  __shared__ int last;
+  __threadfence();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    last = atomicAdd(&rg.inj_done, 1u) == gridDim.x - 1;
+    if (last) {
+      placed[0] = atomicExch(&rg.inj[0], 0u);
+      placed[1] = atomicExch(&rg.inj[1], 0u);
+      rg.inj_done = 0;
+    }
+  }
+  __syncthreads();
+  if (!last) return;
+  // pages taken: set aside and there; filled: those with tracks (entries
+  // outside the world took none)
+  const long long take = min((long long)np[0] + np[1], spare);
+  const long long u0 = min((long long)((placed[0] + fill - 1) / fill), take);
+  const long long u1 = max(min((long long)((placed[1] + fill - 1) / fill), take - np[0]), 0LL);
+  for (long long k = threadIdx.x; k < take; k += blockDim.x) {
+    const int r = k < np[0] ? 0 : 1;
+    const long long v = k - (r == 0 ? 0 : np[0]);
+    const uint32_t page = a.freel[(uint32_t)(fhead + (unsigned long long)k) & a.mask];
+    if (v < (r == 0 ? u0 : u1))
+      a.list[(uint32_t)(ltail + (unsigned long long)(v + (r == 0 ? 0 : u0))) & a.mask] =
+          page_entry(page, r, (int)min((long long)placed[r] - v * fill, (long long)fill));
+    else
+      a.freel[(uint32_t)(ftail + (unsigned long long)(v - (r == 0 ? u0 : u1) + (r == 0 ? 0 : min((long long)np[0], take) - u0))) &
+              a.mask] = page;
+  }
+  if (threadIdx.x == 0) {
+    rg.ltail = ltail + (unsigned long long)(u0 + u1);
+    rg.fhead = fhead + (unsigned long long)take;
+    rg.ftail = ftail + (unsigned long long)(take - u0 - u1);
+    rg.live += (long long)placed[0] + placed[1];
   }
 }
 
@@ -109,6 +160,7 @@ __global__ __launch_bounds__(kBlock) void k_pages_init(Counters *cnt, uint32_t *
     r.parity = 0;
     r.seg_lo = r.seg_hi = 0;
     r.live = 0;
+    r.inj[0] = r.inj[1] = r.inj_done = 0;
   }
 }
 
@@ -373,19 +425,16 @@ template hipError_t launch_loop<double>(const LoopArgs &, hipStream_t, hipEvent_
 template hipError_t launch_loop<float>(const LoopArgs &, hipStream_t, hipEvent_t, hipEvent_t);
 
 template <class R, class In>
-hipError_t launch_inject(const LoopArgs &a, const In *prim, int n, int fill, int event_base, hipStream_t st) {
+hipError_t launch_inject(const LoopArgs &a, const InjectArgs &in, hipStream_t st) {
+  const int n = in.n[0] + in.n[1];
   if (n <= 0) return hipSuccess;
-  const int waves = (n + fill - 1) / fill;
-  hipLaunchKernelGGL((k_inject<R, In>), dim3(grid_for(waves * 64)), dim3(kBlock), 0, st, a, prim, n, fill,
-                     event_base);
+  hipLaunchKernelGGL((k_inject<R, In>), dim3(grid_for(n)), dim3(kBlock), 0, st, a, in);
   return hipGetLastError();
 }
-template hipError_t launch_inject<double, gxt_primary>(const LoopArgs &, const gxt_primary *, int, int, int,
-                                                       hipStream_t);
-template hipError_t launch_inject<float, gxt_primary>(const LoopArgs &, const gxt_primary *, int, int, int,
-                                                      hipStream_t);
-template hipError_t launch_inject<double, gxt_track>(const LoopArgs &, const gxt_track *, int, int, int, hipStream_t);
-template hipError_t launch_inject<float, gxt_track>(const LoopArgs &, const gxt_track *, int, int, int, hipStream_t);
+template hipError_t launch_inject<double, gxt_primary>(const LoopArgs &, const InjectArgs &, hipStream_t);
+template hipError_t launch_inject<float, gxt_primary>(const LoopArgs &, const InjectArgs &, hipStream_t);
+template hipError_t launch_inject<double, gxt_track>(const LoopArgs &, const InjectArgs &, hipStream_t);
+template hipError_t launch_inject<float, gxt_track>(const LoopArgs &, const InjectArgs &, hipStream_t);
 
 hipError_t launch_pages_init(const LoopArgs &a, hipStream_t st) {
   hipLaunchKernelGGL(k_pages_init, dim3(grid_for(std::max(a.npages, 2 * a.groups))), dim3(kBlock), 0, st, a.cnt,

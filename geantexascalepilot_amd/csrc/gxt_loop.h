@@ -29,8 +29,6 @@ constexpr int kLoopWaves = GXT_LOOP_WAVES;  // per workgroup: kLoopWaves / 4 per
 constexpr int kLoopBlock = 64 * kLoopWaves;
 constexpr int kLP = 512;    // pages a workgroup holds at once, at most
 constexpr int kTake = 256;  // of which with tracks at its start, at most
-constexpr int kMinFree = 96;  // free pages per workgroup at its start, at least (one workgroup: what there is):
-                              // an open page for each type and what 12 running tasks may need
 
 // Shared state of a workgroup.  A page is known by its local number lp < kLP.
 // The waves work on it with LDS atomics and no lock: a lock around each of

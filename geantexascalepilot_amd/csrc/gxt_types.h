@@ -260,11 +260,15 @@ struct alignas(128) Rings {
   int parity;
   unsigned long long seg_lo, seg_hi;
   long long live;           // tracks in pages
+  unsigned int inj[2];      // photons, e-/e+ placed by an injection in progress
+  unsigned int inj_done;    // its workgroups that have ended
 };
 struct PageSeg {
   uint32_t first, count;    // entries [seg_lo + first, + count)
 };
 constexpr int kMaxGroups = 512;
+constexpr int kMinFree = 96;  // free pages per workgroup at its start, at least (one workgroup: what there is):
+                              // an open page for each type and what 12 running tasks may need
 
 enum StatKind { kStatSteps = 0, kStatStepsCharged, kStatKilled, kStatInteractions, kStatCreated, kStatLoaded0,
                 kStatLoaded1, kStatInteractions0, kStatCreated0,
