@@ -301,6 +301,13 @@ struct gxt_ctx {
   std::atomic<int> serve_rc{GXT_OK};  // first error of the serving thread
   std::mutex err_mu;                  // guards err (the serving thread writes it)
 
+  // Live tracks that are sure to find room.  Tracks wait in pages of one type
+  // each, so a workgroup's open pages, one per type, may hold a track each.  Where
+  // there are several workgroups these pages come on top of the capacity; in the
+  // pool of one they are part of it, so that the smallest pools go on refusing
+  // the showers that they refused when tracks had slots (10 GeV in 1024).
+  int64_t capacity() const { return groups == 1 ? cap - kTypes * kPageTracks : cap; }
+
   LoopArgs args() {
     LoopArgs a;
     a.P = dd.P;
@@ -338,6 +345,7 @@ struct gxt_ctx {
     // 1.5 ms 11.8; 10 e- of 50 GeV 4.5, at 2 ms 5.1; 0.7 ms: all the same, and so
     // are 2 ms where nothing waits and every workgroup has 512 tracks or more).
     a.ticks = 100000;
+    a.max_tracks = groups == 1 ? (int)capacity() : 0;
     a.prof = prof ? 1 : 0;
     return a;
   }
@@ -401,7 +409,7 @@ int alloc_events(gxt_ctx *c, int n) {
 // admitted whole (all primaries of an event together) and in order, so a job's
 // admitted primaries are contiguous.
 int admit(gxt_ctx *c) {
-  const double budget = 0.8 * (double)c->cap;
+  const double budget = 0.8 * (double)c->capacity();
   struct Range {
     const void *src;
     int n, photons, event_base;
@@ -1061,8 +1069,9 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
     c->lds_bytes = c->lds_tab_bytes + c->ev_slots * kEventSumBytes;
   }
   // pages, counters, tallies: pages for the capacity, and for each workgroup
-  // but one what it holds open or partly filled
-  const int64_t np = (c->cap + kPageTracks - 1) / kPageTracks + (int64_t)(c->groups - 1) * kMinFree;
+  // what it holds open or its tasks may need (but see capacity() for one)
+  const int64_t np = (c->cap + kPageTracks - 1) / kPageTracks + (int64_t)c->groups * kMinFree -
+                     (c->groups == 1 ? kTypes : 0);
   c->npages = (int)np;
   // (a launch reads a ring's entries while workgroups that have ended write
   // behind them: twice the pages)

@@ -42,6 +42,7 @@ struct LoopArgs {
   int ev_slots;      // events with sums in LDS
   int groups;        // workgroups launched (at most)
   int keep;          // workgroups keep their pages from launch to launch
+  int max_tracks;    // tracks the pool holds (one workgroup); 0: as many as find pages
   int ticks;         // 100 MHz ticks after which a workgroup starts no further task
   int prof;          // accumulate the time of the loop's parts (kStatTime*)
 };

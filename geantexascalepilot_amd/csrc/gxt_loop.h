@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <climits>
 
 #include "gxt_step.h"
 
@@ -50,13 +51,15 @@ constexpr int kTake = 256;  // of which with tracks at its start, at most
 //    compare-and-swap; cnt counts the tracks written into a page.
 constexpr uint16_t kNone16 = 0xffffu;
 constexpr uint32_t kNoEntry = 0xffffffffu;
+constexpr int kNoPages = 1, kFull = 2;  // Sched::stop: no free pages for the next task; more tracks than the pool holds
 struct Sched {
   int head[16], tail[16];  // tickets of the ready rings, by type
   int open[16];            // lp << 7 | entries given out (1 .. 63); -1: none
   int busy;                // running tasks, + 256 x tasks ended
   int avail;
   int ftop;                // tickets of the free stack
-  int stop;                // no further tasks
+  int stop;                // no further tasks, and why
+  int live, max_live;      // tracks made less those ended since the launch's start, and what they may be
   int ran;                 // a task has run
   unsigned int base[2];
   int cnt[kLP];
@@ -141,6 +144,7 @@ __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
     const bool over = wall_clock64() - t_end >= 0;
     const int busy = __builtin_amdgcn_readfirstlane(lds_ld(S.busy));
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    if (lds_ld(S.live) > lds_ld(S.max_live)) lds_st(S.stop, kFull);
     int key = -1, h = 0, o = -1;
     if (l < kTypes) {
       h = lds_ld(S.head[l]);
@@ -208,7 +212,7 @@ __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
         // workgroup hands its pages back
         wait = (busy & 255) != 0;
         if (!wait && __builtin_amdgcn_readfirstlane(lds_ld(S.busy)) == busy) {
-          if (l == 0) lds_st(S.stop, 1);
+          if (l == 0) lds_st(S.stop, kNoPages);
           return t;
         }
       }
@@ -273,10 +277,14 @@ __device__ __forceinline__ int reserve(Sched &S, const Task &task, int n) {
       slot_put(S.fs[lds_add(S.ftop, 1)], (uint32_t)pg);
     }
   }
-  // what the task did not take of its needs, and its own page
-  const int took = __builtin_amdgcn_readlane(row_incl_scan(np), kTypes - 1);
+  // what the task did not take of its needs, and its own page; the tracks it
+  // gives beyond its own
+  const int sum = __builtin_amdgcn_readlane(row_incl_scan(np | n << 8), kTypes - 1);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  if (l == 0) lds_add(S.avail, task.need + 1 - took);
+  if (l == 0) {
+    lds_add(S.avail, task.need + 1 - (sum & 255));
+    lds_add(S.live, (sum >> 8) - task.n);
+  }
   return f;
 }
 
@@ -969,8 +977,10 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
       S.stat[tid] = 0;
     }
     if (tid == 0) {
-      S.busy = S.stop = S.ran = 0;
+      S.busy = S.stop = S.ran = S.live = 0;
       S.ftop = S.avail = nf;
+      // (a pool of one workgroup: all tracks are here or in the list)
+      S.max_live = a.max_tracks ? a.max_tracks - (int)rg.live : INT_MAX;
     }
     for (int j = tid; j < kTypes * kLP; j += kLoopBlock) S.rq[j / kLP][j % kLP] = kNone16;
     for (int j = tid; j < kLP; j += kLoopBlock) S.fs[j] = kNoEntry;
@@ -1054,6 +1064,7 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
       my_seg = PageSeg{(uint32_t)lp, (uint32_t)np};
       S.base[1] = (uint32_t)(ftail + fp);
       if (S.ran) atomicAdd(&rg.ran, 1u);
+      if (S.stop == kFull) atomicOr(&a.cnt->overflow, 1);
     }
     __syncthreads();
     uint32_t at = S.base[0];

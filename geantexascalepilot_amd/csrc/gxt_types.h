@@ -267,8 +267,9 @@ struct PageSeg {
   uint32_t first, count;    // entries [seg_lo + first, + count)
 };
 constexpr int kMaxGroups = 512;
-constexpr int kMinFree = 96;  // free pages per workgroup at its start, at least (one workgroup: what there is):
-                              // an open page for each type and what 12 running tasks may need
+// Free pages per workgroup at its start, at least (one workgroup: what there is):
+// an open page for each type and what 12 running tasks may need.
+constexpr int kMinFree = 96;
 
 enum StatKind { kStatSteps = 0, kStatStepsCharged, kStatKilled, kStatInteractions, kStatCreated, kStatLoaded0,
                 kStatLoaded1, kStatInteractions0, kStatCreated0,

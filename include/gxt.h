@@ -91,7 +91,8 @@ typedef struct gxt_config {
   double rbin_mm;           /* radial tally bin (mm)                                */
   int32_t n_zbins;
   int32_t n_rbins;
-  int64_t pool_capacity;    /* live-track pool size (tracks)                        */
+  int64_t pool_capacity;    /* live tracks that find room (a pool below 8192: 704 fewer,
+                               the slots of part-filled pages); GXT_ECAPACITY beyond */
   int32_t max_steps;        /* per-track step limit (track killed beyond it)        */
   int32_t max_events;       /* per-event tally slots                                */
   int32_t max_jobs;         /* concurrent job slots                                 */

@@ -73,3 +73,12 @@ def test_one_event_of_both_species_classes_fills_the_pool(gpu_lib):
     assert gpu["leak"][0] >= e * (n // 1000) * (1 - 1e-9)
     assert abs((gpu["edep"][0] + gpu["leak"][0]) / (e * n) - 1.0) < 1e-9
     assert gpu["n_steps"][0] >= n - n // 1000
+
+
+# the smallest pools, of one workgroup: jobs of one event, up to the default
+# max_jobs and more, and jobs whose showers use most of what the pool holds
+@pytest.mark.parametrize("jobs,per,pool,ekin,mixed", [
+    (17, 1, 1024, 10.0, False), (64, 1, 1024, 10.0, False), (62, 1, 4096, 10.0, False), (200, 1, 4096, 10.0, False),
+    (1, 16, 1024, 300.0, True), (1, 31, 1024, 1000.0, True), (10, 30, 1024, 20.0, True), (2, 10, 1500, 2000.0, True)])
+def test_smallest_pools(gpu_lib, jobs, per, pool, ekin, mixed):
+    run_jobs(gpu_lib, jobs, per, pool, ekin, mixed)
