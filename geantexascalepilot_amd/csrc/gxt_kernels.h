@@ -24,7 +24,7 @@ struct LoopArgs {
   const DevParams *P;
   Counters *cnt;
   DevEvent *ev;
-  int *ev_live;      // live tracks of event slot e at ev_live[e * kLiveStride]
+  int *ev_live;      // live tracks of event slot e from ev_live[e * kLiveStride] on (kLive*)
   char *pages;       // npages pages of page_bytes<R>()
   uint32_t *list;    // ring of the pages with tracks, mask + 1 entries (Rings)
   uint32_t *freel;   // ring of the free pages, mask + 1 entries
@@ -93,12 +93,14 @@ hipError_t launch_pages_init(const LoopArgs &a, hipStream_t st);
 // What the host reads of the device's state after a launch.
 struct Snapshot {
   long long live;    // tracks in pages
+  long long peak;    // Rings::peak
   unsigned int ran;  // workgroups that ran a task in the last launch
   int overflow;
 };
 // The host's snapshot, into pinned host memory (device addresses out,
-// out_live): out_live[e] = ev_live[e * kLiveStride] for e < n.
-hipError_t launch_snapshot(const Counters *cnt, const int *ev_live, int n, Snapshot *out, int *out_live,
+// out_live, out_peak): each event's live tracks and the most that were live at
+// once (kLivePeak, which it brings up to date), e < n.
+hipError_t launch_snapshot(const Counters *cnt, int *ev_live, int n, Snapshot *out, int *out_live, int *out_peak,
                            hipStream_t st);
 hipError_t launch_rng_init(const DevParams *P, const uint32_t *seed, const uint64_t *idx, int n, uint32_t *out,
                            hipStream_t st);

@@ -88,7 +88,9 @@ __global__ __launch_bounds__(kBlock) void k_inject(LoopArgs a, InjectArgs in) {
       unsafeAtomicAdd(&a.ev[t.event].leak, p.ekin);
     } else {
       region = t.species == 0 ? 0 : 1;
-      atomicAdd(&a.ev_live[(int64_t)t.event * kLiveStride], 1);
+      int *live = a.ev_live + (int64_t)t.event * kLiveStride;
+      atomicAdd(&live[kLiveNow], 1);
+      atomicAdd(&live[kLiveGrow], 1);
     }
   }
 #pragma unroll
@@ -144,6 +146,7 @@ __global__ __launch_bounds__(kBlock) void k_inject(LoopArgs a, InjectArgs in) {
     rg.fhead = fhead + (unsigned long long)take;
     rg.ftail = ftail + (unsigned long long)(take - u0 - u1);
     rg.live += (long long)placed[0] + placed[1];
+    rg.peak = max(rg.peak, rg.live);
   }
 }
 
@@ -159,7 +162,7 @@ __global__ __launch_bounds__(kBlock) void k_pages_init(Counters *cnt, uint32_t *
     r.done = r.ran = r.ran_last = 0;
     r.parity = 0;
     r.seg_lo = r.seg_hi = 0;
-    r.live = 0;
+    r.live = r.net = r.grow = r.peak = 0;
     r.inj[0] = r.inj[1] = r.inj_done = 0;
   }
 }
@@ -443,22 +446,35 @@ hipError_t launch_pages_init(const LoopArgs &a, hipStream_t st) {
 }
 
 // The host's snapshot of the step loop, written straight into its pinned
-// buffers: the per-event live counts packed (ev_live[e * kLiveStride] at
-// out_live[e]), the tracks in pages, the overflow flag.
-__global__ void k_snapshot(const Counters *cnt, const int *ev_live, int n, Snapshot *out, int *out_live) {
+// buffers: the per-event live counts and bounds of their peaks packed, the tracks
+// in pages, the overflow flag.
+__global__ void k_snapshot(const Counters *cnt, int *ev_live, int n, Snapshot *out, int *out_live, int *out_peak) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) out_live[e] = ev_live[(int64_t)e * kLiveStride];
+  if (e < n) {
+    int *L = ev_live + (int64_t)e * kLiveStride;
+    const int live = L[kLiveNow], grow = L[kLiveGrow], before = L[kLiveBefore];
+    int peak = L[kLivePeak];
+    if (grow) {
+      peak = max(peak, before + grow);
+      L[kLivePeak] = peak;
+      L[kLiveGrow] = 0;
+    }
+    if (live != before) L[kLiveBefore] = live;
+    out_live[e] = live;
+    out_peak[e] = peak;
+  }
   if (e == 0) {
+    out->peak = cnt->rings.peak;
     out->live = cnt->rings.live;
     out->ran = cnt->rings.ran_last;
     out->overflow = cnt->overflow;
   }
 }
 
-hipError_t launch_snapshot(const Counters *cnt, const int *ev_live, int n, Snapshot *out, int *out_live,
+hipError_t launch_snapshot(const Counters *cnt, int *ev_live, int n, Snapshot *out, int *out_live, int *out_peak,
                            hipStream_t st) {
   const int grid = n > kBlock ? (n + kBlock - 1) / kBlock : 1;
-  hipLaunchKernelGGL(k_snapshot, dim3(grid), dim3(kBlock), 0, st, cnt, ev_live, n, out, out_live);
+  hipLaunchKernelGGL(k_snapshot, dim3(grid), dim3(kBlock), 0, st, cnt, ev_live, n, out, out_live, out_peak);
   return hipGetLastError();
 }
 

@@ -59,7 +59,8 @@ struct Sched {
   int avail;
   int ftop;                // tickets of the free stack
   int stop;                // no further tasks, and why
-  int live, max_live;      // tracks made less those ended since the launch's start, and what they may be
+  int live, top, max_live;  // tracks made less those ended since the launch's start, their largest number, the
+                            // number from which the pool is full
   int ran;                 // a task has run
   unsigned int base[2];
   int cnt[kLP];
@@ -129,6 +130,7 @@ __device__ __forceinline__ int task_need(int type, int n) {
 struct Task {
   int type, lp, n;  // type < 0: the wave ends
   int need;
+  int live;  // Sched::live with the task's tracks (lane 0, from reserve on)
 };
 
 // The next task of a wave: a ready page of the type that has most of them;
@@ -139,12 +141,11 @@ __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
   const int l = lane();
   Task t;
   t.type = -1;
-  t.lp = t.n = t.need = 0;
+  t.lp = t.n = t.need = t.live = 0;
   for (;;) {
     const bool over = wall_clock64() - t_end >= 0;
     const int busy = __builtin_amdgcn_readfirstlane(lds_ld(S.busy));
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    if (lds_ld(S.live) > lds_ld(S.max_live)) lds_st(S.stop, kFull);
     int key = -1, h = 0, o = -1;
     if (l < kTypes) {
       h = lds_ld(S.head[l]);
@@ -225,7 +226,7 @@ __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
 // Frees the task's page and gives out entries: lane t < kTypes asks for n
 // entries of type t and gets its first entry f; entry e of the type is slot
 // e % 64 of page S.dest[wave][t][e / 64].
-__device__ __forceinline__ int reserve(Sched &S, const Task &task, int n) {
+__device__ __forceinline__ int reserve(Sched &S, Task &task, int n) {
   const int l = lane();
   const int w = (int)(threadIdx.x >> 6);
   // the task's tracks have been read before the page may be written again
@@ -283,14 +284,15 @@ __device__ __forceinline__ int reserve(Sched &S, const Task &task, int n) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   if (l == 0) {
     lds_add(S.avail, task.need + 1 - (sum & 255));
-    lds_add(S.live, (sum >> 8) - task.n);
+    const int net = (sum >> 8) - task.n;
+    task.live = lds_add(S.live, net) + net;
   }
   return f;
 }
 
 // The wave's outputs are written: lane t's n entries of type t from entry f
 // on.  Pages that are now whole become ready; the task has ended.
-__device__ __forceinline__ void commit(Sched &S, int f, int n) {
+__device__ __forceinline__ void commit(Sched &S, const Task &task, int f, int n) {
   const int l = lane();
   const int w = (int)(threadIdx.x >> 6);
   // the tracks' stores before the other waves can see the pages
@@ -303,6 +305,10 @@ __device__ __forceinline__ void commit(Sched &S, int f, int n) {
       if (lds_add(S.cnt[pg], c) + c == kPageTracks)
         ring_put(S.rq[l][lds_add(S.tail[l], 1) & (kLP - 1)], pg | (kPageTracks - 1) << 9);
     }
+  }
+  if (l == 0) {
+    atomicMax(&S.top, task.live);
+    if (task.live > S.max_live) lds_st(S.stop, kFull);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   if (l == 0) lds_add(S.busy, 256 - 1);
@@ -324,7 +330,8 @@ struct EventSum {
   unsigned long long nsteps;
   int tag;  // event slot, -1: none
   int live;
-  unsigned int nsec[3], npairs, nannihil, pad;
+  unsigned int nsec[3], npairs, nannihil;
+  int grow;  // largest `live` in this launch
 };
 static_assert(sizeof(EventSum) == kEventSumBytes, "LDS of the event sums");
 struct EventSums {
@@ -364,7 +371,10 @@ __device__ __forceinline__ void event_add(const LoopArgs &a, const EventSums &S,
     if (c.leak != 0.0) unsafeAtomicAdd(&E.leak, c.leak);
     if (c.clen != 0.0) unsafeAtomicAdd(&E.clen, c.clen);
     if (c.nsteps) atomicAdd(&E.nsteps, (unsigned long long)c.nsteps);
-    if (c.live) atomicAdd(&E.live, c.live);
+    if (c.live > 0)
+      atomicMax(&E.grow, atomicAdd(&E.live, c.live) + c.live);
+    else if (c.live)
+      atomicAdd(&E.live, c.live);
     if (c.nsec0) atomicAdd(&E.nsec[0], c.nsec0);
     if (c.nsec1) atomicAdd(&E.nsec[1], c.nsec1);
     if (c.nsec2) atomicAdd(&E.nsec[2], c.nsec2);
@@ -377,7 +387,9 @@ __device__ __forceinline__ void event_add(const LoopArgs &a, const EventSums &S,
     if (c.leak != 0.0) unsafeAtomicAdd(&E.leak, c.leak);
     if (c.clen != 0.0) unsafeAtomicAdd(&E.clen, c.clen);
     if (c.nsteps) atomicAdd(&E.nsteps, (unsigned long long)c.nsteps);
-    if (c.live) atomicAdd(&a.ev_live[(int64_t)event * kLiveStride], c.live);
+    int *live = a.ev_live + (int64_t)event * kLiveStride;
+    if (c.live) atomicAdd(&live[kLiveNow], c.live);
+    if (c.live > 0) atomicAdd(&live[kLiveGrow], c.live);
     if (c.nsec0) atomicAdd(&E.nsec[0], (unsigned long long)c.nsec0);
     if (c.nsec1) atomicAdd(&E.nsec[1], (unsigned long long)c.nsec1);
     if (c.nsec2) atomicAdd(&E.nsec[2], (unsigned long long)c.nsec2);
@@ -394,6 +406,7 @@ __device__ __forceinline__ void events_clear(const EventSums &S) {
     E.tag = -1;
     E.live = 0;
     E.nsec[0] = E.nsec[1] = E.nsec[2] = E.npairs = E.nannihil = 0;
+    E.grow = 0;
   }
 }
 
@@ -409,7 +422,9 @@ __device__ __forceinline__ void events_flush(const LoopArgs &a, const EventSums 
     if (L.leak != 0.0) unsafeAtomicAdd(&E.leak, L.leak);
     if (L.clen != 0.0) unsafeAtomicAdd(&E.clen, L.clen);
     if (L.nsteps) atomicAdd(&E.nsteps, L.nsteps);
-    if (L.live) atomicAdd(&a.ev_live[(int64_t)event * kLiveStride], L.live);
+    int *live = a.ev_live + (int64_t)event * kLiveStride;
+    if (L.live) atomicAdd(&live[kLiveNow], L.live);
+    if (L.grow) atomicAdd(&live[kLiveGrow], L.grow);
     for (int k = 0; k < 3; ++k)
       if (L.nsec[k]) atomicAdd(&E.nsec[k], (unsigned long long)L.nsec[k]);
     if (L.npairs) atomicAdd(&E.npairs, (unsigned long long)L.npairs);
@@ -486,7 +501,7 @@ constexpr int kPhotonSteps = 8;  // most steps of a photon in one task
 // kMode as LoopArgs::mode.
 template <class R, bool kCharged, int kMode, class NS>
 __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParams *P, const NS &N, Sched &S,
-                                               Hist &wh, const EventSums &ES, const Task &task) {
+                                               Hist &wh, const EventSums &ES, Task &task) {
   const bool trace = P->trace_events > 0;
   const R mine = (R)P->tracking_cut;
   constexpr int kG = kMode == 4 ? 1 : 0;  // geo_cell form
@@ -650,7 +665,7 @@ __device__ __forceinline__ void transport_task(const LoopArgs &a, const DevParam
     store_track(p, t, trace);
     if (trace && q >= 0 && q != kQueueAtRest) p.f64(kPtedep) = edep;
   }
-  commit(S, f, n);
+  commit(S, task, f, n);
   if (killed) atomicAdd(&S.stat[kStatKilled], 1ULL);
   if (dies) {
     add.nsteps = t.nsteps;
@@ -693,7 +708,7 @@ __device__ __forceinline__ int sec_fate(const DevParams *P, const TrackRegs<R> &
 template <class R, class NS>
 __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams *P, const NS &N,
                                               const uint32_t *jump, Sched &S, Hist &wh, const EventSums &ES,
-                                              const Task &task, long long &t_derive) {
+                                              Task &task, long long &t_derive) {
   const bool trace = P->trace_events > 0;
   const R mine = (R)P->tracking_cut;
   const int q = task.type - 2;
@@ -809,7 +824,7 @@ __device__ __forceinline__ void interact_task(const LoopArgs &a, const DevParams
     const int pg = S.dest[w][t.species == 0 ? 0 : 1][idx >> 6];
     store_track(PageSlot<R>(page_at<R>(a, S, pg), idx & 63), t, trace);
   }
-  commit(S, f, n);
+  commit(S, task, f, n);
   if (a.prof) t_derive += wall_clock64() - t0;
   if (active) {
     dp.flush(wh, P->geo.nvol > 1);
@@ -977,7 +992,7 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
       S.stat[tid] = 0;
     }
     if (tid == 0) {
-      S.busy = S.stop = S.ran = S.live = 0;
+      S.busy = S.stop = S.ran = S.live = S.top = 0;
       S.ftop = S.avail = nf;
       // (a pool of one workgroup: all tracks are here or in the list)
       S.max_live = a.max_tracks ? a.max_tracks - (int)rg.live : INT_MAX;
@@ -986,7 +1001,6 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     for (int j = tid; j < kLP; j += kLoopBlock) S.fs[j] = kNoEntry;
     __syncthreads();
     // local pages: [0, nt) with tracks, [nt, nt + nf) free
-    int start_live = 0;
     for (int j = tid; j < nt + nf; j += kLoopBlock) {
       if (j < nt) {
         const unsigned long long at = by_rank ? lhead + (unsigned)b + (unsigned long long)groups * j
@@ -995,7 +1009,6 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
         const int type = (int)(en >> 6 & 15u), n = (int)(en & 63u) + 1;
         S.gpage[j] = en >> 10;
         S.cnt[j] = n;
-        start_live += n;
         // the first partial page of a type is filled further, the others are
         // tasks as they are
         if (n == kPageTracks || !lds_cas(S.open[type], -1, j << 7 | n))
@@ -1035,7 +1048,7 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
           return P->jump8;
       }();
       for (;;) {
-        const Task task = next_task(S, t_end);
+        Task task = next_task(S, t_end);
         if (task.type < 0) break;
         const long long t0 = a.prof ? wall_clock64() : 0;
         long long td = 0;
@@ -1064,33 +1077,28 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
       my_seg = PageSeg{(uint32_t)lp, (uint32_t)np};
       S.base[1] = (uint32_t)(ftail + fp);
       if (S.ran) atomicAdd(&rg.ran, 1u);
+      if (S.live) atomicAdd((unsigned long long *)&rg.net, (unsigned long long)(long long)S.live);
+      if (S.top) atomicAdd((unsigned long long *)&rg.grow, (unsigned long long)S.top);
       if (S.stop == kFull) atomicOr(&a.cnt->overflow, 1);
     }
     __syncthreads();
     uint32_t at = S.base[0];
-    int live = -start_live;
     for (int t = 0; t < kTypes; ++t) {
       const int h = S.head[t], n = S.tail[t] - h;
       for (int j = tid; j < n; j += kLoopBlock) {
         const int v = S.rq[t][(h + j) & (kLP - 1)];
         const int c = (v >> 9) + 1;
         a.list[(at + (uint32_t)j) & a.mask] = page_entry(S.gpage[v & (kLP - 1)], t, c);
-        live += c;
       }
       at += (uint32_t)n;
       const int o = S.open[t];
       if (o >= 0) {
-        if (tid == 0) {
-          a.list[at & a.mask] = page_entry(S.gpage[o >> 7], t, o & 127);
-          live += o & 127;
-        }
+        if (tid == 0) a.list[at & a.mask] = page_entry(S.gpage[o >> 7], t, o & 127);
         ++at;
       }
     }
     for (int j = tid; j < nfree; j += kLoopBlock)
       a.freel[(S.base[1] + (uint32_t)j) & a.mask] = S.gpage[S.fs[j]];
-    live = __builtin_amdgcn_readlane(wave_incl_scan(live), 63);
-    if (lane() == 0 && live != 0) atomicAdd((unsigned long long *)&rg.live, (unsigned long long)(long long)live);
     hist_flush(a.rows, a.P, wh);
     events_flush(a, ES);
     if (tid < kNumStats && S.stat[tid]) atomicAdd(&a.cnt->stat[b % kStripes][tid], S.stat[tid]);
@@ -1109,6 +1117,10 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     rg.fhead = fhead + (unsigned long long)groups * nf;
     rg.ftail = ftail + fp;
     rg.ran_last = atomicExch(&rg.ran, 0u);
+    const long long net = (long long)atomicExch((unsigned long long *)&rg.net, 0ULL);
+    const long long grow = (long long)atomicExch((unsigned long long *)&rg.grow, 0ULL);
+    rg.peak = max(rg.peak, rg.live + grow);
+    rg.live += net;
     rg.done = 0;
   }
 }

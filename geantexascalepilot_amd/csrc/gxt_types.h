@@ -259,7 +259,9 @@ struct alignas(128) Rings {
   unsigned int ran, ran_last;  // workgroups that ran a task in this launch, in the last one
   int parity;
   unsigned long long seg_lo, seg_hi;
-  long long live;           // tracks in pages
+  long long live;           // tracks in pages when the last launch ended
+  long long net, grow;      // tracks made less those ended in this launch; sum of the workgroups' largest growths
+  long long peak;           // most tracks that may have been live at once
   unsigned int inj[2];      // photons, e-/e+ placed by an injection in progress
   unsigned int inj_done;    // its workgroups that have ended
 };
@@ -288,10 +290,18 @@ struct alignas(256) Counters {
   }
 };
 
-// Live-track count of event e at ev_live[e * kLiveStride]: one 128-byte line
-// per event, so the +/- 1 atomics of one event's tracks never queue behind
-// another event's.
+// Live tracks of event e: kLive.. at ev_live[e * kLiveStride + ..], one 128-byte
+// line per event, so the atomics of one event's tracks never queue behind another
+// event's.  Its live count exists only when a launch ends, and an event may grow,
+// shrink and end in between; so each workgroup gives, beside the change, the
+// largest growth that it saw, and the sum of those on top of the count before
+// bounds what was live at once (exact for an event in one workgroup).  The growths
+// cost 10,000 e- of 10 GeV 1 % (FP32 34.0 -> 34.4 ms).
 constexpr int kLiveStride = 32;
+enum { kLiveNow = 0,
+       kLiveGrow,    // sum of the growths since the last snapshot
+       kLiveBefore,  // count at the last snapshot
+       kLivePeak };  // largest bound until the last snapshot
 
 // Per-event tallies on the device (FP64, atomics), one or more whole 128-byte
 // lines per event for the same reason.

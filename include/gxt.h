@@ -154,7 +154,8 @@ typedef struct gxt_event_tally {
 typedef struct gxt_stats {
   int64_t track_steps;      /* total track-steps                       */
   int64_t iterations;       /* launches of the step loop               */
-  int64_t max_live;         /* peak live tracks                        */
+  int64_t max_live;         /* peak live tracks: a bound, as the workgroups' peaks within
+                               a launch are added up                   */
   int64_t killed_by_limit;  /* tracks killed by max_steps              */
   double wall_ms;           /* device time of the last gxt_run          */
 } gxt_stats;
