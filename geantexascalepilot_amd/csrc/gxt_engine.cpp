@@ -13,6 +13,7 @@
 #include <array>
 #include <atomic>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <condition_variable>
 #include <cstring>
@@ -228,6 +229,10 @@ struct Job {
 
 }  // namespace
 
+// An iteration of gxt_run: transports of a track.
+constexpr int kIterTransports = 4;
+constexpr long long kOnceBelow = 65536;
+
 struct gxt_ctx {
   gxt_config cfg{};
   std::string data_dir;
@@ -293,6 +298,7 @@ struct gxt_ctx {
   gxt_kernel_stats kst{};
   // stats
   int64_t iterations = 0;
+  long long iter_end = LLONG_MAX;  // LoopArgs
   int64_t max_live = 0;
   double wall_ms = 0;
   std::chrono::steady_clock::time_point t0;
@@ -348,6 +354,11 @@ struct gxt_ctx {
     // are 2 ms where nothing waits and every workgroup has 512 tracks or more).
     a.ticks = 100000;
     a.max_tracks = groups == 1 ? (int)capacity() : 0;
+    // A run of limited iterations: launches of one transport of each track
+    // (kOnceBelow of them at most), before that launches of 1 ms, which count as
+    // the tasks of their busiest workgroup: a few hundred.
+    a.iter_end = iter_end;
+    a.once = iter_end != LLONG_MAX && iter_end - hsnap->iters < kOnceBelow;
     a.prof = prof ? 1 : 0;
     return a;
   }
@@ -544,8 +555,9 @@ int collect(gxt_ctx *c, bool &idle) {
   c->ev_snap = 0;
   const Snapshot &h = *c->hsnap;
   const int64_t live = h.live;
-  // a launch that found tracks but no page to run a task with will not get further
-  if (h.overflow || (live > 0 && c->snap_iter > 0 && h.ran == 0))
+  // a launch that found tracks but no page to run a task with will not get
+  // further (one that found no iterations left may)
+  if (h.overflow || (live > 0 && c->snap_iter > 0 && h.ran == 0 && h.iters < c->iter_end))
     return c->fail(GXT_ECAPACITY, "track pool overflow (increase pool_capacity)");
   c->max_live = std::max<int64_t>(c->max_live, h.peak);
   std::vector<Job *> fin;
@@ -1215,17 +1227,22 @@ int gxt_submit_tracks(gxt_ctx *c, const gxt_track *trk, int n, int n_events, uin
 int gxt_run(gxt_ctx *c, int64_t max_iterations) {
   if (!c) return set_err(GXT_EINVAL, "null context");
   if (c->serving.load()) return c->fail(GXT_ESTATE, "gxt_run while serving");
+  c->iter_end = LLONG_MAX;
+  if (max_iterations > 0 && max_iterations < (int64_t)1 << 60) {
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    HIP_TRY(hipMemcpy(&c->hsnap->iters, &c->cnt->rings.iters, sizeof(c->hsnap->iters), hipMemcpyDeviceToHost));
+    c->iter_end = c->hsnap->iters + kIterTransports * max_iterations;
+  }
   hipEvent_t e0, e1;
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
   HIP_TRY(hipEventRecord(e0, c->stream));
-  const int64_t start = c->iterations;
   int rc = GXT_OK;
   for (;;) {
     bool idle = false;
     rc = round_trip(c, idle);
     if (rc || idle) break;
-    if (max_iterations > 0 && c->iterations - start >= max_iterations) break;
+    if (c->hsnap->iters >= c->iter_end) break;
   }
   (void)hipEventRecord(e1, c->stream);
   (void)hipEventSynchronize(e1);
@@ -1404,6 +1421,7 @@ int gxt_serve_start(gxt_ctx *c) {
   if (c->serving.load()) return c->fail(GXT_ESTATE, "already serving");
   c->stop = false;
   c->serve_rc = GXT_OK;
+  c->iter_end = LLONG_MAX;
   c->serving = true;
   c->server = std::thread(serve_loop, c);
   return GXT_OK;

@@ -43,6 +43,8 @@ struct LoopArgs {
   int groups;        // workgroups launched (at most)
   int keep;          // workgroups keep their pages from launch to launch
   int max_tracks;    // tracks the pool holds (one workgroup); 0: as many as find pages
+  int once;          // transport each track once at most
+  long long iter_end;  // Rings::iters from which no task runs; LLONG_MAX: no limit
   int ticks;         // 100 MHz ticks after which a workgroup starts no further task
   int prof;          // accumulate the time of the loop's parts (kStatTime*)
 };
@@ -94,6 +96,7 @@ hipError_t launch_pages_init(const LoopArgs &a, hipStream_t st);
 struct Snapshot {
   long long live;    // tracks in pages
   long long peak;    // Rings::peak
+  long long iters;   // Rings::iters
   unsigned int ran;  // workgroups that ran a task in the last launch
   int overflow;
 };

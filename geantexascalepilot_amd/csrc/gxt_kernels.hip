@@ -163,6 +163,7 @@ __global__ __launch_bounds__(kBlock) void k_pages_init(Counters *cnt, uint32_t *
     r.parity = 0;
     r.seg_lo = r.seg_hi = 0;
     r.live = r.net = r.grow = r.peak = 0;
+    r.iters = r.launch_iters = 0;
     r.inj[0] = r.inj[1] = r.inj_done = 0;
   }
 }
@@ -465,6 +466,7 @@ __global__ void k_snapshot(const Counters *cnt, int *ev_live, int n, Snapshot *o
   }
   if (e == 0) {
     out->peak = cnt->rings.peak;
+    out->iters = cnt->rings.iters;
     out->live = cnt->rings.live;
     out->ran = cnt->rings.ran_last;
     out->overflow = cnt->overflow;

@@ -51,10 +51,13 @@ constexpr int kTake = 256;  // of which with tracks at its start, at most
 //    compare-and-swap; cnt counts the tracks written into a page.
 constexpr uint16_t kNone16 = 0xffffu;
 constexpr uint32_t kNoEntry = 0xffffffffu;
-constexpr int kNoPages = 1, kFull = 2;  // Sched::stop: no free pages for the next task; more tracks than the pool holds
+// Sched::stop: no free pages for the next task; more tracks than the pool holds;
+// no iterations left.
+constexpr int kNoPages = 1, kFull = 2, kNoIters = 3;
 struct Sched {
   int head[16], tail[16];  // tickets of the ready rings, by type
   int open[16];            // lp << 7 | entries given out (1 .. 63); -1: none
+  int until[16];           // tickets below are tasks of this launch; INT_MAX: all, and open pages
   int busy;                // running tasks, + 256 x tasks ended
   int avail;
   int ftop;                // tickets of the free stack
@@ -136,7 +139,8 @@ struct Task {
 // The next task of a wave: a ready page of the type that has most of them;
 // with none ready, the fullest open page that no wave is writing to; with
 // neither and no task running, or after the launch's time, none.  While other
-// waves run tasks the wave waits for one to end or begin.
+// waves run tasks the wave waits for one to end or begin.  (A launch of one
+// iteration transports only the pages that it began with, Sched::until.)
 __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
   const int l = lane();
   Task t;
@@ -149,11 +153,12 @@ __device__ __forceinline__ Task next_task(Sched &S, long long t_end) {
     int key = -1, h = 0, o = -1;
     if (l < kTypes) {
       h = lds_ld(S.head[l]);
-      const int r = lds_ld(S.tail[l]) - h;
+      const int until = lds_ld(S.until[l]);
+      const int r = min(lds_ld(S.tail[l]), until) - h;
       o = lds_ld(S.open[l]);
       if (r > 0)
         key = (1 << 16) | (r << 4) | l;
-      else if (o >= 0 && lds_ld(S.cnt[o >> 7]) == (o & 127))
+      else if (o >= 0 && until == INT_MAX && lds_ld(S.cnt[o >> 7]) == (o & 127))
         key = ((o & 127) << 4) | l;
     }
     key = row0_max(key);
@@ -969,6 +974,8 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     nt = sh.nt;
     at_free = sh.rank;
   }
+  // iterations left to a run that counts them
+  const bool none_left = rg.iters >= a.iter_end;
   const int nf = have > 0 ? (int)min(spare / groups, (long long)(kLP - kTake)) : 0;
   PageSeg my_seg = {0u, 0u};
   if (nt > 0) {
@@ -989,6 +996,7 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     if (tid < 16) {
       S.head[tid] = S.tail[tid] = 0;
       S.open[tid] = -1;
+      S.until[tid] = INT_MAX;
       S.stat[tid] = 0;
     }
     if (tid == 0) {
@@ -1009,9 +1017,9 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
         const int type = (int)(en >> 6 & 15u), n = (int)(en & 63u) + 1;
         S.gpage[j] = en >> 10;
         S.cnt[j] = n;
-        // the first partial page of a type is filled further, the others are
-        // tasks as they are
-        if (n == kPageTracks || !lds_cas(S.open[type], -1, j << 7 | n))
+        // the first partial page of a type is filled further (not with tracks that
+        // the launch is not to transport again), the others are tasks as they are
+        if (n == kPageTracks || (a.once && type < 2) || !lds_cas(S.open[type], -1, j << 7 | n))
           S.rq[type][lds_add(S.tail[type], 1)] = (uint16_t)(j | (n - 1) << 9);
       } else {
         S.gpage[j] = a.freel[(uint32_t)(fhead + (unsigned long long)at_free * nf + (j - nt)) & a.mask];
@@ -1020,6 +1028,8 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     }
     __syncthreads();
     events_clear(ES);
+    if (a.once && tid < 2) S.until[tid] = S.tail[tid];
+    if (none_left && tid == 0) S.stop = kNoIters;
     __syncthreads();
     {
       const DevParams *P = &sP;
@@ -1076,7 +1086,11 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
       S.base[0] = (uint32_t)(ltail + lp);
       my_seg = PageSeg{(uint32_t)lp, (uint32_t)np};
       S.base[1] = (uint32_t)(ftail + fp);
-      if (S.ran) atomicAdd(&rg.ran, 1u);
+      if (S.ran) {
+        atomicAdd(&rg.ran, 1u);
+        // (no track's chain of tasks is longer than all the workgroup's)
+        atomicMax(&rg.launch_iters, a.once ? 1 : S.busy >> 8);
+      }
       if (S.live) atomicAdd((unsigned long long *)&rg.net, (unsigned long long)(long long)S.live);
       if (S.top) atomicAdd((unsigned long long *)&rg.grow, (unsigned long long)S.top);
       if (S.stop == kFull) atomicOr(&a.cnt->overflow, 1);
@@ -1121,6 +1135,7 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
     const long long grow = (long long)atomicExch((unsigned long long *)&rg.grow, 0ULL);
     rg.peak = max(rg.peak, rg.live + grow);
     rg.live += net;
+    rg.iters += atomicExch(&rg.launch_iters, 0);
     rg.done = 0;
   }
 }

@@ -262,6 +262,8 @@ struct alignas(128) Rings {
   long long live;           // tracks in pages when the last launch ended
   long long net, grow;      // tracks made less those ended in this launch; sum of the workgroups' largest growths
   long long peak;           // most tracks that may have been live at once
+  long long iters;          // transports of any track so far, at most
+  int launch_iters;         // the same of this launch
   unsigned int inj[2];      // photons, e-/e+ placed by an injection in progress
   unsigned int inj_done;    // its workgroups that have ended
 };

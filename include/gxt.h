@@ -153,7 +153,7 @@ typedef struct gxt_event_tally {
 /* Run statistics. */
 typedef struct gxt_stats {
   int64_t track_steps;      /* total track-steps                       */
-  int64_t iterations;       /* launches of the step loop               */
+  int64_t iterations;       /* launches of the step loop (up to 1 ms)  */
   int64_t max_live;         /* peak live tracks: a bound, as the workgroups' peaks within
                                a launch are added up                   */
   int64_t killed_by_limit;  /* tracks killed by max_steps              */
@@ -295,8 +295,9 @@ typedef struct gxt_track {
  * that holds the position) before anything is queued.  No reference
  * counterpart beyond the hand-off point cited above. */
 int gxt_submit_tracks(gxt_ctx *ctx, const gxt_track *tracks, int n, int n_events, uint64_t job_id);
-/* Run the step loop until every submitted job has finished, in launches of
- * about a millisecond, at most max_iterations of them and one more (replaces
+/* Run the step loop until every submitted job has finished, or for
+ * max_iterations iterations: in each a track goes through at most four transports
+ * (a step, or up to 8 of a photon), with the interactions that follow (replaces
  * ProxyDeviceManager::DoStep/DoGPIL, ProxyDeviceManager.cpp:206-276, and the
  * host wave loop DoStep<>, proxy/test/test_BasicCpuTransport.cpp:517-550).
  * max_iterations <= 0 means no limit. */
