@@ -278,9 +278,12 @@ def tracks_array(n):
 
 
 def tallies_to_numpy(t):
-    """Event tallies (EventTally array) as one numpy array per field, copied out of
-    the array in one pass per field (a loop over events and fields took 1 us per
-    value, 10 ms for 10,000 events beside the 58 ms of their transport)."""
+    """Event tallies (an EventTally array, or any sequence of them, as a slice of the
+    array is) as one numpy array per field, copied out of the array in one pass per
+    field (a loop over events and fields took 1 us per value, 10 ms for 10,000
+    events beside the 39 ms of their transport)."""
+    if not isinstance(t, C.Array):
+        t = (EventTally * len(t))(*t)
     a = np.frombuffer(t, dtype=np.dtype(EventTally), count=len(t))
     return {k: np.array(a[k]) for k in ("edep", "visible", "leak", "charged_length", "n_secondaries", "n_steps",
                                         "n_pairs", "n_annihil")}
