@@ -1099,6 +1099,8 @@ int gxt_create(const gxt_config *cfg, gxt_ctx **out) {
     while (c->ev_slots < kMaxEvSlots && c->lds_tab_bytes + 2 * c->ev_slots * kEventSumBytes <= all) c->ev_slots *= 2;
     c->lds_bytes = c->lds_tab_bytes + c->ev_slots * kEventSumBytes;
   }
+  HIP_TRY(c->precision == GXT_FP32 ? prepare_loop<float>(c->transport_mode, c->lds_tables)
+                                   : prepare_loop<double>(c->transport_mode, c->lds_tables));
   // pages, counters, tallies: pages for the capacity, and for each workgroup
   // what it holds open or its tasks may need (but see capacity() for one)
   const int64_t np = (c->cap + kPageTracks - 1) / kPageTracks + (int64_t)c->groups * kMinFree -

@@ -63,13 +63,21 @@ struct SampleArgs {
   double *sec_dir;
 };
 
-// One launch of the step loop (gxt_loop.h) on a.groups workgroups.  e0, e1 (may
-// be null) take the kernel's start and end.
 // LDS of a launch beside its tables and event sums, and all of a workgroup's.
 constexpr int kLoopLdsFixed = 31 * 1024;
 constexpr int kEventSumBytes = 72;
 constexpr int kMinEvSlots = 128, kMaxEvSlots = 512;
 constexpr int kLoopLds = 160 * 1024;
+// Raises the LDS limit of the loop of a mode (LoopArgs::mode, lds_tables) on the
+// current device, where its launches need it: once for every context, on the
+// device of its stream, as launches may come from threads with another current
+// device.
+template <class R>
+hipError_t prepare_loop(int mode, int lds_tables);
+template <class R, int kMode>
+hipError_t prepare_loop_mode(int lds_tables);
+// One launch of the step loop (gxt_loop.h) on a.groups workgroups.  e0, e1 (may
+// be null) take the kernel's start and end.
 template <class R>
 hipError_t launch_loop(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1);
 // The launch of one transport mode (each mode is compiled in a unit of its own).

@@ -425,6 +425,18 @@ hipError_t launch_loop(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEven
     default: return launch_loop_mode<R, 4>(a, st, e0, e1);
   }
 }
+template <class R>
+hipError_t prepare_loop(int mode, int lds_tables) {
+  switch (mode) {
+    case 0: return prepare_loop_mode<R, 0>(lds_tables);
+    case 1: return prepare_loop_mode<R, 1>(lds_tables);
+    case 2: return prepare_loop_mode<R, 2>(lds_tables);
+    case 3: return prepare_loop_mode<R, 3>(lds_tables);
+    default: return prepare_loop_mode<R, 4>(lds_tables);
+  }
+}
+template hipError_t prepare_loop<double>(int, int);
+template hipError_t prepare_loop<float>(int, int);
 template hipError_t launch_loop<double>(const LoopArgs &, hipStream_t, hipEvent_t, hipEvent_t);
 template hipError_t launch_loop<float>(const LoopArgs &, hipStream_t, hipEvent_t, hipEvent_t);
 

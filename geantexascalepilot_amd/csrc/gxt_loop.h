@@ -19,7 +19,6 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
-#include <atomic>
 #include <climits>
 
 #include "gxt_step.h"
@@ -1143,18 +1142,6 @@ __global__ __launch_bounds__(kLoopBlock, kLoopWaves / 4) void k_loop(LoopArgs a)
 template <class R, int kMode, int kLds>
 static hipError_t launch_one(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
   auto kernel = k_loop<R, kMode, kLds>;
-  // once per device: a kernel's LDS limit belongs to its module there
-  static std::atomic<uint64_t> raised{0};
-  int dev = 0;
-  hipError_t rc = hipGetDevice(&dev);
-  if (rc != hipSuccess) return rc;
-  const uint64_t bit = 1ULL << (dev & 63);
-  if (dev > 63 || !(raised.load(std::memory_order_relaxed) & bit)) {
-    rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                             kLoopLds - kLoopLdsFixed);
-    if (rc != hipSuccess) return rc;
-    raised.fetch_or(bit, std::memory_order_relaxed);
-  }
   if (e0 || e1)
     hipExtLaunchKernelGGL(kernel, dim3(a.groups), dim3(kLoopBlock), (uint32_t)a.lds_bytes, st, e0, e1, 0, a);
   else
@@ -1169,6 +1156,15 @@ hipError_t launch_loop_mode(const LoopArgs &a, hipStream_t st, hipEvent_t e0, hi
     case kLdsPhotons: return launch_one<R, kMode, kLdsPhotons>(a, st, e0, e1);
     default: return launch_one<R, kMode, kLdsNone>(a, st, e0, e1);
   }
+}
+
+template <class R, int kMode>
+hipError_t prepare_loop_mode(int lds_tables) {
+  auto kernel = lds_tables == kLdsAll ? k_loop<R, kMode, kLdsAll>
+                                      : (lds_tables == kLdsPhotons ? k_loop<R, kMode, kLdsPhotons>
+                                                                   : k_loop<R, kMode, kLdsNone>);
+  return hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                             kLoopLds - kLoopLdsFixed);
 }
 
 }  // namespace gxt
