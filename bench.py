@@ -42,6 +42,18 @@ def profiled_traffic(kernel, summary="hbm_traffic_c1_fp64.md"):
     return float(m.group(1)) if m else None
 
 
+def profiled_issue(summary="counters_c1_fp64.md"):
+    """Percent of the SIMDs' cycles in which a vector instruction issues, from the
+    committed rocprofv3 counter summary of the headline batch; None without it."""
+    import re
+    try:
+        text = open(os.path.join(ROOT, "profiles", summary)).read()
+    except OSError:
+        return None
+    m = re.search(r"^\| VALU issue per SIMD [^|]*\|\s*([0-9.]+) %", text, re.M)
+    return float(m.group(1)) if m else None
+
+
 def log(msg):
     sys.stderr.write("[bench] %s\n" % msg)
     sys.stderr.flush()
@@ -74,7 +86,7 @@ def run_batch(g, abi, precision, n_events, steps, warmup, seed=777, pool=2_000_0
         ks = t.kernel_stats()
         st = t.stats()
         edep = t.event_tallies(job - 1, n_events)
-    log("timed %d batches in %.3f s (precision %d): %d iterations, peak %d live tracks"
+    log("timed %d batches in %.3f s (precision %d): %d launches, peak %d live tracks"
         % (steps, elapsed, precision, st.iterations, st.max_live))
     return dict(seconds=elapsed, ks=ks, stats=st, edep=edep)
 
@@ -141,8 +153,8 @@ def field_forms(g, abi, n_events=20000, seed=2468, cpu=False):
             ev = t.event_tallies(1, n_events)
             st = t.stats()
             ks = t.kernel_stats()
-        # the e-/e+ transport against the HBM roofline: 2 x 148 B per e-/e+
-        # step over its part of the launches' time
+        # the e-/e+ transport against the HBM roofline, as a model: 2 x 148 B per
+        # e-/e+ step over its part of the launches' time
         gbs = 2 * 148 * ks.charged_steps / max(ks.transport_charged_ms * 1e-3, 1e-12) / 1e9
         out[name] = dict(events_per_s=n_events / dt, seconds=dt, track_steps=int(st.track_steps),
                          ns_per_track_step=1e9 * dt / max(int(st.track_steps), 1),
@@ -353,9 +365,9 @@ def serving(g, abi, seconds, rate_jobs_s, mix="c4", warm_s=2.0, drain_s=60.0, se
     lat = np.array([r.done_ms - r.submit_ms for r in late]) if late else np.zeros(1)
     single = np.array([r.done_ms - r.submit_ms for r in late if kinds[r.job_id] == "gamma1"])
     backlog = sum(1 for j in range(submitted) if sub_t[j] <= t_window) - sum(1 for tc, _ in done if tc <= t_window)
-    # a job's latency over the step-loop iterations it spent in flight: the
-    # host finds a finished job at the next counter snapshot, at most one
-    # round (4-8 iterations) after its last track died
+    # a job's latency over the step-loop launches it spent in flight: the host
+    # finds a finished job at the next counter snapshot, at most one round (two
+    # launches) after its last track died
     its = np.array([max(r.iterations, 1) for r in late]) if late else np.ones(1)
     ms_per_it = float(np.median(lat / its))
     single_its = np.array([r.iterations for r in late if kinds[r.job_id] == "gamma1"])
@@ -548,13 +560,16 @@ def main():
     value = a.steps * n / r64["seconds"]
     ks = r64["ks"]
     steps_per_s = ks.track_steps / r64["seconds"]
-    # Algorithmic bytes of the step loop's kernel: one read and one write of a
-    # track record (116 B in the FP64 form: position 24, direction 24, energy 8,
-    # 3 interaction lengths 24, RNG 24, event, volume|species, step count 4
-    # each) for every track a transport or an interaction task loads, and one
-    # write for every track created.  (The per-track-step figure of 2 x 148 B,
-    # a nominal record with inverse mean free paths and safety, is reported
-    # beside it.)
+    # What bounds the step loop's kernel is the issue of vector instructions: the
+    # share of the SIMDs' cycles in which one issues, from the committed counter
+    # summary of this workload.  Beside it the HBM traffic, from the committed
+    # FETCH_SIZE / WRITE_SIZE summary over this run's launch time, and, as a model,
+    # the bytes of the track records (116 B in the FP64 form: position 24,
+    # direction 24, energy 8, 3 interaction lengths 24, RNG 24, event,
+    # volume|species, step count 4 each): one read and one write for every track
+    # that a transport or an interaction task loads, one write for every track
+    # created.  (The per-track-step figure of 2 x 148 B, a nominal record with
+    # inverse mean free paths and safety, is the model's too.)
     rec = int(ks.record_bytes)
     # The launches carry HIP events during the timed batches, taken from the
     # kernel's own dispatches (profile_kernels); the parts share a launch's
@@ -571,13 +586,15 @@ def main():
                 "%d + %d tracks loaded by photon and e-/e+ transport, %d by interactions, %d created"
                 % (rec, rec, ks.neutral_loaded, ks.charged_loaded, ks.interactions, ks.created))
     avg_us = 1e3 * ms / launches
-    achieved = (nbytes / launches) / (avg_us * 1e-6) / 1e9
-    roofline = dict(bound="hbm", achieved=achieved, peak=PEAK_HBM_GBS, unit="GB/s", frac=achieved / PEAK_HBM_GBS,
-                    traffic=profiled_traffic(name), kernel=name, launches=int(ks.launches), avg_launch_us=avg_us,
-                    bytes_per_launch=nbytes / launches, per_unit=per_unit, record_bytes_in_pool=rec,
-                    kernel_ms=ms, parts=parts,
-                    per_track_step_296b_gbs=ks.track_steps * 2 * 148 / (ms * 1e-3) / 1e9,
-                    whole_run_gbs=nbytes / r64["seconds"] / 1e9)
+    issue = profiled_issue()
+    traffic = profiled_traffic(name)
+    gbs = traffic / (avg_us * 1e-6) / 1e9 if traffic else None
+    roofline = dict(bound="vector instruction issue", achieved=issue, peak=100.0, unit="% of SIMD cycles",
+                    frac=issue / 100.0 if issue else None, kernel=name, launches=int(ks.launches),
+                    avg_launch_us=avg_us, kernel_ms=ms, parts=parts, traffic=traffic,
+                    hbm=dict(achieved=gbs, peak=PEAK_HBM_GBS, unit="GB/s", frac=gbs / PEAK_HBM_GBS if gbs else None),
+                    records_model=dict(bytes_per_launch=nbytes / launches, per_unit=per_unit, record_bytes=rec,
+                                       per_track_step_296b_gbs=ks.track_steps * 2 * 148 / (ms * 1e-3) / 1e9))
     e64 = r64["edep"]["edep"]
     out = dict(metric="events/s and track-steps/s, FP32 vs FP64 on 1 MI355X; p99 job latency", value=value,
                unit="events/s", n_gpus=1, steps=a.steps, warmup=a.warmup,

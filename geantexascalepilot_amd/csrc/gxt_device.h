@@ -39,8 +39,10 @@ __device__ __forceinline__ float div_by(float n, float d, float y) {
   q = fmaf(fmaf(-d, q, n), y, q);
   return fmaf(fmaf(-d, q, n), y, q);
 }
-// The same for a d without a known reciprocal: the steps of a division without
-// the scaling for extreme exponents (8 operations, 3 more for each further n).
+// The same for a d without a known reciprocal, without the scaling that a
+// division has for extreme exponents: two Newton-Raphson steps from the hardware's
+// reciprocal estimate, then the quotient corrected once with its exact remainder (8
+// operations, 3 more for each further n).
 __device__ __forceinline__ double rcp_normal(double d) {
   double y = __builtin_amdgcn_rcp(d);
   y = fma(fma(-d, y, 1.0), y, y);

@@ -222,7 +222,7 @@ struct Job {
   int ev_base = -1;                 // first event slot of the job
   bool started = false;
   double submit_ms = 0, admit_ms = 0, done_ms = 0;
-  int64_t admit_iter = 0, done_iter = 0;  // step-loop iterations launched at admission / at the finding snapshot
+  int64_t admit_iter = 0, done_iter = 0;  // step-loop launches queued at admission / at the finding snapshot
   std::vector<gxt_event_tally> tallies;
   int64_t steps = 0;
 };
@@ -379,7 +379,6 @@ struct gxt_ctx {
 
 namespace {
 
-// Estimated peak live tracks of an event, from its primaries' energy.
 // Peak live tracks expected of event e: 16 per primary plus the learned
 // number per GeV.
 double event_peak(const gxt_ctx *c, const Job *j, int e) {
@@ -481,7 +480,7 @@ int admit(gxt_ctx *c) {
   // everything below is queued on the stream behind the work in flight (the
   // jobs' primaries were copied to the device at submission, earlier on the
   // same stream); the slots of a new job belong to events without tracks, so
-  // the look-ahead iterations still running do not touch them
+  // the look-ahead launch still running does not touch them
   for (auto &r : zero_ranges) {
     HIP_TRY(hipMemsetAsync(c->ev + r.first, 0, r.second * sizeof(DevEvent), c->stream));
     HIP_TRY(hipMemsetAsync(c->ev_live + (size_t)r.first * kLiveStride, 0, (size_t)r.second * kLiveStride * sizeof(int),
@@ -714,7 +713,7 @@ void destroy_ctx(gxt_ctx *c) {
     c->stop = true;
     if (c->server.joinable()) c->server.join();
   }
-  // look-ahead iterations may still be in flight
+  // a look-ahead launch may still be in flight
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (auto &q : c->ev_free)
     for (auto &x : q)
@@ -1377,7 +1376,6 @@ int gxt_get_kernel_stats(gxt_ctx *c, gxt_kernel_stats *o) {
   o->neutral_interactions = (int64_t)h.total(kStatInteractions0);
   o->neutral_created = (int64_t)h.total(kStatCreated0);
   // x, y, z (FP64) + dir, E, 3 interaction lengths (R) + 6 RNG words + event, meta, nsteps
-  // + 3 FP64 per-track tallies
   const int r = c->precision == GXT_FP32 ? 4 : 8;
   o->record_bytes = 3 * 8 + 7 * r + 6 * 4 + 3 * 4;
   return GXT_OK;
@@ -1435,7 +1433,7 @@ int gxt_serve_stop(gxt_ctx *c) {
   c->stop = true;
   if (c->server.joinable()) c->server.join();
   c->serving = false;
-  // the last round's look-ahead iterations
+  // the last round's look-ahead launch
   HIP_TRY(hipStreamSynchronize(c->stream));
   const int rc = c->serve_rc.load();
   if (rc != GXT_OK) return set_err(rc, c->error());

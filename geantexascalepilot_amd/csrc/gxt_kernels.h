@@ -7,10 +7,8 @@
 
 namespace gxt {
 
-// Per-workgroup tally rows: bins[row * stride + (z | nz + r | nz + nr + vol)]
-// and spec[row * 3 * kSpecBins + species * kSpecBins + bin].
-// Per-workgroup histogram rows: workgroup b adds into row b % nrows
-// (z bins, r bins, volumes; spectra: 3 species x kSpecBins).
+// Histogram rows: workgroup b adds into row b % nrows, bins[row * stride + (z | nz
+// + r | nz + nr + vol)] and spec[row * 3 * kSpecBins + species * kSpecBins + bin].
 struct TallyRows {
   double *bins;
   unsigned long long *spec;
