@@ -298,7 +298,7 @@ struct alignas(256) Counters {
 // shrink and end in between; so each workgroup gives, beside the change, the
 // largest growth that it saw, and the sum of those on top of the count before
 // bounds what was live at once (exact for an event in one workgroup).  The growths
-// cost 10,000 e- of 10 GeV 1 % (FP32 34.0 -> 34.4 ms).
+// cost 10,000 e- of 10 GeV 2 % in FP32 (33.8 -> 34.5 ms), 0.3 % in FP64.
 constexpr int kLiveStride = 32;
 enum { kLiveNow = 0,
        kLiveGrow,    // sum of the growths since the last snapshot

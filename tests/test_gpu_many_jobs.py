@@ -46,10 +46,10 @@ def run_jobs(gpu_lib, jobs, per, pool, ekin, mixed):
             np.testing.assert_allclose(gpu, cpu[k], rtol=1e-9, atol=1e-9, err_msg=k)
 
 
-# one primary for each workgroup and job (97 and 256 of them), jobs of one event,
+# one primary for each workgroup and job (97 and 256 of them) and one more, jobs of one event,
 # more jobs than one injection takes, both species classes
 @pytest.mark.parametrize("jobs,per,pool,ekin,mixed", [
-    (300, 1, 8192, 1.0, False), (65, 3, 65536, 5.0, True), (200, 97, 400_000, 1.0, False),
+    (300, 1, 8192, 1.0, False), (65, 3, 65536, 5.0, True), (200, 97, 400_000, 1.0, False), (120, 98, 400_000, 1.0, False),
     (400, 256, 2_000_000, 1.0, False)])
 def test_jobs_share_pages(gpu_lib, jobs, per, pool, ekin, mixed):
     run_jobs(gpu_lib, jobs, per, pool, ekin, mixed)
